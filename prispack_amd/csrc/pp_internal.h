@@ -228,19 +228,19 @@ struct DevSweep {
     void free_all();
 };
 
-// PP_TRSV_BLOCK: the rows split into contiguous chunks that no dependency of
-// either sweep crosses, each small enough for its part of the vector to sit
-// in LDS.  One workgroup per chunk runs both sweeps over its rows, level by
-// level with a workgroup barrier between levels, so a dependency chain of L
-// levels costs L barriers instead of L launches, and independent diagonal
-// blocks (the subdomains of a multilevel preconditioner) run side by side.
+// PP_TRSV_BLOCK, PP_TRSV_PIPE: the rows split into contiguous chunks that no
+// dependency of either sweep crosses, each small enough for its part of the
+// vector to sit in LDS.  One workgroup per chunk runs both sweeps over its
+// rows, so a dependency chain of L levels costs L steps of one workgroup
+// instead of L launches, and independent diagonal blocks (the subdomains of
+// a multilevel preconditioner) run side by side.
 struct ChunkSet {
     std::vector<uint32_t> start;   // host [nchunk+1] first original row of each chunk
     uint32_t *dstart = nullptr;    // the same on the device
     uint32_t nchunk = 0, max_rows = 0;
     void free_all();
 };
-// Rows are stored by position (chunk-major, level order inside a chunk), the
+// PP_TRSV_PIPE's storage: rows by position (chunk-major, level order inside a chunk), the
 // entries of consecutive positions contiguous, so the entries of a level are
 // one contiguous range: the workgroup loads them coalesced, forms the
 // products in LDS, and each row's thread subtracts its products in storage
@@ -256,6 +256,22 @@ struct DevChunkSweep {
     uint32_t *lp = nullptr;        // level boundaries (positions); chunk c: lp[lev_off[c] .. lev_off[c+1]-1]
     uint32_t *le = nullptr;        // rp at those boundaries (first entry of each level)
     uint32_t *lev_off = nullptr;   // [nchunk+1]
+    void free_all();
+};
+
+// Both sweeps of every chunk as one stream of steps (pp_sweep_lanes.hip).
+constexpr int kLaneAhead = 8;
+struct LaneHead {
+    uint64_t first = 0;                    // byte offset of the chunk's steps
+    uint32_t rounds_lo = 0, rounds_up = 0; // kLaneAhead steps each
+    uint32_t active[kLaneAhead];           // lanes of its first steps
+};
+template <class T>
+struct LaneSweep {
+    LaneHead *head = nullptr;  // [nchunk]
+    unsigned char *data = nullptr;
+    int waves = 0, group = 0, slots = 0;  // wavefronts of the workgroup, lanes of a row, entries of a lane
+    int mode_lo = 0, mode_up = 0;         // the sweeps' diagonal modes
     void free_all();
 };
 
@@ -479,6 +495,8 @@ struct pp_precond {
     pp::ChunkSet chunks;
     pp::DevChunkSweep<double> clow64, cup64;
     pp::DevChunkSweep<float> clow32, cup32;
+    pp::LaneSweep<double> lanes64;
+    pp::LaneSweep<float> lanes32;
 };
 
 namespace pp {
@@ -695,12 +713,16 @@ pp_csr *csr_from_device(pp_ctx *ctx, uint32_t nrow, uint32_t ncol, uint32_t *rp,
 template <class T>
 void launch_sweep(pp_ctx *ctx, const DevSweep<T> &s, int mode, const T *b, T *x);
 // Both sweeps of an apply in one launch, one workgroup per chunk
-// (PP_TRSV_BLOCK; DevChunkSweep).  y = U^{-1} L^{-1} x, y may alias x.
+// (PP_TRSV_BLOCK).  y = U^{-1} L^{-1} x, y may alias x.  lane_sweep_max_rows:
+// the rows of a chunk that fit an LDS of that size.
+uint32_t lane_sweep_max_rows(size_t lds);
 template <class T>
-void launch_sweep_pair_chunks(pp_ctx *ctx, const ChunkSet &C, const DevChunkSweep<T> &lo, int mlo,
-                              const DevChunkSweep<T> &up, int mup, const T *x, T *y);
-// The same sweeps, one wavefront computing the levels while the rest of the
-// workgroup stages their data in LDS (pp_sweep_pipe.hip); sweep_pipe_rings:
+void build_lane_sweep(const HostSweep &lo, const HostSweep &up, const ChunkSet &C, LaneSweep<T> &S);
+template <class T>
+void launch_lane_sweep(pp_ctx *ctx, const ChunkSet &C, const LaneSweep<T> &S, const T *x, T *y);
+// The same sweeps from the level-ordered storage (DevChunkSweep), one
+// wavefront computing the levels while the rest of the workgroup stages
+// their data in LDS (PP_TRSV_PIPE, pp_sweep_pipe.hip); sweep_pipe_rings:
 // the LDS ring sizes, false when the chunks leave too little LDS for them.
 template <class T>
 void launch_sweep_pair_pipe(pp_ctx *ctx, const ChunkSet &C, const DevChunkSweep<T> &lo, int mlo,

@@ -389,40 +389,48 @@ static void upload_chunk_sweep(const HostSweep &s, const ChunkSet &C, DevChunkSw
     if (s.mode != HostSweep::UNIT) up(pdiag, d.pdiag);
 }
 
-// PP_TRSV_BLOCK storage for M (FP64; FP32 too when the FP32 sweeps exist).
-// false (nothing kept) when the rows do not chunk within the LDS size.
-static void ensure_host_setup(pp_precond *M);
-
-static bool build_block_sweeps(pp_ctx *ctx, pp_precond *M) {
-    ensure_host_setup(M);  // the chunks are cut from the host sweeps
+static void free_block_sweeps(pp_precond *M) {
     M->chunks.free_all();
+    M->lanes64.free_all();
+    M->lanes32.free_all();
     M->clow64.free_all();
     M->cup64.free_all();
     M->clow32.free_all();
     M->cup32.free_all();
-    const uint32_t cap = (uint32_t)std::min<size_t>(ctx->max_lds / sizeof(double), 65535);
-    if (!build_chunks({&M->hlow, &M->hup}, M->n, cap, M->chunks)) {
+}
+
+// the FP32 storage of the chunked schedule in use
+static void build_block_sweeps32(pp_precond *M) {
+    if (M->clow64.row) {
+        upload_chunk_sweep(M->hlow, M->chunks, M->clow32);
+        upload_chunk_sweep(M->hup, M->chunks, M->cup32);
+    } else {
+        build_lane_sweep<float>(M->hlow, M->hup, M->chunks, M->lanes32);
+    }
+}
+
+// PP_TRSV_BLOCK storage for M, or (pipe) PP_TRSV_PIPE storage (FP64; FP32 too
+// when the FP32 sweeps exist).  false (nothing kept) when the rows do not
+// chunk within the LDS size.
+static void ensure_host_setup(pp_precond *M);
+
+static bool build_block_sweeps(pp_ctx *ctx, pp_precond *M, bool pipe) {
+    ensure_host_setup(M);  // the chunks are cut from the host sweeps
+    free_block_sweeps(M);
+    if (!build_chunks({&M->hlow, &M->hup}, M->n, lane_sweep_max_rows(ctx->max_lds), M->chunks)) {
         M->chunks.free_all();
         return false;
     }
     M->chunks.dstart = dalloc<uint32_t>(M->chunks.start.size());
     PP_HIP(hipMemcpy(M->chunks.dstart, M->chunks.start.data(), M->chunks.start.size() * sizeof(uint32_t),
                      hipMemcpyHostToDevice));
-    upload_chunk_sweep(M->hlow, M->chunks, M->clow64);
-    upload_chunk_sweep(M->hup, M->chunks, M->cup64);
-    // the chunk's vector and both sweeps' level boundaries must fit in LDS
-    const size_t need = (size_t)M->chunks.max_rows * sizeof(double) +
-                        4 * (size_t)(2 * (M->clow64.max_levels + 1) + 2 * (M->cup64.max_levels + 1));
-    if (need > ctx->max_lds) {
-        M->chunks.free_all();
-        M->clow64.free_all();
-        M->cup64.free_all();
-        return false;
+    if (pipe) {
+        upload_chunk_sweep(M->hlow, M->chunks, M->clow64);
+        upload_chunk_sweep(M->hup, M->chunks, M->cup64);
+    } else {
+        build_lane_sweep<double>(M->hlow, M->hup, M->chunks, M->lanes64);
     }
-    if (M->have32) {
-        upload_chunk_sweep(M->hlow, M->chunks, M->clow32);
-        upload_chunk_sweep(M->hup, M->chunks, M->cup32);
-    }
+    if (M->have32) build_block_sweeps32(M);
     return true;
 }
 
@@ -973,10 +981,7 @@ void precond_need_f32(pp_precond *M) {
     M->low32.variant = M->up32.variant = M->sweep_variant;
     if (M->trsv == PP_TRSV_LEVELS && M->n >= kTuneSweepRows && (M->low32.blocks || M->up32.blocks) && !M->sweep_pinned)
         tune_sweep_pair<float>(M->ctx, M, M->low32, M->up32, M->sweep_variant);
-    if (M->chunks.nchunk) {
-        upload_chunk_sweep(M->hlow, M->chunks, M->clow32);
-        upload_chunk_sweep(M->hup, M->chunks, M->cup32);
-    }
+    if (M->chunks.nchunk) build_block_sweeps32(M);
     M->have32 = true;
 }
 
@@ -1064,15 +1069,23 @@ void precond_apply(pp_ctx *ctx, pp_precond *M, int dtype, const void *x, void *y
         }
         return;
     }
-    if (M->trsv == PP_TRSV_BLOCK || M->trsv == PP_TRSV_PIPE) {
-        const bool pipe = M->trsv == PP_TRSV_PIPE;
+    if (M->trsv == PP_TRSV_BLOCK) {
         if (dtype == PP_F64) {
-            (pipe ? launch_sweep_pair_pipe<double> : launch_sweep_pair_chunks<double>)(
-                ctx, M->chunks, M->clow64, M->hlow.mode, M->cup64, M->hup.mode, (const double *)x, (double *)y);
+            launch_lane_sweep<double>(ctx, M->chunks, M->lanes64, (const double *)x, (double *)y);
         } else {
             precond_need_f32(M);
-            (pipe ? launch_sweep_pair_pipe<float> : launch_sweep_pair_chunks<float>)(
-                ctx, M->chunks, M->clow32, M->hlow.mode, M->cup32, M->hup.mode, (const float *)x, (float *)y);
+            launch_lane_sweep<float>(ctx, M->chunks, M->lanes32, (const float *)x, (float *)y);
+        }
+        return;
+    }
+    if (M->trsv == PP_TRSV_PIPE) {
+        if (dtype == PP_F64) {
+            launch_sweep_pair_pipe<double>(ctx, M->chunks, M->clow64, M->hlow.mode, M->cup64, M->hup.mode,
+                                           (const double *)x, (double *)y);
+        } else {
+            precond_need_f32(M);
+            launch_sweep_pair_pipe<float>(ctx, M->chunks, M->clow32, M->hlow.mode, M->cup32, M->hup.mode,
+                                          (const float *)x, (float *)y);
         }
         return;
     }
@@ -1148,36 +1161,32 @@ static void tune_sweeps(pp_ctx *ctx, pp_precond *M) {
     M->sweep_variant = tune_sweep_pair<double>(ctx, M, M->low64, M->up64, M->sweep_variant);
 }
 
-// PP_TRSV_AUTO: the fastest of one launch per level and, when the rows chunk
-// within LDS, the chunked one-workgroup schedules (barrier per level, and
-// the pipelined form when its rings fit), timed here over a few applies
-// each.  PP_TRSV_BLOCK / PP_TRSV_PIPE asked for explicitly (force) fall
-// back to levels when the rows do not chunk, and PIPE to BLOCK when the
-// rings do not fit.
+// PP_TRSV_AUTO: the faster of one launch per level and, when the rows chunk
+// within LDS, the chunked one-workgroup schedule (PP_TRSV_BLOCK), timed here
+// over a few applies each.  PP_TRSV_BLOCK / PP_TRSV_PIPE asked for
+// explicitly (force) fall back to levels when the rows do not chunk, and
+// PIPE to BLOCK when its rings do not fit.
 static int choose_schedule(pp_ctx *ctx, pp_precond *M, int force) {
     const uint32_t nlev = M->low64.nlev + M->up64.nlev;
-    if ((!force && nlev < 8) || !build_block_sweeps(ctx, M)) return PP_TRSV_LEVELS;
-    uint32_t re = 0, rr = 0;
-    const bool pipe_ok = sweep_pipe_rings<double>(ctx, M->chunks, re, rr);
-    if (force == PP_TRSV_BLOCK || (force == PP_TRSV_PIPE && !pipe_ok)) return PP_TRSV_BLOCK;
-    if (force == PP_TRSV_PIPE) return PP_TRSV_PIPE;
+    if (!force && nlev < 8) return PP_TRSV_LEVELS;
+    if (force == PP_TRSV_PIPE) {
+        if (!build_block_sweeps(ctx, M, true)) return PP_TRSV_LEVELS;
+        uint32_t re = 0, rr = 0;
+        if (sweep_pipe_rings<double>(ctx, M->chunks, re, rr)) return PP_TRSV_PIPE;
+        force = PP_TRSV_BLOCK;
+    }
+    if (!build_block_sweeps(ctx, M, false)) return PP_TRSV_LEVELS;
+    if (force) return PP_TRSV_BLOCK;
     double *v = dalloc<double>(M->n);
-    const int cand[3] = {PP_TRSV_LEVELS, PP_TRSV_BLOCK, PP_TRSV_PIPE};
-    float ms[3] = {0.f, 0.f, 0.f};
-    const int ncand = pipe_ok ? 3 : 2;
+    float ms[2] = {0.f, 0.f};
     try {
         launch_fill_zero(ctx, v, (size_t)M->n * sizeof(double));
-        launch_fill_zero(ctx, ctx->ctl, C_COUNT * sizeof(int));
-        for (int k = 0; k < ncand; ++k) {
+        for (int k = 0; k < 2; ++k) {
             auto apply = [&] {
-                if (cand[k] == PP_TRSV_LEVELS)
+                if (k == 0)
                     launch_sweep_pair<double>(ctx, M->low64, M->hlow.mode, M->up64, M->hup.mode, M->fuse_mid, v, v);
-                else if (cand[k] == PP_TRSV_BLOCK)
-                    launch_sweep_pair_chunks<double>(ctx, M->chunks, M->clow64, M->hlow.mode, M->cup64, M->hup.mode,
-                                                     v, v);
                 else
-                    launch_sweep_pair_pipe<double>(ctx, M->chunks, M->clow64, M->hlow.mode, M->cup64, M->hup.mode,
-                                                   v, v);
+                    launch_lane_sweep<double>(ctx, M->chunks, M->lanes64, v, v);
             };
             apply();
             PP_HIP(hipEventRecord(ctx->ev0, ctx->stream));
@@ -1186,26 +1195,13 @@ static int choose_schedule(pp_ctx *ctx, pp_precond *M, int force) {
             PP_HIP(hipEventSynchronize(ctx->ev1));
             PP_HIP(hipEventElapsedTime(&ms[k], ctx->ev0, ctx->ev1));
         }
-        if (ncand == 3) {  // a pipelined sweep that gave up waiting is not a candidate
-            int ctl[C_COUNT];
-            read_ctl(ctx, ctl);
-            if (ctl[C_SPIN]) {
-                ms[2] = 1e30f;
-                launch_fill_zero(ctx, ctx->ctl, C_COUNT * sizeof(int));
-            }
-        }
     } catch (...) {
         dfree(v);
         throw;
     }
     dfree(v);
-    int best = 0;
-    for (int k = 1; k < ncand; ++k)
-        if (ms[k] < ms[best]) best = k;
-    if (cand[best] != PP_TRSV_LEVELS) return cand[best];
-    M->chunks.free_all();  // not used: give the memory back
-    M->clow64.free_all();
-    M->cup64.free_all();
+    if (ms[1] < ms[0]) return PP_TRSV_BLOCK;
+    free_block_sweeps(M);  // not used: give the memory back
     return PP_TRSV_LEVELS;
 }
 
@@ -1328,11 +1324,7 @@ int pp_precond_refactor(pp_ctx *ctx, pp_precond *M) {
             M->dorder = nullptr;
             dfree(M->xp64);
             M->xp64 = nullptr;
-            M->chunks.free_all();
-            M->clow64.free_all();
-            M->cup64.free_all();
-            M->clow32.free_all();
-            M->cup32.free_all();
+            free_block_sweeps(M);
             if (M->multilevel) ml_free(M);
             reduced_free(M);
             M->uid = next_uid();  // graphs captured with the freed arrays are never replayed
@@ -1587,11 +1579,7 @@ void pp_precond_destroy(pp_precond *M) {
     dfree(M->tmp32);
     csr_free(M->Aperm);
     pp::reduced_free(M);
-    M->chunks.free_all();
-    M->clow64.free_all();
-    M->cup64.free_all();
-    M->clow32.free_all();
-    M->cup32.free_all();
+    free_block_sweeps(M);
     M->low64.free_all();
     M->up64.free_all();
     M->low32.free_all();

@@ -1,0 +1,114 @@
+"""The chunked triangular sweeps (PP_TRSV_BLOCK) against one launch per level
+(PP_TRSV_LEVELS, itself pinned to the oracle): every step shape, all three
+pairs of diagonal modes, rows of no, one and many steps, operands whose
+quotients leave the range of the reciprocal division.  Equal bit for bit in
+both precisions: the sweeps do the same operations in the same order."""
+import numpy as np
+import pytest
+
+from oracle import ppo
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+@pytest.fixture(scope="module")
+def pp(torch):
+    import prispack_amd
+    return prispack_amd
+
+
+def blocks(A, count):
+    """count copies of A on the diagonal, every second one cut to half its rows."""
+    rp, ci, v = A
+    n = len(rp) - 1
+    rps, cis, vs, row, nnz = [np.zeros(1, np.int64)], [], [], 0, 0
+    for k in range(count):
+        m = n // 2 if k % 2 else n
+        keep = (np.arange(len(ci)) < rp[m]) & (ci < m)
+        cnt = np.add.reduceat(keep[:rp[m]].astype(np.int64), rp[:m].astype(np.int64))
+        rps.append(np.cumsum(cnt) + nnz)
+        cis.append(ci[keep].astype(np.int64) + row)
+        vs.append(v[keep])
+        row, nnz = row + m, nnz + int(keep.sum())
+    return np.concatenate(rps).astype(np.uint32), np.concatenate(cis).astype(np.uint32), np.concatenate(vs)
+
+
+def diagonal(d):
+    n = len(d)
+    return np.arange(n + 1, dtype=np.uint32), np.arange(n, dtype=np.uint32), d
+
+
+CASES = {
+    # name: matrix, kind, arguments
+    "one_row": lambda: (diagonal(np.array([3.0])), "ict", dict(threshold=1e-3)),
+    "chain": lambda: (ppo.laplacian(700, 1, 1), "ict", dict(threshold=0.0)),
+    "narrow": lambda: (ppo.laplacian(37, 31, 1), "ict", dict(threshold=1e-3)),
+    "2d_fill": lambda: (ppo.laplacian(90, 81, 1), "ict", dict(threshold=1e-3)),
+    "2d_short": lambda: (ppo.laplacian(101, 90, 1), "ict", dict(threshold=1e-2)),
+    "long_rows": lambda: (ppo.laplacian(41, 40, 1), "ict", dict(threshold=0.0)),
+    "3d_wide": lambda: (ppo.laplacian(25, 24, 23), "ict", dict(threshold=3e-3)),
+    "two_levels": lambda: (ppo.laplacian(113, 90, 1), "ic0", dict(ordering=1)),
+    "ildlt": lambda: (ppo.laplacian(61, 54, 1), "ildlt", dict(tolerance=1e-3)),
+    "ilut": lambda: (ppo.upwind(19, 18, 17, 20.0, 10.0, 5.0), "ilut", dict(lfill=20, tolerance=1e-2)),
+    "ilu0": lambda: (ppo.upwind(19, 18, 17, 20.0, 10.0, 5.0), "ilu0", dict()),
+    "blocks": lambda: (blocks(ppo.laplacian(22, 21, 20), 9), "ildlt", dict(tolerance=1e-3)),
+}
+
+
+def bits(torch, t):
+    return t.view(torch.int64 if t.dtype == torch.float64 else torch.int32)
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_block_sweeps_match_levels(pp, torch, name):
+    A, kind, kw = CASES[name]()
+    n = len(A[0]) - 1
+    print(f"[sweeps] {name} n={n}", flush=True)
+    M = pp.CSRMatrix(*A)
+    cls = {"ict": pp.IncompleteCholesky, "ildlt": pp.IncompleteLDLT, "ilut": pp.IncompleteLU, "ic0": pp.IC0,
+           "ilu0": pp.ILU0}[kind]
+    P1, P3 = (cls(M, trsv=t, **kw) for t in (1, 3))
+    P1.setup()
+    P3.setup()
+    assert P1.info().trsv == 1 and P3.info().trsv == 3
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(n)
+    x[rng.random(n) < 0.2] = 0.0   # zeros of both signs take the division itself
+    x[rng.random(n) < 0.05] = -0.0
+    scaled = [x, x * 1e-300, x * 2.0 ** 900, np.where(np.arange(n) == n // 2, np.inf, x)]
+    for k, xs in enumerate(scaled):
+        for dt in (torch.float64, torch.float32):
+            v = torch.tensor(xs, dtype=dt, device="cuda")
+            want, got = P1.MInvSolve(v.clone()), torch.full_like(v, 7.0)
+            P3.MInvSolve(v, got)
+            same = (bits(torch, want) == bits(torch, got)) | (torch.isnan(want) & torch.isnan(got))
+            assert bool(same.all()), (name, k, dt, int((~same).sum()))
+
+
+def test_block_sweep_quotients(pp, torch):
+    # a diagonal factor divides twice by each pivot: mantissas and exponents
+    # over the whole range, pivots past the reciprocals' range among them
+    rng = np.random.default_rng(3)
+    n = 20000
+    e = rng.integers(-200, 200, n)
+    e[::40] = rng.integers(-500, 500, len(e[::40]))
+    A = diagonal(rng.uniform(1.0, 2.0, n) * 2.0 ** (2 * e))
+    M = pp.CSRMatrix(*A)
+    P1, P3 = (pp.IncompleteCholesky(M, 1e-3, trsv=t) for t in (1, 3))
+    P1.setup()
+    P3.setup()
+    assert P3.info().trsv == 3
+    for dt, span in ((torch.float64, 1000), (torch.float32, 130)):
+        x = rng.uniform(-2.0, 2.0, n) * 2.0 ** rng.integers(-span, span, n)
+        v = torch.tensor(x, dtype=dt, device="cuda")
+        want, got = P1.MInvSolve(v.clone()), P3.MInvSolve(v.clone())
+        same = (bits(torch, want) == bits(torch, got)) | (torch.isnan(want) & torch.isnan(got))
+        assert bool(same.all()), int((~same).sum())
