@@ -146,14 +146,16 @@ enum {
     PP_TRSV_AUTO = 0,
     PP_TRSV_LEVELS = 1,    /* one launch per level (graph-captured)               */
     PP_TRSV_SYNCFREE = 2,  /* one launch per sweep, per-row ready flags            */
-    PP_TRSV_BLOCK = 3,     /* both sweeps in one workgroup, the vector in LDS, a
-                              barrier per level (n * 8 bytes must fit in LDS;
-                              larger systems use LEVELS).  AUTO times it against
-                              LEVELS at setup when it fits                         */
-    PP_TRSV_PIPE = 4       /* BLOCK's storage; one wavefront computes the levels
-                              with no barrier while the workgroup's other waves
-                              stage the level data in LDS ahead of it (for many
-                              narrow levels).  AUTO times it with the others      */
+    PP_TRSV_BLOCK = 3,     /* both sweeps in one workgroup, the vector in LDS (n * 8
+                              bytes must fit in LDS; larger systems use LEVELS).
+                              AUTO times it against LEVELS at setup when it fits   */
+    PP_TRSV_PIPE = 4,      /* one workgroup as BLOCK, level data staged in an LDS
+                              ring by the workgroup's other waves (AUTO does not
+                              pick it)                                             */
+    PP_TRSV_STRIPS = 5     /* contiguous strips of rows, a workgroup each, that pass
+                              the values they share while the sweep runs.  AUTO
+                              times it against LEVELS at setup for threshold
+                              factors that BLOCK does not fit                      */
 };
 
 /* Row ordering of the factor (no reference counterpart; the reference factors

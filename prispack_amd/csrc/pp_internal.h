@@ -275,6 +275,26 @@ struct LaneSweep {
     void free_all();
 };
 
+// PP_TRSV_STRIPS: the rows cut into contiguous strips, a workgroup each,
+// which exchange the values they need of one another while a sweep runs
+// (pp_sweep_lanes.hip).
+template <class T>
+struct StripSide {
+    unsigned char *head = nullptr, *data = nullptr;  // per strip, steps
+    uint32_t *imp = nullptr;        // imported slots
+    T *slots = nullptr;             // exchange buffer
+    uint32_t nslots = 0, max_words = 0;
+    int mode = 0;
+    void free_all();
+};
+template <class T>
+struct StripSweep {
+    StripSide<T> lo, up;
+    uint32_t nstrip = 0, max_words = 0;  // strips, LDS words of the largest
+    int group = 0, slots = 0;
+    void free_all();
+};
+
 // Host gather-form sweep: row i = s_i -> (b_i - sum val*x[ci]) op diag_i.
 // Symbolic state of a numeric re-factorization on the device
 // (pp_precond_refactor, IC(0) / ILU(0)): the factor's pattern, its
@@ -497,6 +517,8 @@ struct pp_precond {
     pp::DevChunkSweep<float> clow32, cup32;
     pp::LaneSweep<double> lanes64;
     pp::LaneSweep<float> lanes32;
+    pp::StripSweep<double> strips64;  // PP_TRSV_STRIPS storage
+    pp::StripSweep<float> strips32;
 };
 
 namespace pp {
@@ -720,6 +742,11 @@ template <class T>
 void build_lane_sweep(const HostSweep &lo, const HostSweep &up, const ChunkSet &C, LaneSweep<T> &S);
 template <class T>
 void launch_lane_sweep(pp_ctx *ctx, const ChunkSet &C, const LaneSweep<T> &S, const T *x, T *y);
+// PP_TRSV_STRIPS: false (nothing kept) when the strips do not fit LDS.
+template <class T>
+bool build_strip_sweeps(pp_ctx *ctx, const HostSweep &lo, const HostSweep &up, StripSweep<T> &L);
+template <class T>
+void launch_strip_sweeps(pp_ctx *ctx, const StripSweep<T> &L, const T *x, T *y);
 // The same sweeps from the level-ordered storage (DevChunkSweep), one
 // wavefront computing the levels while the rest of the workgroup stages
 // their data in LDS (PP_TRSV_PIPE, pp_sweep_pipe.hip); sweep_pipe_rings:

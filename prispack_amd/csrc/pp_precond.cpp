@@ -391,6 +391,8 @@ static void upload_chunk_sweep(const HostSweep &s, const ChunkSet &C, DevChunkSw
 
 static void free_block_sweeps(pp_precond *M) {
     M->chunks.free_all();
+    M->strips64.free_all();
+    M->strips32.free_all();
     M->lanes64.free_all();
     M->lanes32.free_all();
     M->clow64.free_all();
@@ -723,7 +725,7 @@ static void lower_levels(uint32_t n, const std::vector<uint32_t> &rp, const std:
 static bool devref_build(pp_ctx *ctx, pp_precond *M) {
     const int kind = M->opts.kind;
     if ((kind != PP_PC_IC0 && kind != PP_PC_ILU0) || M->trsv == PP_TRSV_BLOCK || M->trsv == PP_TRSV_PIPE ||
-        M->multilevel)
+        M->trsv == PP_TRSV_STRIPS || M->multilevel)
         return false;
     const bool ordered = !M->order.empty();
     if (ordered && !M->Aperm) return false;
@@ -982,6 +984,8 @@ void precond_need_f32(pp_precond *M) {
     if (M->trsv == PP_TRSV_LEVELS && M->n >= kTuneSweepRows && (M->low32.blocks || M->up32.blocks) && !M->sweep_pinned)
         tune_sweep_pair<float>(M->ctx, M, M->low32, M->up32, M->sweep_variant);
     if (M->chunks.nchunk) build_block_sweeps32(M);
+    if (M->strips64.nstrip)
+        PP_CHECK(build_strip_sweeps<float>(M->ctx, M->hlow, M->hup, M->strips32), PP_ERR_HIP, "FP32 strips");
     M->have32 = true;
 }
 
@@ -1078,6 +1082,15 @@ void precond_apply(pp_ctx *ctx, pp_precond *M, int dtype, const void *x, void *y
         }
         return;
     }
+    if (M->trsv == PP_TRSV_STRIPS) {
+        if (dtype == PP_F64) {
+            launch_strip_sweeps<double>(ctx, M->strips64, (const double *)x, (double *)y);
+        } else {
+            precond_need_f32(M);
+            launch_strip_sweeps<float>(ctx, M->strips32, (const float *)x, (float *)y);
+        }
+        return;
+    }
     if (M->trsv == PP_TRSV_PIPE) {
         if (dtype == PP_F64) {
             launch_sweep_pair_pipe<double>(ctx, M->chunks, M->clow64, M->hlow.mode, M->cup64, M->hup.mode,
@@ -1161,11 +1174,17 @@ static void tune_sweeps(pp_ctx *ctx, pp_precond *M) {
     M->sweep_variant = tune_sweep_pair<double>(ctx, M, M->low64, M->up64, M->sweep_variant);
 }
 
-// PP_TRSV_AUTO: the faster of one launch per level and, when the rows chunk
-// within LDS, the chunked one-workgroup schedule (PP_TRSV_BLOCK), timed here
-// over a few applies each.  PP_TRSV_BLOCK / PP_TRSV_PIPE asked for
-// explicitly (force) fall back to levels when the rows do not chunk, and
-// PIPE to BLOCK when its rings do not fit.
+// The least a level's launch takes (4.1 to 4.4 us measured on narrow levels).
+constexpr float kLevelMs = 3.5e-3f;
+
+// PP_TRSV_AUTO: the faster of one launch per level and the storage in LDS,
+// PP_TRSV_BLOCK when the rows chunk, else PP_TRSV_STRIPS for the threshold
+// factors (a re-factorization of IC(0) / ILU(0) refills the level sweeps on
+// the device).  The latter is timed over a few applies, the levels only
+// where their launches might cost less (the narrow factors' 1000 levels
+// would spend 16 ms of a setup on being timed).  BLOCK, PIPE and
+// STRIPS asked for explicitly (force) fall back to levels when the rows do
+// not fit, and PIPE to BLOCK when its rings do not fit.
 static int choose_schedule(pp_ctx *ctx, pp_precond *M, int force) {
     const uint32_t nlev = M->low64.nlev + M->up64.nlev;
     if (!force && nlev < 8) return PP_TRSV_LEVELS;
@@ -1175,32 +1194,55 @@ static int choose_schedule(pp_ctx *ctx, pp_precond *M, int force) {
         if (sweep_pipe_rings<double>(ctx, M->chunks, re, rr)) return PP_TRSV_PIPE;
         force = PP_TRSV_BLOCK;
     }
-    if (!build_block_sweeps(ctx, M, false)) return PP_TRSV_LEVELS;
-    if (force) return PP_TRSV_BLOCK;
+    const bool threshold = M->opts.kind != PP_PC_IC0 && M->opts.kind != PP_PC_ILU0;
+    int other = PP_TRSV_BLOCK;
+    if (force == PP_TRSV_STRIPS || !build_block_sweeps(ctx, M, false)) {
+        if (force == PP_TRSV_BLOCK || (!force && !threshold)) return PP_TRSV_LEVELS;
+        ensure_host_setup(M);
+        free_block_sweeps(M);
+        if (!build_strip_sweeps<double>(ctx, M->hlow, M->hup, M->strips64)) return PP_TRSV_LEVELS;
+        if (M->have32 && !build_strip_sweeps<float>(ctx, M->hlow, M->hup, M->strips32)) {
+            free_block_sweeps(M);
+            return PP_TRSV_LEVELS;
+        }
+        other = PP_TRSV_STRIPS;
+    }
+    if (force) return other;
     double *v = dalloc<double>(M->n);
-    float ms[2] = {0.f, 0.f};
+    float ms[2] = {kLevelMs * nlev, 0.f};
+    int ctl[C_COUNT] = {};
     try {
         launch_fill_zero(ctx, v, (size_t)M->n * sizeof(double));
-        for (int k = 0; k < 2; ++k) {
+        launch_fill_zero(ctx, ctx->ctl, C_COUNT * sizeof(int));
+        for (int k = 1; k >= 0; --k) {
             auto apply = [&] {
                 if (k == 0)
                     launch_sweep_pair<double>(ctx, M->low64, M->hlow.mode, M->up64, M->hup.mode, M->fuse_mid, v, v);
-                else
+                else if (other == PP_TRSV_BLOCK)
                     launch_lane_sweep<double>(ctx, M->chunks, M->lanes64, v, v);
+                else
+                    launch_strip_sweeps<double>(ctx, M->strips64, v, v);
             };
+            constexpr int reps = 2;
             apply();
             PP_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-            for (int r = 0; r < 3; ++r) apply();
+            for (int r = 0; r < reps; ++r) apply();
             PP_HIP(hipEventRecord(ctx->ev1, ctx->stream));
             PP_HIP(hipEventSynchronize(ctx->ev1));
             PP_HIP(hipEventElapsedTime(&ms[k], ctx->ev0, ctx->ev1));
+            ms[k] /= reps;
+            if (k == 1) {
+                read_ctl(ctx, ctl);
+                if (ctl[C_SPIN]) launch_fill_zero(ctx, ctx->ctl, C_COUNT * sizeof(int));
+                if (!ctl[C_SPIN] && ms[1] < ms[0]) break;  // the levels' launches alone take longer
+            }
         }
     } catch (...) {
         dfree(v);
         throw;
     }
     dfree(v);
-    if (ms[1] < ms[0]) return PP_TRSV_BLOCK;
+    if (ms[1] < ms[0] && !ctl[C_SPIN]) return other;
     free_block_sweeps(M);  // not used: give the memory back
     return PP_TRSV_LEVELS;
 }
@@ -1289,7 +1331,7 @@ int pp_precond_setup(pp_ctx *ctx, pp_precond *M) {
             M->phase_ms[2] = (float)(std::chrono::duration<double, std::milli>(tp - t0).count() - M->phase_ms[0] -
                                      M->phase_ms[1]);
             const int want = M->opts.trsv;
-            M->trsv = want == PP_TRSV_AUTO || want == PP_TRSV_BLOCK || want == PP_TRSV_PIPE
+            M->trsv = want == PP_TRSV_AUTO || want == PP_TRSV_BLOCK || want == PP_TRSV_PIPE || want == PP_TRSV_STRIPS
                           ? choose_schedule(ctx, M, want)
                           : want;
             if (M->trsv == PP_TRSV_LEVELS) tune_sweeps(ctx, M);
@@ -1346,7 +1388,10 @@ int pp_precond_apply(pp_ctx *ctx, pp_precond *M, int dtype, const void *x, void 
         if (dtype == PP_F32) precond_need_f32(M);  // FP32 copies, once, outside any capture
         launch_fill_zero(ctx, ctx->ctl, C_COUNT * sizeof(int));  // clear stop / error words (graph-safe)
         precond_apply(ctx, M, dtype, x, y);
-        if (M->trsv == PP_TRSV_SYNCFREE || M->trsv == PP_TRSV_PIPE) {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (M->trsv == PP_TRSV_STRIPS) PP_HIP(hipStreamIsCapturing(ctx->stream, &capturing));
+        if (M->trsv == PP_TRSV_SYNCFREE || M->trsv == PP_TRSV_PIPE ||
+            (M->trsv == PP_TRSV_STRIPS && capturing == hipStreamCaptureStatusNone)) {
             int ctl[C_COUNT];
             read_ctl(ctx, ctl);
             PP_CHECK(!ctl[C_SPIN], PP_ERR_HIP, "sync-free triangular sweep timed out waiting for a dependency");

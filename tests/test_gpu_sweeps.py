@@ -1,8 +1,9 @@
-"""The chunked triangular sweeps (PP_TRSV_BLOCK) against one launch per level
-(PP_TRSV_LEVELS, itself pinned to the oracle): every step shape, all three
-pairs of diagonal modes, rows of no, one and many steps, operands whose
-quotients leave the range of the reciprocal division.  Equal bit for bit in
-both precisions: the sweeps do the same operations in the same order."""
+"""The chunked (PP_TRSV_BLOCK) and the strip-wise (PP_TRSV_STRIPS) triangular
+sweeps against one launch per level (PP_TRSV_LEVELS, itself pinned to the
+oracle): every step shape, all three pairs of diagonal modes, rows of no, one
+and many steps, operands whose quotients leave the range of the reciprocal
+division.  Equal bit for bit in both precisions: the sweeps do the same
+operations in the same order."""
 import numpy as np
 import pytest
 
@@ -67,18 +68,33 @@ def bits(torch, t):
     return t.view(torch.int64 if t.dtype == torch.float64 else torch.int32)
 
 
-@pytest.mark.parametrize("name", list(CASES))
-def test_block_sweeps_match_levels(pp, torch, name):
-    A, kind, kw = CASES[name]()
+LARGE = {
+    # connected parts larger than LDS holds: short rows, two-lane rows, rows of several steps
+    "3d_short": lambda: (ppo.laplacian(40, 33, 29), "ict", dict(threshold=1e-2)),
+    "3d_long": lambda: (ppo.laplacian(33, 32, 31), "ict", dict(threshold=1e-3)),
+    "2d_large": lambda: (ppo.laplacian(211, 190, 1), "ict", dict(threshold=1e-3)),
+    "2d_rcm": lambda: (ppo.laplacian(190, 151, 1), "ict", dict(threshold=1e-2, ordering=2)),
+    "ildlt_large": lambda: (ppo.laplacian(40, 31, 30), "ildlt", dict(tolerance=3e-3)),
+    "ilut_large": lambda: (ppo.upwind(43, 31, 29, 20.0, 10.0, 5.0), "ilut", dict(lfill=20, tolerance=1e-2)),
+    "ilu0_large": lambda: (ppo.upwind(43, 31, 29, 20.0, 10.0, 5.0), "ilu0", dict()),
+}
+
+
+@pytest.mark.parametrize("trsv,name", [(3, k) for k in CASES] + [(5, k) for k in [*CASES, *LARGE]])
+def test_sweeps_match_levels(pp, torch, trsv, name):
+    A, kind, kw = {**CASES, **LARGE}[name]()
     n = len(A[0]) - 1
-    print(f"[sweeps] {name} n={n}", flush=True)
+    print(f"[sweeps] {name} n={n} trsv={trsv}", flush=True)
     M = pp.CSRMatrix(*A)
     cls = {"ict": pp.IncompleteCholesky, "ildlt": pp.IncompleteLDLT, "ilut": pp.IncompleteLU, "ic0": pp.IC0,
            "ilu0": pp.ILU0}[kind]
-    P1, P3 = (cls(M, trsv=t, **kw) for t in (1, 3))
+    P1, P3 = (cls(M, trsv=t, **kw) for t in (1, trsv))
     P1.setup()
     P3.setup()
-    assert P1.info().trsv == 1 and P3.info().trsv == 3
+    if trsv == 5 and n == 1:
+        assert P3.info().trsv in (1, 5)
+    else:
+        assert P1.info().trsv == 1 and P3.info().trsv == trsv
     rng = np.random.default_rng(n)
     x = rng.standard_normal(n)
     x[rng.random(n) < 0.2] = 0.0   # zeros of both signs take the division itself
@@ -112,3 +128,35 @@ def test_block_sweep_quotients(pp, torch):
         want, got = P1.MInvSolve(v.clone()), P3.MInvSolve(v.clone())
         same = (bits(torch, want) == bits(torch, got)) | (torch.isnan(want) & torch.isnan(got))
         assert bool(same.all()), int((~same).sum())
+
+
+@pytest.mark.parametrize("launch", [0, 1])  # captured bodies replayed, bodies launched on the stream
+@pytest.mark.parametrize("kind", ["cg", "cg_mixed", "gmres"])
+def test_strip_solves_match_levels(pp, torch, kind, launch):
+    # whole solves, twice each: the exchange buffers are empty again for every apply
+    A = ppo.upwind(33, 31, 29, 20.0, 10.0, 5.0) if kind == "gmres" else ppo.laplacian(33, 31, 29)
+    n = len(A[0]) - 1
+    M = pp.CSRMatrix(*A)
+    b = torch.tensor(ppo.spmv(A, ppo.uniform(n, 4)), device="cuda")
+    out = []
+    for trsv in (1, 5, 0):
+        if kind == "gmres":
+            P = pp.IncompleteLU(M, 20, 1e-2, trsv=trsv)
+        else:
+            P = pp.IncompleteCholesky(M, 1e-2, trsv=trsv, make_f32=kind == "cg_mixed")
+        P.setup()
+        assert P.info().trsv == trsv or (trsv == 0 and P.info().trsv in (1, 5))
+        for _ in range(2):
+            if kind == "gmres":
+                s = pp.GMRES(n, P, 1e-8, pp.FlexibleGMRES, maxIter=3000)
+                s.setRestart(True, 30)
+            else:
+                s = pp.CG(n, P, pp.FlexibleCG, tol=1e-8, maxIter=1000,
+                          precision="mixed" if kind == "cg_mixed" else "fp64")
+            s.opts.launch = launch
+            x = torch.zeros(n, dtype=torch.float64, device="cuda")
+            s.solve(M, b, x)
+            assert s.getConvergence()
+            out.append((s.getNumIter(), x))
+    for it, x in out[1:]:
+        assert it == out[0][0] and torch.equal(x, out[0][1])
