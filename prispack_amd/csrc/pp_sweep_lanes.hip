@@ -9,13 +9,14 @@
 // write, and the instructions around them, which one wavefront issues at one
 // per four cycles or so.  So the rows are scheduled on the host into steps
 // that one wavefront executes in lockstep without any barrier (LDS accesses
-// of a wavefront stay in order); a row is spread over several lanes, which
+// of a wavefront stay in order); a row may be spread over several lanes, which
 // gather and multiply its entries at once; every step's data comes in a
 // ready-to-use layout, loaded kLaneAhead steps ahead; and divisions go by
 // the pivots' reciprocals (five operations, same bits).  An apply of that
-// factor takes 0.45 ms in FP64 (0.19 us a step); one workgroup barrier and
+// factor takes 0.42 ms in FP64 (0.18 us a step); one workgroup barrier and
 // one LDS round trip more per level, with data loaded one level ahead, took
-// 2.0 ms (1.0 us a level).
+// 2.0 ms (1.0 us a level).  Rows of several parts kept in consecutive steps,
+// their sums carried in registers, took 0.45 ms (flags and selects a step).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,26 +36,22 @@ namespace {
 constexpr int kAhead = kLaneAhead;  // steps whose data is in flight or in registers
 constexpr int kLaneThreads = 256;
 constexpr uint32_t kExtra = 1;      // LDS words past the chunk's rows: a zero
-
-// Flags of a step, the same in all its lanes: the first, the last of its rows' steps.
-// From bit kNeedShift on: what a strip's step waits for (how many imports, in
-// units of kNeedUnit, must be there before it).
-enum : uint32_t { F_FIRST = 1, F_LAST = 2 };
-constexpr int kNeedShift = 2;
-constexpr uint32_t kNeedUnit = 8;
+constexpr uint32_t kNeedUnit = 8;   // a strip's step waits for so many imports at a time
+constexpr uint32_t kNoExport = 0xffffu;
 
 // What a lane needs of one step: 16-byte pieces, piece k of the step's
-// `active` lanes contiguous, so every load is one coalesced 16-byte load per lane.
+// active lanes contiguous, so every load is one coalesced 16-byte load per lane.
 //   values   S values of T
-//   indices  S 16-bit LDS words of the dependencies, then the row's word, the
-//            flags, the step's active lanes, the active lanes kAhead steps later
-//            and (S = 8) the row's 32-bit exchange slot or kNoSlot
+//   indices  16 bits each: the S dependencies' LDS words; the row's word; the
+//            imports the step waits for (kNeedUnit each, strips only); the
+//            step's rows - 1 and those of the step kAhead later (8 bits each);
+//            the row's export number in its strip or kNoExport
 //   pivot    the row's diagonal and its reciprocal rounded to FP64
-constexpr uint32_t kNoSlot = 0xffffffffu;
 template <class T, int S>
 struct Step {
     static constexpr int kVal = S * (int)sizeof(T) / 16, kIdx = (2 * S + 8 + 15) / 16;
     static constexpr int kPieces = kVal + kIdx + 1;
+    static constexpr int kRowWord = S / 2, kInfoWord = S / 2 + 1;  // 32-bit words of the indices
     int4 p[kPieces];
     __device__ static int word(const int4 &q, int w) { return w == 0 ? q.x : w == 1 ? q.y : w == 2 ? q.z : q.w; }
     __device__ T v(int j) const {
@@ -121,7 +118,7 @@ template <int CTRL>
 __device__ inline float dpp(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
-constexpr int kRowShl = 0x100, kRowShr = 0x110;  // DPP: lane i takes lane i + n, i - n of its 16
+constexpr int kRowShr = 0x110;  // DPP: lane i takes lane i - n of its 16
 
 // Word h (0 low, 1 high) of a pair of 16-bit LDS words, as a byte offset.
 template <class T, int H>
@@ -173,7 +170,7 @@ struct StepAddr {
             dep[j] = lds_byte<T, 0>(q.ix(j / 2));
             dep[j + 1] = lds_byte<T, 1>(q.ix(j / 2));
         }
-        row = lds_byte<T, 0>(q.ix(S / 2));
+        row = lds_byte<T, 0>(q.ix(Step<T, S>::kRowWord));
     }
 };
 
@@ -181,46 +178,40 @@ struct StepAddr {
 template <class T, int S>
 struct Carry {
     StepAddr<T, S> addr;  // of the next step
-    uint32_t flags;       // of the next step
+    uint32_t need;        // imports the next step waits for
     uint32_t active;      // lanes of the step kAhead - 1 past the next one
-    T t;                  // the rows' sums after the last step
 };
 
-// Step k, its data in q: G lanes a row, S entries a lane, in storage order
+// One step, its data in q: G lanes a row, S entries a lane, in storage order
 // along the row's lanes.  Every lane gathers and multiplies its entries at
 // once; the subtractions follow one after another, the partial sum moving
 // from lane to lane (DPP), so the row's operations are those of the serial
-// sweep.  The gathers go out first: while they are on their way, the loads
-// of step k + kAhead - 1 (into `past`, step k - 1's slot) are issued and the
-// next step's addresses unpacked.
-// xchg.wait(need) returns once the step's imports are in LDS, xchg.put
-// passes a finished row on.
+// sweep.  A row of more than G S entries is several such parts, each in a
+// step of its own: the partial sum waits in the row's LDS word, and a part
+// whose diagonal operation is not due holds the pivot 1 (s / 1 and s * 1 are
+// s).  The gathers go out first: while they are on their way, the loads of
+// the step kAhead - 1 later (into `past`, the last step's slot) are issued
+// and the next step's addresses unpacked.  xchg.wait(need) returns once the
+// step's imports are in LDS, xchg.put passes a finished row on.
 template <class T, int W, int G, int S, int MODE, class Xchg>
 __device__ inline void run_step(const Step<T, S> &q, const Step<T, S> &next, Step<T, S> &past, const char *&p,
                                 Carry<T, S> &c, uint32_t lane, uint32_t tail_lane, Xchg &xchg) {
 #pragma clang fp contract(off)
-    const uint32_t flags = c.flags;
-    xchg.wait(flags >> kNeedShift);
+    xchg.wait(c.need);
     T x[S];
 #pragma unroll
     for (int j = 0; j < S; ++j) x[j] = *lds_word<T>(c.addr.dep[j]);
     LdsWord<T> *mine = lds_word<T>(c.addr.row);
-    const T rhs = *mine;
+    T s = *mine;
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     load_step<T, S>(past, p, c.active, lane);
-    const uint32_t active = (uint32_t)__builtin_amdgcn_readfirstlane(q.ix(S / 2 + 1));
+    const uint32_t info = (uint32_t)__builtin_amdgcn_readfirstlane(q.ix(Step<T, S>::kInfoWord));
+    c.active = ((info >> 8 & 0xffu) + 1) * G;
     c.addr.set(next);
-    c.flags = (uint32_t)__builtin_amdgcn_readfirstlane(next.ix(S / 2)) >> 16;
-    c.active = active >> 16;
+    if constexpr (Xchg::kOn) c.need = (uint32_t)__builtin_amdgcn_readfirstlane(next.ix(Step<T, S>::kRowWord)) >> 16;
     __builtin_amdgcn_sched_barrier(0);
-    T s = rhs;
-    if (flags & F_FIRST) {
-        if constexpr (MODE == HostSweep::PREDIVIDE) s = quotient(s, q.d(), q.rcp());
-    } else {
-        if constexpr (G > 1) s = dpp<kRowShl + G - 1>(c.t);
-        else s = c.t;
-    }
+    if constexpr (MODE == HostSweep::PREDIVIDE) s = quotient(s, q.d(), q.rcp());
 #pragma unroll
     for (int j = 0; j < S; ++j) x[j] = q.v(j) * x[j];
 #pragma unroll
@@ -229,22 +220,20 @@ __device__ inline void run_step(const Step<T, S> &q, const Step<T, S> &next, Ste
         for (int j = 0; j < S; ++j) s = s - x[j];
         if (g < G - 1) s = dpp<kRowShr + 1>(s);
     }
-    c.t = s;
-    if (flags & F_LAST) {
-        if constexpr (MODE == HostSweep::DIVIDE) s = quotient(s, q.d(), q.rcp());
-        else if constexpr (MODE == HostSweep::MULTIPLY) s = s * q.d();
-        if (tail_lane < (active & 0xffffu)) {
-            *mine = s;
-            xchg.put(q, s);
-        }
-        if constexpr (W > 1) __syncthreads();
+    if constexpr (MODE == HostSweep::DIVIDE) s = quotient(s, q.d(), q.rcp());
+    else if constexpr (MODE == HostSweep::MULTIPLY) s = s * q.d();
+    if (tail_lane < ((info & 0xffu) + 1) * G) {
+        *mine = s;
+        xchg.put((uint32_t)q.ix(Step<T, S>::kInfoWord) >> 16, s);
     }
+    if constexpr (W > 1) __syncthreads();
 }
 
 struct NoExchange {
+    static constexpr bool kOn = false;
     __device__ void wait(uint32_t) {}
-    template <class Q, class T>
-    __device__ void put(const Q &, T) {}
+    template <class T>
+    __device__ void put(uint32_t, T) {}
 };
 
 // Copies n elements between global memory and LDS, eight loads of a thread
@@ -286,207 +275,24 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
 #pragma unroll
         for (int a = 0; a < kAhead - 1; ++a) load_step<T, S>(q[a], p, head[c].active[a], lane);
         Carry<T, S> st;
-        st.t = 0;
         st.active = head[c].active[kAhead - 1];
         st.addr.set(q[0]);
-        st.flags = (uint32_t)__builtin_amdgcn_readfirstlane(q[0].ix(S / 2)) >> 16;
-        NoExchange no_xchg;
+        NoExchange xchg;
         for (uint32_t k = 0; k < lo; ++k) {
 #pragma unroll
             for (int a = 0; a < kAhead; ++a)
                 run_step<T, W, G, S, MLO>(q[a], q[(a + 1) % kAhead], q[(a + kAhead - 1) % kAhead], p, st, lane,
-                                          tail_lane, no_xchg);
+                                          tail_lane, xchg);
         }
         for (uint32_t k = 0; k < up; ++k) {
 #pragma unroll
             for (int a = 0; a < kAhead; ++a)
                 run_step<T, W, G, S, MUP>(q[a], q[(a + 1) % kAhead], q[(a + kAhead - 1) % kAhead], p, st, lane,
-                                          tail_lane, no_xchg);
+                                          tail_lane, xchg);
         }
     }
     __syncthreads();
     copy_rows(y + r0, xs, nr);
-}
-
-// Rows of one chunk in the order and grouping of its steps.
-struct LanePlan {
-    struct Group {
-        uint32_t first, count, steps;  // rows[first, first + count), each taking `steps` steps
-    };
-    std::vector<uint32_t> rows;
-    std::vector<Group> groups;
-    uint32_t steps = 0;
-};
-
-// Groups the rows [r0, r1) of a sweep: a group holds at most `width` rows
-// whose dependencies all lie in earlier groups, the rows with the longest
-// chains behind them first (list scheduling), so the groups are about as few
-// as the longest chain, or the rows over `width`, allows.  A row of more
-// entries than one step takes runs over several steps; a group takes only
-// rows of at most its first row's steps.
-LanePlan plan_chunk(const HostSweep &s, uint32_t r0, uint32_t r1, uint32_t width, uint32_t entries) {
-    const uint32_t n = r1 - r0;
-    LanePlan P;
-    std::vector<uint32_t> ns(n), wait(n), sp(n + 1, 0), sc, height(n, 0);
-    for (uint32_t i = 0; i < n; ++i) {
-        const uint32_t a = s.rp[r0 + i], b = s.rp[r0 + i + 1];
-        ns[i] = std::max(1u, (b - a + entries - 1) / entries);
-        wait[i] = b - a;
-        for (uint32_t e = a; e < b; ++e) sp[s.ci[e] - r0 + 1]++;
-    }
-    for (uint32_t i = 0; i < n; ++i) sp[i + 1] += sp[i];
-    sc.resize(sp[n]);
-    {
-        std::vector<uint32_t> at(sp.begin(), sp.end() - 1);
-        for (uint32_t i = 0; i < n; ++i)
-            for (uint32_t e = s.rp[r0 + i]; e < s.rp[r0 + i + 1]; ++e) sc[at[s.ci[e] - r0]++] = i;
-    }
-    // dependents of a row come after it (lower) or before it (upper)
-    for (uint32_t k = 0; k < n; ++k) {
-        const uint32_t i = s.lower ? n - 1 - k : k;
-        uint32_t h = 0;
-        for (uint32_t e = sp[i]; e < sp[i + 1]; ++e) h = std::max(h, height[sc[e]]);
-        height[i] = h + ns[i];
-    }
-    auto less = [&](uint32_t a, uint32_t b) { return height[a] != height[b] ? height[a] < height[b] : a > b; };
-    std::priority_queue<uint32_t, std::vector<uint32_t>, decltype(less)> ready(less);
-    for (uint32_t i = 0; i < n; ++i)
-        if (!wait[i]) ready.push(i);
-    P.rows.reserve(n);
-    std::vector<uint32_t> skipped;
-    while (!ready.empty()) {
-        LanePlan::Group g{(uint32_t)P.rows.size(), 0, ns[ready.top()]};
-        skipped.clear();
-        while (!ready.empty() && g.count < width) {
-            const uint32_t i = ready.top();
-            ready.pop();
-            if (ns[i] > g.steps) {
-                skipped.push_back(i);
-                continue;
-            }
-            P.rows.push_back(i);
-            ++g.count;
-        }
-        for (uint32_t i : skipped) ready.push(i);
-        for (uint32_t k = g.first; k < g.first + g.count; ++k) {
-            const uint32_t i = P.rows[k];
-            for (uint32_t e = sp[i]; e < sp[i + 1]; ++e)
-                if (--wait[sc[e]] == 0) ready.push(sc[e]);
-        }
-        P.groups.push_back(g);
-        P.steps += g.steps;
-    }
-    return P;
-}
-
-// A chunk's steps: what each holds, before it is written out.
-struct StepRef {
-    const HostSweep *sweep;  // nullptr: idle (fills a sweep's last round)
-    uint32_t row, count, part, parts;  // plan rows [row, row + count), step `part` of their `parts`
-    const LanePlan *plan;
-    uint32_t need;           // imports (kNeedUnit each) it waits for
-};
-
-void append_steps(const HostSweep &s, const LanePlan &P, std::vector<StepRef> &out) {
-    for (const auto &g : P.groups)
-        for (uint32_t k = 0; k < g.steps; ++k) out.push_back({&s, g.first, g.count, k, g.steps, &P, 0});
-    while (out.size() % kAhead) out.push_back({nullptr, 0, 0, 0, 0, nullptr, 0});
-}
-
-// One step at `out` (zeroed), `active` lanes; ahead: the lanes kAhead steps later.
-// word(row): the LDS word of a dependency; slot: the exchange slots of all
-// rows (kNoSlot: none), or nullptr.
-template <class T, int S, class Word>
-void write_step(const StepRef &r, uint32_t r0, uint32_t nr, int G, uint32_t active, uint32_t ahead,
-                unsigned char *out, const Word &word, const uint32_t *slot = nullptr) {
-    using St = Step<T, S>;
-    const size_t piece = (size_t)active * 16;
-    for (uint32_t l = 0; l < active; ++l) {
-        T v[S] = {}, d = T(1);
-        uint16_t ix[St::kIdx * 8] = {};
-        uint32_t flags = 0;
-        if (r.sweep) {
-            const HostSweep &s = *r.sweep;
-            const uint32_t i = r.plan->rows[r.row + l / G];
-            const uint32_t a = s.rp[r0 + i] + (r.part * G + l % G) * S, b = s.rp[r0 + i + 1];
-            for (int j = 0; j < S; ++j) {
-                const bool has = a + j < b;
-                if (has) v[j] = (T)s.val[a + j];
-                ix[j] = (uint16_t)(has ? word(s.ci[a + j]) : nr);  // word nr holds a zero
-            }
-            ix[S] = (uint16_t)i;
-            if constexpr (S == 8) {
-                const uint32_t to = slot ? slot[r0 + i] : kNoSlot;
-                ix[S + 4] = (uint16_t)to;
-                ix[S + 5] = (uint16_t)(to >> 16);
-            }
-            flags = (r.part == 0 ? F_FIRST : 0u) | (r.part + 1 == r.parts ? F_LAST : 0u);
-            if (s.mode != HostSweep::UNIT) d = (T)s.diag[r0 + i];
-        }
-        ix[S + 1] = (uint16_t)(flags | r.need << kNeedShift);
-        ix[S + 2] = (uint16_t)active;
-        ix[S + 3] = (uint16_t)ahead;
-        const double rcp = step_reciprocal<T>(d);
-        for (int q = 0; q < St::kVal; ++q) std::memcpy(out + q * piece + 16 * l, (unsigned char *)v + 16 * q, 16);
-        for (int q = 0; q < St::kIdx; ++q)
-            std::memcpy(out + (St::kVal + q) * piece + 16 * l, (unsigned char *)ix + 16 * q, 16);
-        unsigned char *pv = out + (St::kPieces - 1) * piece + 16 * l;
-        std::memset(pv, 0, 8);
-        std::memcpy(pv, &d, sizeof(T));
-        std::memcpy(pv + 8, &rcp, 8);
-    }
-}
-
-template <class T, int S>
-void build_steps(const HostSweep &lo, const HostSweep &up, const ChunkSet &C, int W, int G, LaneSweep<T> &L) {
-    std::vector<LanePlan> pl(C.nchunk), pu(C.nchunk);
-    std::vector<LaneHead> head(C.nchunk);
-    std::vector<std::vector<StepRef>> steps(C.nchunk);
-    auto lanes = [&](const std::vector<StepRef> &v, size_t k) {
-        return k < v.size() && v[k].sweep ? v[k].count * (uint32_t)G : 1u;
-    };
-    parallel_for(C.nchunk, 1, [&](size_t c0, size_t c1) {
-        for (size_t c = c0; c < c1; ++c) {
-            pl[c] = plan_chunk(lo, C.start[c], C.start[c + 1], 64 * W / G, G * S);
-            pu[c] = plan_chunk(up, C.start[c], C.start[c + 1], 64 * W / G, G * S);
-            append_steps(lo, pl[c], steps[c]);
-            head[c].rounds_lo = (uint32_t)steps[c].size() / kAhead;
-            append_steps(up, pu[c], steps[c]);
-            head[c].rounds_up = (uint32_t)steps[c].size() / kAhead - head[c].rounds_lo;
-        }
-    });
-    constexpr size_t kLane = (size_t)Step<T, S>::kPieces * 16;
-    uint64_t total = 0;
-    for (uint32_t c = 0; c < C.nchunk; ++c) {
-        head[c].first = total;
-        for (int a = 0; a < kAhead; ++a) head[c].active[a] = lanes(steps[c], a);
-        for (size_t k = 0; k < steps[c].size(); ++k) total += kLane * lanes(steps[c], k);
-    }
-    // the loads past the last chunk's steps: kAhead steps of one lane
-    const uint64_t spare = kLane * kAhead;
-    std::unique_ptr<unsigned char[]> host(new unsigned char[total + spare]);
-    std::memset(host.get() + total, 0, spare);
-    parallel_for(C.nchunk, 1, [&](size_t c0, size_t c1) {
-        for (size_t c = c0; c < c1; ++c) {
-            const uint32_t r0 = C.start[c], nr = C.start[c + 1] - r0;
-            unsigned char *p = host.get() + head[c].first;
-            for (size_t k = 0; k < steps[c].size(); ++k) {
-                const uint32_t active = lanes(steps[c], k);
-                write_step<T, S>(steps[c][k], r0, nr, G, active, lanes(steps[c], k + kAhead), p,
-                                 [r0](uint32_t j) { return j - r0; });
-                p += kLane * active;
-            }
-        }
-    });
-    L.data = dalloc<unsigned char>(total + spare);
-    L.head = (LaneHead *)dalloc<unsigned char>(std::max<size_t>(1, head.size()) * sizeof(LaneHead));
-    PP_HIP(hipMemcpy(L.data, host.get(), total + spare, hipMemcpyHostToDevice));
-    PP_HIP(hipMemcpy(L.head, head.data(), head.size() * sizeof(LaneHead), hipMemcpyHostToDevice));
-    L.waves = W;
-    L.group = G;
-    L.slots = S;
-    L.mode_lo = lo.mode;
-    L.mode_up = up.mode;
 }
 
 // ---------------------------------------------------------------------------
@@ -526,6 +332,7 @@ struct StripHead {
     LaneHead lanes;                 // rounds_lo: all of the sweep's rounds
     uint32_t row = 0, rows = 0;
     uint32_t imp = 0, nimp = 0;     // imports: slots, by the step that first needs them
+    uint32_t exp = 0;               // first slot of its exported rows
 };
 
 // control words in LDS (not through a generic pointer: a flat access would
@@ -535,8 +342,9 @@ using CtlWord = volatile __attribute__((address_space(3))) uint32_t;
 // Wavefront 0's side of the exchange.
 template <class T>
 struct Exchange {
+    static constexpr bool kOn = true;
     CtlWord *cw;
-    T *slots;
+    T *slots;       // the strip's own
     uint32_t have;  // imports known to be in LDS
     __device__ void wait(uint32_t need) {
         while (have < need * kNeedUnit) {
@@ -547,12 +355,10 @@ struct Exchange {
             have = (uint32_t)__builtin_amdgcn_readfirstlane(done);
         }
     }
-    template <class Q>
-    __device__ void put(const Q &q, T s) {
+    __device__ void put(uint32_t number, T s) {
         using U = typename SlotBits<T>::U;
-        const uint32_t to = (uint32_t)q.ix(6);
-        if (to != kNoSlot)
-            __hip_atomic_store(reinterpret_cast<U *>(slots) + to, __builtin_bit_cast(U, s), __ATOMIC_RELAXED,
+        if (number != kNoExport)
+            __hip_atomic_store(reinterpret_cast<U *>(slots) + number, __builtin_bit_cast(U, s), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
     }
 };
@@ -570,7 +376,6 @@ template <class T, int G, int S, int MODE>
 __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_sweep_strips(
     const StripHead *__restrict__ heads, const char *data, const uint32_t *__restrict__ imp, T *slots,
     uint32_t other_n, T *other, uint32_t ctl_off, const T *x, T *y, long long deadline, int *ctl, const int *stop) {
-    static_assert(S == 8, "the steps carry exchange slots");
     using U = typename SlotBits<T>::U;
     constexpr U kEmpty = SlotBits<T>::empty;
     extern __shared__ unsigned char lds_raw[];
@@ -594,11 +399,10 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
 #pragma unroll
         for (int a = 0; a < kAhead - 1; ++a) load_step<T, S>(q[a], p, h.lanes.active[a], lane);
         Carry<T, S> st;
-        st.t = 0;
         st.active = h.lanes.active[kAhead - 1];
         st.addr.set(q[0]);
-        st.flags = (uint32_t)__builtin_amdgcn_readfirstlane(q[0].ix(S / 2)) >> 16;
-        Exchange<T> xchg{cw, slots, 0};
+        st.need = (uint32_t)__builtin_amdgcn_readfirstlane(q[0].ix(S / 2)) >> 16;
+        Exchange<T> xchg{cw, slots + h.exp, 0};
         for (uint32_t k = 0; k < rounds; ++k) {
 #pragma unroll
             for (int a = 0; a < kAhead; ++a)
@@ -664,97 +468,236 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
     copy_rows(y + h.row, xs, nr);
 }
 
-// The strips' plans: list scheduling of all strips together, a step of every
-// strip at a time, a row of another strip visible kStripLag steps after its
-// step (the exchange takes about 1.5 us), so that the order in which a strip
-// takes its rows is one in which it rarely waits.
+// ---------------------------------------------------------------------------
+// Host: which rows go into which step.
+// ---------------------------------------------------------------------------
+
+// A row's entries [a, b) of one step (a row of more entries than a step's G S
+// is several parts, the remainder first, so that the last part, which the
+// rows after it wait for, holds as many of the latest dependencies as it can).
+struct Part {
+    uint32_t row, a, b;
+    bool first, last;
+};
+// The parts of one chunk or strip in the order of its steps.
+struct LanePlan {
+    struct Group {
+        uint32_t first, count;  // parts[first, first + count) make a step
+    };
+    std::vector<Part> parts;
+    std::vector<Group> steps;
+};
+
+// List scheduling of the rows [bound[0], bound.back()) of a sweep, all strips
+// [bound[k], bound[k + 1]) together, a step of every strip at a time: a step
+// takes up to `width` parts whose dependencies are visible, those with the
+// longest chains behind them first; so the steps are about as few as the
+// longest chain, or the parts over `width`, allows.  A row of another strip
+// is visible kStripLag steps after its step (the exchange takes about
+// 1.5 us), so the order in which a strip takes its rows is one in which it
+// rarely waits.  span: the steps until the last strip ends.
 constexpr uint32_t kStripLag = 10;
-std::vector<LanePlan> plan_strips(const HostSweep &s, const std::vector<uint32_t> &start, uint32_t width,
-                                  uint32_t entries) {
-    const uint32_t n = s.n, K = (uint32_t)start.size() - 1;
+std::vector<LanePlan> plan_steps(const HostSweep &s, const std::vector<uint32_t> &bound, uint32_t width,
+                                 uint32_t entries, uint32_t &span) {
+    const uint32_t K = (uint32_t)bound.size() - 1, r0 = bound[0], n = bound[K] - r0;
     std::vector<LanePlan> P(K);
-    std::vector<uint32_t> sp(n + 1, 0), sc(s.rp[n]), height(n, 0), ns(n), strip_of(n);
-    std::vector<int32_t> wait(n);
-    std::vector<uint32_t> at_time(n, 0);  // when the dependencies seen so far are visible
-    for (uint32_t k = 0; k < K; ++k) std::fill(strip_of.begin() + start[k], strip_of.begin() + start[k + 1], k);
+    span = 0;
+    if (!n) return P;
+    // parts, row after row; part[i] .. part[i + 1] are row r0 + i's
+    std::vector<uint32_t> part(n + 1, 0), strip_of(n);
+    for (uint32_t k = 0; k < K; ++k)
+        std::fill(strip_of.begin() + (bound[k] - r0), strip_of.begin() + (bound[k + 1] - r0), k);
+    for (uint32_t i = 0; i < n; ++i)
+        part[i + 1] = part[i] + std::max(1u, (s.rp[r0 + i + 1] - s.rp[r0 + i] + entries - 1) / entries);
+    const uint32_t np = part[n];
+    std::vector<Part> parts(np);
+    std::vector<uint32_t> wait(np), seen(np, 0), height(np), sp(n + 1, 0), sc(s.rp[r0 + n] - s.rp[r0]);
     for (uint32_t i = 0; i < n; ++i) {
-        wait[i] = (int32_t)(s.rp[i + 1] - s.rp[i]);
-        ns[i] = std::max(1u, ((uint32_t)wait[i] + entries - 1) / entries);
-        for (uint32_t e = s.rp[i]; e < s.rp[i + 1]; ++e) sp[s.ci[e] + 1]++;
+        const uint32_t m = part[i + 1] - part[i], e1 = s.rp[r0 + i + 1];
+        uint32_t a = s.rp[r0 + i], b = e1 - (m - 1) * entries;
+        for (uint32_t u = part[i]; u < part[i + 1]; ++u, a = b, b += entries) {
+            parts[u] = {r0 + i, a, b, u == part[i], u + 1 == part[i + 1]};
+            wait[u] = b - a + (u == part[i] ? 0 : 1);
+            for (uint32_t e = a; e < b; ++e) sp[s.ci[e] - r0 + 1]++;
+        }
     }
     for (uint32_t i = 0; i < n; ++i) sp[i + 1] += sp[i];
     {
         std::vector<uint32_t> at(sp.begin(), sp.end() - 1);
-        for (uint32_t i = 0; i < n; ++i)
-            for (uint32_t e = s.rp[i]; e < s.rp[i + 1]; ++e) sc[at[s.ci[e]]++] = i;
+        for (uint32_t u = 0; u < np; ++u)
+            for (uint32_t e = parts[u].a; e < parts[u].b; ++e) sc[at[s.ci[e] - r0]++] = u;
     }
+    auto strip = [&](uint32_t u) { return strip_of[parts[u].row - r0]; };
+    // dependents of a row come after it (lower) or before it (upper)
     for (uint32_t k = 0; k < n; ++k) {
         const uint32_t i = s.lower ? n - 1 - k : k;
         uint32_t h = 0;
         for (uint32_t e = sp[i]; e < sp[i + 1]; ++e)
-            h = std::max(h, height[sc[e]] + (strip_of[sc[e]] != strip_of[i] ? kStripLag : 0u));
-        height[i] = h + ns[i];
+            h = std::max(h, height[sc[e]] + (strip(sc[e]) != strip_of[i] ? kStripLag : 0u));
+        for (uint32_t u = part[i + 1]; u-- > part[i];) height[u] = ++h;
     }
     auto less = [&](uint32_t a, uint32_t b) { return height[a] != height[b] ? height[a] < height[b] : a > b; };
-    std::vector<std::vector<uint32_t>> ready(K), due;  // due[t]: rows whose dependencies are visible at step t
-    std::vector<uint32_t> busy(K, 0);
-    auto make_due = [&](uint32_t i, uint32_t t) {
+    std::vector<std::vector<uint32_t>> ready(K), due;  // due[t]: parts whose dependencies are visible at step t
+    auto make_due = [&](uint32_t u, uint32_t t) {
         if (t >= due.size()) due.resize(t + 1 + t / 2);
-        due[t].push_back(i);
+        due[t].push_back(u);
     };
-    for (uint32_t i = 0; i < n; ++i)
-        if (!wait[i]) make_due(i, 0);
-    std::vector<uint32_t> skipped, group;
-    uint32_t left = n;
+    for (uint32_t u = 0; u < np; ++u)
+        if (!wait[u]) make_due(u, 0);
+    uint32_t left = np;
     for (uint32_t t = 0; left; ++t) {
         if (t < due.size()) {
             std::vector<uint32_t> now;
             now.swap(due[t]);
-            for (uint32_t i : now) {
-                auto &q = ready[strip_of[i]];
-                q.push_back(i);
+            for (uint32_t u : now) {
+                auto &q = ready[strip(u)];
+                q.push_back(u);
                 std::push_heap(q.begin(), q.end(), less);
             }
         }
         for (uint32_t k = 0; k < K; ++k) {
             auto &q = ready[k];
-            if (busy[k] > t || q.empty()) continue;
+            if (q.empty()) continue;
             LanePlan &p = P[k];
-            LanePlan::Group g{(uint32_t)p.rows.size(), 0, ns[q.front()]};
-            skipped.clear();
+            LanePlan::Group g{(uint32_t)p.parts.size(), 0};
+            const auto visible = [&](uint32_t u, uint32_t at) {
+                seen[u] = std::max(seen[u], at);
+                if (--wait[u] == 0) make_due(u, seen[u]);
+            };
             while (!q.empty() && g.count < width) {
                 std::pop_heap(q.begin(), q.end(), less);
-                const uint32_t i = q.back();
+                const uint32_t u = q.back();
                 q.pop_back();
-                if (ns[i] > g.steps) {
-                    skipped.push_back(i);
-                    if (skipped.size() > 64) break;
+                p.parts.push_back(parts[u]);
+                ++g.count;
+                if (!parts[u].last) {
+                    visible(u + 1, t + 1);
                     continue;
                 }
-                p.rows.push_back(i - start[k]);
-                ++g.count;
+                const uint32_t i = parts[u].row - r0;
+                for (uint32_t e = sp[i]; e < sp[i + 1]; ++e)
+                    visible(sc[e], t + 1 + (strip(sc[e]) != k ? kStripLag : 0u));
             }
-            for (uint32_t i : skipped) {
-                q.push_back(i);
-                std::push_heap(q.begin(), q.end(), less);
-            }
-            busy[k] = t + g.steps;
             left -= g.count;
-            for (uint32_t r = g.first; r < g.first + g.count; ++r) {
-                const uint32_t i = p.rows[r] + start[k];
-                for (uint32_t e = sp[i]; e < sp[i + 1]; ++e) {
-                    const uint32_t j = sc[e], vis = t + g.steps + (strip_of[j] != k ? kStripLag : 0u);
-                    at_time[j] = std::max(at_time[j], vis);
-                    if (--wait[j] == 0) make_due(j, std::max(at_time[j], t + 1));
-                }
-            }
-            p.groups.push_back(g);
-            p.steps += g.steps;
+            p.steps.push_back(g);
         }
+        span = t + 1;
     }
     return P;
 }
 
+// A step to write: nullptr: idle (fills a sweep's last round).
+struct StepRef {
+    const HostSweep *sweep = nullptr;
+    const LanePlan *plan = nullptr;
+    LanePlan::Group group{0, 1};
+    uint32_t need = 0;  // imports (kNeedUnit each) it waits for
+};
+inline uint32_t rows_of(const std::vector<StepRef> &v, size_t k) { return k < v.size() ? v[k].group.count : 1u; }
+
+void append_steps(const HostSweep &s, const LanePlan &P, std::vector<StepRef> &out) {
+    for (const auto &g : P.steps) out.push_back({&s, &P, g, 0});
+    while (out.size() % kAhead) out.push_back({});
+}
+
+// One step at `out`, `rows` of it and `ahead` of the step kAhead later; its
+// LDS holds the rows from r0 on at words 0 .. nr - 1 and a zero at nr.
+// word(row): the LDS word of a dependency; number(row): its export number.
+template <class T, int S, class Word, class Number>
+void write_step(const StepRef &r, uint32_t r0, uint32_t nr, int G, uint32_t ahead, unsigned char *out,
+                const Word &word, const Number &number) {
+    using St = Step<T, S>;
+    const uint32_t rows = r.group.count, lanes = rows * G;
+    const size_t piece = (size_t)lanes * 16;
+    for (uint32_t l = 0; l < lanes; ++l) {
+        T v[S] = {}, d = T(1);
+        uint16_t ix[St::kIdx * 8];
+        std::fill(ix, ix + St::kIdx * 8, (uint16_t)nr);
+        uint32_t exported = kNoExport;
+        if (r.sweep) {
+            const HostSweep &s = *r.sweep;
+            const Part &q = r.plan->parts[r.group.first + l / G];
+            const uint32_t a = q.a + (l % G) * S;
+            for (int j = 0; j < S; ++j)
+                if (a + j < q.b) {
+                    v[j] = (T)s.val[a + j];
+                    ix[j] = (uint16_t)word(s.ci[a + j]);
+                }
+            ix[S] = (uint16_t)(q.row - r0);
+            if (s.mode == HostSweep::PREDIVIDE ? q.first : s.mode != HostSweep::UNIT && q.last) d = (T)s.diag[q.row];
+            if (q.last) exported = number(q.row);
+        }
+        ix[S + 1] = (uint16_t)r.need;
+        ix[S + 2] = (uint16_t)((rows - 1) | (ahead - 1) << 8);
+        ix[S + 3] = (uint16_t)exported;
+        const double rcp = step_reciprocal<T>(d);
+        for (int q = 0; q < St::kVal; ++q) std::memcpy(out + q * piece + 16 * l, (unsigned char *)v + 16 * q, 16);
+        for (int q = 0; q < St::kIdx; ++q)
+            std::memcpy(out + (St::kVal + q) * piece + 16 * l, (unsigned char *)ix + 16 * q, 16);
+        unsigned char *pv = out + (St::kPieces - 1) * piece + 16 * l;
+        std::memset(pv, 0, 8);
+        std::memcpy(pv, &d, sizeof(T));
+        std::memcpy(pv + 8, &rcp, 8);
+    }
+}
+
+// Byte offset and lane counts of every chunk's or strip's steps; returns the total.
+template <class Head>
+uint64_t place_steps(const std::vector<std::vector<StepRef>> &steps, int G, size_t lane_bytes, std::vector<Head> &head,
+                     LaneHead &(*lanes)(Head &)) {
+    uint64_t total = 0;
+    for (size_t c = 0; c < steps.size(); ++c) {
+        LaneHead &h = lanes(head[c]);
+        h.first = total;
+        for (int a = 0; a < kAhead; ++a) h.active[a] = rows_of(steps[c], a) * G;
+        for (size_t k = 0; k < steps[c].size(); ++k) total += lane_bytes * G * rows_of(steps[c], k);
+    }
+    return total;
+}
+
+template <class T, int S>
+void build_steps(const HostSweep &lo, const HostSweep &up, const ChunkSet &C, int W, int G, LaneSweep<T> &L) {
+    std::vector<LanePlan> pl(C.nchunk), pu(C.nchunk);
+    std::vector<LaneHead> head(C.nchunk);
+    std::vector<std::vector<StepRef>> steps(C.nchunk);
+    parallel_for(C.nchunk, 1, [&](size_t c0, size_t c1) {
+        for (size_t c = c0; c < c1; ++c) {
+            uint32_t span;
+            pl[c] = std::move(plan_steps(lo, {C.start[c], C.start[c + 1]}, 64 * W / G, G * S, span)[0]);
+            pu[c] = std::move(plan_steps(up, {C.start[c], C.start[c + 1]}, 64 * W / G, G * S, span)[0]);
+            append_steps(lo, pl[c], steps[c]);
+            head[c].rounds_lo = (uint32_t)steps[c].size() / kAhead;
+            append_steps(up, pu[c], steps[c]);
+            head[c].rounds_up = (uint32_t)steps[c].size() / kAhead - head[c].rounds_lo;
+        }
+    });
+    constexpr size_t kLane = (size_t)Step<T, S>::kPieces * 16;
+    const uint64_t total = place_steps<LaneHead>(steps, G, kLane, head, [](LaneHead &h) -> LaneHead & { return h; });
+    // the loads past the last chunk's steps: kAhead steps of one row
+    const uint64_t spare = kLane * G * kAhead;
+    std::unique_ptr<unsigned char[]> host(new unsigned char[total + spare]);
+    std::memset(host.get() + total, 0, spare);
+    parallel_for(C.nchunk, 1, [&](size_t c0, size_t c1) {
+        for (size_t c = c0; c < c1; ++c) {
+            const uint32_t r0 = C.start[c], nr = C.start[c + 1] - r0;
+            unsigned char *p = host.get() + head[c].first;
+            for (size_t k = 0; k < steps[c].size(); ++k) {
+                write_step<T, S>(steps[c][k], r0, nr, G, rows_of(steps[c], k + kAhead), p,
+                                 [r0](uint32_t j) { return j - r0; }, [](uint32_t) { return kNoExport; });
+                p += kLane * G * rows_of(steps[c], k);
+            }
+        }
+    });
+    L.data = dalloc<unsigned char>(total + spare);
+    L.head = (LaneHead *)dalloc<unsigned char>(std::max<size_t>(1, head.size()) * sizeof(LaneHead));
+    PP_HIP(hipMemcpy(L.data, host.get(), total + spare, hipMemcpyHostToDevice));
+    PP_HIP(hipMemcpy(L.head, head.data(), head.size() * sizeof(LaneHead), hipMemcpyHostToDevice));
+    L.waves = W;
+    L.group = G;
+    L.slots = S;
+    L.mode_lo = lo.mode;
+    L.mode_up = up.mode;
+}
 
 // LDS words of the largest strip: its rows, a zero, the rows it imports.
 uint32_t strip_words(const HostSweep &s, const std::vector<uint32_t> &start) {
@@ -780,83 +723,72 @@ struct StripHost {
     std::vector<uint32_t> imp;
     std::unique_ptr<unsigned char[]> data;
     uint64_t bytes = 0;
-    uint32_t nslots = 0, max_words = 0;
+    uint32_t nslots = 0, max_words = 0, span = 0;
 };
 
 template <class T, int S>
 void build_strips_host(const HostSweep &s, const std::vector<uint32_t> &start, int G, StripHost<T> &D) {
     const uint32_t K = (uint32_t)start.size() - 1, n = s.n;
-    std::vector<LanePlan> P = plan_strips(s, start, 64 / G, G * S);
+    std::vector<LanePlan> P = plan_steps(s, start, 64 / G, G * S, D.span);
     std::vector<StripHead> &head = D.head;
     head.resize(K);
     std::vector<std::vector<StepRef>> steps(K);
-    std::vector<std::vector<uint32_t>> imports(K);          // rows, in the order their values are needed
+    std::vector<std::vector<uint32_t>> imports(K);  // rows, in the order their values are needed
     std::vector<std::unordered_map<uint32_t, uint32_t>> word(K);
     parallel_for(K, 1, [&](size_t k0, size_t k1) {
         for (size_t k = k0; k < k1; ++k) {
             const uint32_t r0 = start[k], r1 = start[k + 1], nr = r1 - r0;
-            for (const auto &g : P[k].groups) {
-                for (uint32_t r = g.first; r < g.first + g.count; ++r) {
-                    const uint32_t i = r0 + P[k].rows[r];
-                    for (uint32_t e = s.rp[i]; e < s.rp[i + 1]; ++e) {
+            for (const auto &g : P[k].steps) {
+                for (uint32_t u = g.first; u < g.first + g.count; ++u) {
+                    const Part &q = P[k].parts[u];
+                    for (uint32_t e = q.a; e < q.b; ++e) {
                         const uint32_t j = s.ci[e];
                         if (j >= r0 && j < r1) continue;
                         if (word[k].emplace(j, nr + 1 + (uint32_t)imports[k].size()).second) imports[k].push_back(j);
                     }
                 }
-                const uint32_t need = ((uint32_t)imports[k].size() + kNeedUnit - 1) / kNeedUnit;
-                for (uint32_t q = 0; q < g.steps; ++q) steps[k].push_back({&s, g.first, g.count, q, g.steps, &P[k], need});
+                steps[k].push_back({&s, &P[k], g, ((uint32_t)imports[k].size() + kNeedUnit - 1) / kNeedUnit});
             }
-            while (steps[k].size() % kAhead)
-                steps[k].push_back({nullptr, 0, 0, 0, 0, nullptr, 0});
+            while (steps[k].size() % kAhead) steps[k].push_back({});
         }
     });
-    // exchange slots: the imported rows, numbered strip by strip in the order
-    // their steps finish them
-    std::vector<uint32_t> slot(n, kNoSlot);
-    std::vector<uint32_t> &imp = D.imp;
-    uint32_t &nslots = D.nslots;
+    // exchange slots: each strip's imported rows, numbered in the order its
+    // steps finish them
+    constexpr uint32_t kUnused = 0xffffffffu, kUsed = 0xfffffffeu;
+    std::vector<uint32_t> slot(n, kUnused);
     for (uint32_t k = 0; k < K; ++k)
-        for (uint32_t j : imports[k]) slot[j] = kNoSlot - 1;  // to be numbered
+        for (uint32_t j : imports[k]) slot[j] = kUsed;
     for (uint32_t k = 0; k < K; ++k) {
         head[k].row = start[k];
         head[k].rows = start[k + 1] - start[k];
-        for (uint32_t r : P[k].rows)
-            if (slot[start[k] + r] != kNoSlot) slot[start[k] + r] = nslots++;
+        head[k].exp = D.nslots;
+        for (const Part &q : P[k].parts)
+            if (q.last && slot[q.row] == kUsed) slot[q.row] = D.nslots++;
     }
     for (uint32_t k = 0; k < K; ++k) {
-        head[k].imp = (uint32_t)imp.size();
+        head[k].imp = (uint32_t)D.imp.size();
         head[k].nimp = (uint32_t)imports[k].size();
-        for (uint32_t j : imports[k]) imp.push_back(slot[j]);
+        for (uint32_t j : imports[k]) D.imp.push_back(slot[j]);
         D.max_words = std::max(D.max_words, head[k].rows + 1 + head[k].nimp);
+        head[k].lanes.rounds_lo = (uint32_t)steps[k].size() / kAhead;
     }
     constexpr size_t kLane = (size_t)Step<T, S>::kPieces * 16;
-    auto lanes = [&](const std::vector<StepRef> &v, size_t k) {
-        return k < v.size() && v[k].sweep ? v[k].count * (uint32_t)G : 1u;
-    };
-    uint64_t total = 0;
-    for (uint32_t k = 0; k < K; ++k) {
-        LaneHead &h = head[k].lanes;
-        h.first = total;
-        h.rounds_lo = (uint32_t)steps[k].size() / kAhead;
-        for (int a = 0; a < kAhead; ++a) h.active[a] = lanes(steps[k], a);
-        for (size_t q = 0; q < steps[k].size(); ++q) total += kLane * lanes(steps[k], q);
-    }
-    const uint64_t spare = kLane * kAhead;
+    const uint64_t total = place_steps<StripHead>(steps, G, kLane, head, [](StripHead &h) -> LaneHead & { return h.lanes; });
+    const uint64_t spare = kLane * G * kAhead;
     D.bytes = total + spare;
     D.data.reset(new unsigned char[D.bytes]);
     std::memset(D.data.get() + total, 0, spare);
     parallel_for(K, 1, [&](size_t k0, size_t k1) {
         for (size_t k = k0; k < k1; ++k) {
-            const uint32_t r0 = start[k], r1 = start[k + 1];
+            const uint32_t r0 = start[k], r1 = start[k + 1], exp0 = head[k].exp;
             const auto &w = word[k];
             unsigned char *p = D.data.get() + head[k].lanes.first;
             for (size_t q = 0; q < steps[k].size(); ++q) {
-                const uint32_t active = lanes(steps[k], q);
-                write_step<T, S>(steps[k][q], r0, r1 - r0, G, active, lanes(steps[k], q + kAhead), p, [&](uint32_t j) {
-                    return j >= r0 && j < r1 ? j - r0 : w.find(j)->second;
-                }, slot.data());
-                p += kLane * active;
+                write_step<T, S>(
+                    steps[k][q], r0, r1 - r0, G, rows_of(steps[k], q + kAhead), p,
+                    [&](uint32_t j) { return j >= r0 && j < r1 ? j - r0 : w.find(j)->second; },
+                    [&](uint32_t j) { return slot[j] == kUnused ? kNoExport : slot[j] - exp0; });
+                p += kLane * G * rows_of(steps[k], q);
             }
         }
     });
@@ -924,44 +856,80 @@ uint32_t lane_sweep_max_rows(size_t lds) {
     return (uint32_t)std::min<size_t>(lds / sizeof(double) - kExtra, 65535 - kExtra);
 }
 
-// The shapes of a step, and what one took on MI355X (us; single wave of
-// 2.4 GHz; ICT(1e-3) and ICT(1e-2) of the 128^2 Poisson problem, ICT(3e-3) of
-// 27^3, 4 to 13 entries a row; FP32 5 to 10% less).  One wavefront needs no
-// barrier; four pay about 0.1 us for it, and win where levels are wide.  A
-// lane's fixed work (loads, addresses, flags: about 50 instructions, which
-// issue one in four cycles) is shared by the rows and entries a step holds,
-// so the shape that needs the fewest steps for its price wins.
+// The shapes of a step, and what one took on MI355X (us, FP64: ICT(1e-3) and
+// ICT(1e-2) of the 128^2 Poisson problem, ICT(3e-3) of 27^3, ILDLT of 16
+// blocks; without divisions 0.03 less, FP32 5 to 10% less).  About half of a
+// step is fixed work (loads, addresses: 40 instructions of about four cycles
+// each), shared by the rows and entries it holds; one wavefront needs no
+// barrier, four pay about 0.1 us for it and win where many rows are ready at
+// a time.  So the shape that needs the fewest steps for its price wins:
+//   128^2 ICT(1e-3), 1012 levels of 16 rows, 13 entries a row, apply in us:
+//     {1,1,4} 500, {1,1,8} 514, {1,4,4} 415, {1,2,8} 459, {4,4,4} 602
+//   128^2 ICT(1e-2), 509 levels of 32 rows, 4 entries: 138, 192, 387, 272, 304
+//   27^3 ICT(3e-3), 312 levels of 63 rows, 12 entries: 257, 251, 450, 289, 211
 struct LaneShape {
     int waves, group, slots;
     float us;
 };
-constexpr LaneShape kShapes[] = {{1, 4, 4, 0.19f}, {1, 2, 8, 0.23f}, {1, 1, 8, 0.18f}, {4, 4, 4, 0.29f}, {4, 2, 4, 0.21f}};
+constexpr LaneShape kShapes[] = {{1, 1, 4, 0.125f}, {1, 1, 8, 0.18f}, {1, 4, 4, 0.18f},
+                                 {1, 2, 8, 0.22f},  {1, 4, 8, 0.30f}, {4, 4, 4, 0.27f}};
+
+// The fewest steps a sweep's rows [r0, r1) can take: the longest chain of
+// parts, the parts over the width.
+uint32_t fewest_steps(const HostSweep &s, uint32_t r0, uint32_t r1, uint32_t width, uint32_t entries) {
+    const uint32_t n = r1 - r0;
+    std::vector<uint32_t> level(n, 0);
+    uint64_t parts = 0;
+    uint32_t chain = 0;
+    for (uint32_t k = 0; k < n; ++k) {
+        const uint32_t i = s.lower ? k : n - 1 - k, e0 = s.rp[r0 + i], e1 = s.rp[r0 + i + 1];
+        const uint32_t m = std::max(1u, (e1 - e0 + entries - 1) / entries);
+        uint32_t a = e0, b = e1 - (m - 1) * entries, l = 0;
+        for (uint32_t q = 0; q < m; ++q, a = b, b += entries) {
+            for (uint32_t e = a; e < b; ++e) l = std::max(l, level[s.ci[e] - r0]);
+            ++l;
+        }
+        level[i] = l;
+        chain = std::max(chain, l);
+        parts += m;
+    }
+    return std::max<uint32_t>(chain, (uint32_t)((parts + width - 1) / width));
+}
 
 template <class T>
 void build_lane_sweep(const HostSweep &lo, const HostSweep &up, const ChunkSet &C, LaneSweep<T> &L) {
     L.free_all();
-    // every shape's steps; chunks share the 256 compute units
     constexpr size_t K = sizeof(kShapes) / sizeof(kShapes[0]);
-    std::vector<uint32_t> steps(K * C.nchunk);
-    parallel_for(K * C.nchunk, 1, [&](size_t q0, size_t q1) {
-        for (size_t q = q0; q < q1; ++q) {
-            const LaneShape &h = kShapes[q % K];
-            const uint32_t r0 = C.start[q / K], r1 = C.start[q / K + 1];
-            steps[q] = plan_chunk(lo, r0, r1, 64 * h.waves / h.group, h.group * h.slots).steps +
-                       plan_chunk(up, r0, r1, 64 * h.waves / h.group, h.group * h.slots).steps;
-        }
-    });
-    size_t best = 0;
-    double best_us = 0;
-    for (size_t k = 0; k < K; ++k) {
+    // chunks share the 256 compute units
+    const auto price = [&](const LaneShape &h, bool planned) {
+        std::vector<uint32_t> steps(C.nchunk, 0);
+        parallel_for(C.nchunk, 1, [&](size_t c0, size_t c1) {
+            for (size_t c = c0; c < c1; ++c)
+                for (const HostSweep *s : {&lo, &up}) {
+                    const uint32_t width = 64 * h.waves / h.group, entries = h.group * h.slots;
+                    uint32_t span = 0;
+                    if (planned) plan_steps(*s, {C.start[c], C.start[c + 1]}, width, entries, span);
+                    else span = fewest_steps(*s, C.start[c], C.start[c + 1], width, entries);
+                    steps[c] += span;
+                }
+        });
         double longest = 0, total = 0;
-        for (uint32_t c = 0; c < C.nchunk; ++c) {
-            longest = std::max(longest, (double)steps[c * K + k]);
-            total += steps[c * K + k];
+        for (uint32_t v : steps) {
+            longest = std::max(longest, (double)v);
+            total += v;
         }
-        const double us = std::max(longest, total / 256) * kShapes[k].us;
-        if (k == 0 || us < best_us) {
-            best = k;
+        return std::max(longest, total / 256) * h.us;
+    };
+    // shapes by their least price; planned until none left can be cheaper
+    std::vector<std::pair<double, size_t>> least(K);
+    for (size_t k = 0; k < K; ++k) least[k] = {price(kShapes[k], false), k};
+    std::sort(least.begin(), least.end());
+    size_t best = least[0].second;
+    double best_us = price(kShapes[best], true);
+    for (size_t q = 1; q < K && least[q].first < best_us; ++q) {
+        const double us = price(kShapes[least[q].second], true);
+        if (us < best_us) {
+            best = least[q].second;
             best_us = us;
         }
     }
@@ -992,11 +960,12 @@ void launch_lane_sweep(pp_ctx *ctx, const ChunkSet &C, const LaneSweep<T> &L, co
         PP_LANES_M(W, G, S, UNIT, MULTIPLY)         \
         PP_LANES_M(W, G, S, UNIT, PREDIVIDE)        \
     }
+    PP_LANES(1, 1, 4)
+    PP_LANES(1, 1, 8)
     PP_LANES(1, 4, 4)
     PP_LANES(1, 2, 8)
-    PP_LANES(1, 1, 8)
+    PP_LANES(1, 4, 8)
     PP_LANES(4, 4, 4)
-    PP_LANES(4, 2, 4)
 #undef PP_LANES
 #undef PP_LANES_M
     PP_HIP(hipGetLastError());
@@ -1033,7 +1002,8 @@ template struct StripSweep<float>;
 // 608, 24 758, 68 717; ICT(1e-3) 400^2 16 strips 1861, 32 1958, 64 2116;
 // ICT(1e-2) 100^3, where LDS asks for 100, 686, 128 731), unless LDS asks for
 // more.  The lanes of a row by its mean entries, eight a lane (64^3, 7
-// entries: one lane 341, two 517; 60x48x68, 12 entries: 801, 608, four 1208).
+// entries: one lane 347, two 520, four 904; 60x48x68, 12 entries: 692, 669,
+// 1419; ILUT, 12 entries: 364, 280, 487).
 template <class T>
 bool build_strip_sweeps(pp_ctx *ctx, const HostSweep &lo, const HostSweep &up, StripSweep<T> &L) {
     L.free_all();
