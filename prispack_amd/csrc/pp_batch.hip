@@ -489,6 +489,365 @@ __global__ __launch_bounds__(BS) void k_batch_pcg(BatchArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// The mixed solve of a batch in reduced form with every system's inner CG
+// spread over tiles, a workgroup each (k_tile_cg), and one launch per
+// refinement step around it (k_batch_step).
+//
+// One workgroup per system left the largest system alone on one compute unit
+// (65,536 rows: 135 us an iteration, 4.4 MB of operators and vectors streamed
+// at the 33 GB/s one unit draws, while the small systems' units idled).  A
+// tile of at most 2048 second-colour rows keeps everything in the unit: the
+// operators' values and the vectors p, s, e in registers, r and y0 = KA r in
+// LDS.  It owns its rows and computes what it reads of its neighbours' twice:
+// F = the first-colour rows its own rows touch, R = its own rows and those F
+// touches (r and s are kept for all of R).  So one exchange an iteration
+// remains: w on R's halo, and the tiles' three partial sums.  Every word
+// carries its iteration's number beside 32 bits of payload, so it is its own
+// ready flag and nothing is reset; two buffers alternate, since a tile may
+// run one iteration ahead of another's reads but not two.
+// Tiles of one system are neighbours in the launch, no more than the chip
+// holds, and workgroups start in order, so the first unfinished system has all
+// its tiles running.  Should other work keep them out all the same, a wait
+// past the deadline raises the abort word, which ends every tile, and the
+// batch is solved by k_batch_pcg instead.
+// A solve of 256 systems of 32^2 to 256^2 rows: 88 ms with one workgroup a
+// system, 8.3 ms now, 6.6 of it here.  Two workgroups of 256 threads a unit
+// hide each other's exchange: one of 512 threads, the same rows and registers
+// a thread, took 8.6 (24 systems of 60^2 to 200^2: 2.72, now 2.51).
+// ---------------------------------------------------------------------------
+constexpr int kTileThreads = 256, kStepThreads = 1024;
+// rows of F, owned rows, halo rows of a thread, by the entries of a row
+template <int W>
+struct TileShape {
+    static constexpr int kF = W <= 4 ? 10 : 8, kS = W <= 4 ? 8 : 5, kH = W <= 4 ? 3 : 5;
+};
+constexpr uint32_t kNoSlot = 0xffffffffu;
+
+struct Tile {
+    uint32_t sys, tile0, ntile;     // its system, the system's first tile and count
+    uint32_t row0, ns, nf, nh;      // first owned row; owned, F, halo rows
+    uint32_t f, h;                  // F's rows in `rows`, then the halo's; the halo's slots in `slots`
+    uint32_t ka, kb;                // local words of F's and the owned rows' entries in `loc` (W a row, by entry)
+    uint32_t out;                   // the owned rows' slots in `slots`
+};
+
+struct TileArgs {
+    const Tile *tiles;
+    const uint32_t *rows, *slots;
+    const uint16_t *loc;
+    unsigned long long *xw, *xp;    // exchanged w (two buffers of nslot), partial sums (two of 6 * ntiles)
+    uint32_t nslot, ntiles;
+    int *abort;
+    long long deadline;
+    const int32_t *active;          // per system, set by k_batch_step
+    const double *want, *rin_norm;
+    const uint32_t *left;           // iterations the system may still take
+    const uint32_t *kab_rp;
+    const float *kab_v, *red_s1, *red_dt;
+    float *z, *e;
+    int32_t *iters;
+};
+
+__device__ inline unsigned long long tagged(uint32_t tag, uint32_t v) { return (unsigned long long)tag << 32 | v; }
+__device__ inline void put_word(unsigned long long *p, unsigned long long v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline unsigned long long get_word(const unsigned long long *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// v, but nothing computed from it leaves the loop it is used in (unpacked
+// addresses kept across iterations would not fit the registers)
+__device__ inline uint32_t here(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+template <int W>
+__global__ __launch_bounds__(kTileThreads) void k_tile_cg(TileArgs a) {
+    using Sh = TileShape<W>;
+    constexpr int F = Sh::kF, S = Sh::kS, H = Sh::kH, BS = kTileThreads;
+    constexpr uint32_t kWords = BS / 6 * 6;  // partial-sum words read at a time, one a thread
+    __shared__ float zr[(S + H) * BS], zy[F * BS];
+    __shared__ double sh3[3 * (BS / 64)];
+    __shared__ uint32_t part[kWords];
+    __shared__ int stop;
+    const Tile t = a.tiles[blockIdx.x];
+    if (!a.active[t.sys]) return;
+    const uint32_t tid = threadIdx.x;
+    // operators and vectors of this thread's rows
+    float kav[F][W], kbv[S][W + 1];
+    uint32_t kai[F][W / 2], kbi[S][W / 2];
+#pragma unroll
+    for (int k = 0; k < F; ++k) {
+        const uint32_t f = tid + k * BS;
+        const bool ok = f < t.nf;
+        const uint32_t i = ok ? a.rows[t.f + f] : 0;
+        const uint32_t e0 = ok ? a.kab_rp[i] : 0, e1 = ok ? a.kab_rp[i + 1] : 0;
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            kav[k][j] = e0 + j < e1 ? a.kab_v[e0 + j] : 0.f;
+            const uint32_t w = ok ? a.loc[t.ka + j * t.nf + f] : 0;
+            kai[k][j / 2] = (j & 1) ? kai[k][j / 2] | w << 16 : w;
+        }
+    }
+    float p[S], sv[S], e[S], dt[S];
+    uint32_t to[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+        const uint32_t q = tid + k * BS;
+        const bool ok = q < t.ns;
+        const uint32_t i = t.row0 + (ok ? q : 0);
+        const uint32_t e0 = ok ? a.kab_rp[i] : 0, e1 = ok ? a.kab_rp[i + 1] : 0;
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            kbv[k][j] = e0 + j + 1 < e1 ? a.kab_v[e0 + j] : 0.f;
+            const uint32_t w = ok ? a.loc[t.kb + j * t.ns + q] : 0;
+            kbi[k][j / 2] = (j & 1) ? kbi[k][j / 2] | w << 16 : w;
+        }
+        kbv[k][W] = ok ? a.kab_v[e1 - 1] : 0.f;  // the diagonal, last
+        p[k] = sv[k] = e[k] = 0.f;
+        dt[k] = ok ? a.red_dt[i] : 0.f;
+        to[k] = ok ? a.slots[t.out + q] : kNoSlot;
+        if (ok) zr[q] = a.z[i];
+    }
+    float hs[H];
+    uint32_t from[H];
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+        const uint32_t h = tid + k * BS;
+        hs[k] = 0.f;
+        from[k] = kNoSlot;
+        if (h < t.nh) {
+            from[k] = a.slots[t.h + h];
+            zr[t.ns + h] = a.z[a.rows[t.f + t.nf + h]];
+        }
+    }
+    if (tid == 0) stop = 0;
+    const double tol = a.want[t.sys], normb = a.rin_norm[t.sys];
+    const uint32_t maxit = a.left[t.sys];
+    const bool shared = t.ntile > 1;
+    const long long t0 = shared ? wall_clock64() : 0;
+    uint32_t m = maxit;
+    double gold = 0.0, aold = 1.0;
+    bool first = true;
+    __syncthreads();
+    for (uint32_t c = 1;; ++c) {
+        // y0 = KA r on F
+#pragma unroll
+        for (int k = 0; k < F; ++k) {
+            float sum = 0.f;
+#pragma unroll
+            for (int j = 0; j < W; j += 2) {
+                const uint32_t pair = here(kai[k][j / 2]);
+                sum += kav[k][j] * zr[pair & 0xffffu];
+                sum += kav[k][j + 1] * zr[pair >> 16];
+            }
+            if (tid + k * BS < t.nf) zy[tid + k * BS] = sum;
+        }
+        __syncthreads();
+        // w = KB [y0; r] with (r, w), (r, r) and sum Dt r^2
+        const uint32_t par = c & 1;
+        unsigned long long *xw = a.xw + (size_t)par * a.nslot, *xp = a.xp + (size_t)par * 6 * a.ntiles;
+        double delta = 0.0, gamma = 0.0, rho = 0.0;
+        float w[S], r[S];
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            const bool ok = tid + k * BS < t.ns;
+            r[k] = ok ? zr[tid + k * BS] : 0.f;
+            float sum = 0.f;
+#pragma unroll
+            for (int j = 0; j < W; j += 2) {
+                const uint32_t pair = here(kbi[k][j / 2]);
+                sum += kbv[k][j] * zy[pair & 0xffffu];
+                sum += kbv[k][j + 1] * zy[pair >> 16];
+            }
+            sum += kbv[k][W] * r[k];
+            w[k] = sum;
+            if (to[k] != kNoSlot) put_word(xw + to[k], tagged(c, __float_as_uint(sum)));
+            if (ok) {
+                delta += (double)(r[k] * sum);
+                gamma += (double)(r[k] * r[k]);
+                rho += (double)dt[k] * (double)(r[k] * r[k]);
+            }
+        }
+        block_reduce3<BS>(delta, gamma, rho, sh3);
+        float hw[H] = {};
+        if (shared) {
+            // this tile's sums out, all tiles' sums and the halo's w in
+            if (tid < 6) {
+                const double v = tid < 2 ? delta : tid < 4 ? gamma : rho;
+                const uint32_t half = (tid & 1) ? (uint32_t)__double2hiint(v) : (uint32_t)__double2loint(v);
+                put_word(xp + 6 * (size_t)blockIdx.x + tid, tagged(c, half));
+            }
+            const uint32_t nw = 6 * t.ntile;
+            double td = 0.0, tg = 0.0, tr = 0.0;
+            bool wait_h[H];
+#pragma unroll
+            for (int k = 0; k < H; ++k) wait_h[k] = from[k] != kNoSlot;
+            for (uint32_t w0 = 0; w0 < nw; w0 += kWords) {
+                const uint32_t cnt = min(nw - w0, kWords);
+                bool wait_p = tid < cnt;
+                const unsigned long long *src = xp + 6 * (size_t)t.tile0 + w0 + tid;
+                for (uint32_t iter = 1;; ++iter) {
+                    bool more = false;
+                    const unsigned long long v = wait_p ? get_word(src) : 0;
+                    unsigned long long hv[H];
+#pragma unroll
+                    for (int k = 0; k < H; ++k) hv[k] = wait_h[k] ? get_word(xw + from[k]) : 0;
+                    if (wait_p && (uint32_t)(v >> 32) == c) {
+                        part[tid] = (uint32_t)v;
+                        wait_p = false;
+                    }
+                    more = wait_p;
+#pragma unroll
+                    for (int k = 0; k < H; ++k) {
+                        if (wait_h[k] && (uint32_t)(hv[k] >> 32) == c) {
+                            hw[k] = __uint_as_float((uint32_t)hv[k]);
+                            wait_h[k] = false;
+                        }
+                        more = more || wait_h[k];
+                    }
+                    if (!__any(more)) break;
+                    if ((iter & 63) == 0 &&
+                        (wall_clock64() - t0 > a.deadline ||
+                         __hip_atomic_load(a.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                        atomicOr(a.abort, 1);
+                        stop = 1;
+                        break;
+                    }
+                }
+                __syncthreads();
+                for (uint32_t q = 0; q < cnt / 6; ++q) {  // in tile order, the same in every tile
+                    td += __hiloint2double((int)part[6 * q + 1], (int)part[6 * q]);
+                    tg += __hiloint2double((int)part[6 * q + 3], (int)part[6 * q + 2]);
+                    tr += __hiloint2double((int)part[6 * q + 5], (int)part[6 * q + 4]);
+                }
+                if (w0 + kWords < nw) __syncthreads();
+            }
+            delta = td;
+            gamma = tg;
+            rho = tr;
+            if (stop) break;
+        }
+        if (c >= maxit) break;
+        const double norm = normb > 0.0 ? sqrt(rho) / normb : 0.0;
+        if (!(norm == norm) || isinf(norm)) break;
+        if (norm < tol) {
+            m = c;
+            break;
+        }
+        const double beta = first ? 0.0 : gamma / gold;
+        const double den = first ? delta : delta - beta * gamma / aold;
+        if (den == 0.0 || !(den == den)) break;
+        const double alpha = gamma / den;
+        gold = gamma;
+        aold = alpha;
+        first = false;
+        const float fa = (float)alpha, fb = (float)beta;
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            p[k] = r[k] + fb * p[k];
+            sv[k] = w[k] + fb * sv[k];
+            e[k] = e[k] + fa * p[k];
+            if (tid + k * BS < t.ns) zr[tid + k * BS] = r[k] - fa * sv[k];
+        }
+#pragma unroll
+        for (int k = 0; k < H; ++k)
+            if (tid + k * BS < t.nh) {
+                hs[k] = hw[k] + fb * hs[k];
+                zr[t.ns + tid + k * BS] -= fa * hs[k];
+            }
+        __syncthreads();
+    }
+    // e_1 = s1 x
+#pragma unroll
+    for (int k = 0; k < S; ++k)
+        if (tid + k * BS < t.ns) {
+            const uint32_t i = t.row0 + tid + k * BS;
+            const float v = a.red_s1[i] * e[k];
+            a.e[i] = v;
+            a.z[i] = v;
+        }
+    if (tid == 0 && blockIdx.x == t.tile0) a.iters[t.sys] += (int32_t)m;
+}
+
+// One refinement step of the batch, a workgroup per system: the last inner
+// solve's correction (not in the first step), the FP64 residual and its
+// test, then the next inner solve's right-hand side r = KF rin, rin = (b -
+// A x) / ||b - A x||.
+struct StepState {
+    int32_t *active;
+    double *want, *rin_norm, *rn, *normb;
+    uint32_t *left;
+    int *any;  // set when a system goes on
+};
+__global__ __launch_bounds__(kStepThreads) void k_batch_step(BatchArgs a, StepState st, int begin) {
+    constexpr int BS = kStepThreads;
+    __shared__ double sh[BS / 64];
+    const uint32_t s = blockIdx.x, r0 = a.roff[s], r1 = a.roff[s + 1], m0 = r0 + a.red_n0[s];
+    if (!begin && !st.active[s]) return;
+    double normb;
+    int outer = 0;
+    uint32_t total = 0;
+    if (begin) {
+        double bb = 0.0;
+        for (uint32_t i = r0 + threadIdx.x; i < r1; i += BS) {
+            bb += a.b[i] * a.b[i];
+            a.x[i] = 0.0;
+        }
+        normb = sqrt(block_reduce<BS>(bb, sh));
+    } else {
+        normb = st.normb[s];
+        outer = a.outer[s] + 1;
+        total = (uint32_t)a.iters[s];
+        // e = [KE [rin_0; e_1]; e_1]
+        for (uint32_t i = r0 + threadIdx.x; i < m0; i += BS) a.q32[i] = a.r32[i];
+        __syncthreads();
+        sys_spmv<float, float>(a.kfe_rp, a.kfe_ci, a.kfe_v, a.q32, a.e32, r0, m0);
+        __syncthreads();
+        const double rn = st.rn[s];
+        for (uint32_t i = r0 + threadIdx.x; i < r1; i += BS) a.x[i] += rn * (double)a.e32[i];
+    }
+    __syncthreads();
+    sys_spmv<double, double>(a.rp, a.ci, a.v64, a.x, a.r64, r0, r1);
+    __syncthreads();
+    double rr = 0.0;
+    for (uint32_t i = r0 + threadIdx.x; i < r1; i += BS) {
+        const double t = a.b[i] - a.r64[i];
+        a.r64[i] = t;
+        rr += t * t;
+    }
+    const double rn = sqrt(block_reduce<BS>(rr, sh));
+    const double rel = normb > 0 ? rn / normb : 0.0;
+    const bool done = rel < a.tol || !(rel == rel) || (uint32_t)outer >= a.max_outer || total >= a.maxit;
+    if (threadIdx.x == 0) {
+        a.iters[s] = (int32_t)total;
+        a.outer[s] = outer;
+        a.conv[s] = rel < a.tol;
+        a.relres[s] = rel;
+        st.active[s] = !done;
+        st.normb[s] = normb;
+        st.rn[s] = rn;
+        st.want[s] = fmax(a.inner_tol, 0.5 * a.tol * normb / rn);
+        st.left[s] = a.maxit - total;
+        if (!done) *st.any = 1;
+    }
+    if (done) return;
+    const float sc = (float)(1.0 / rn);
+    double bb = 0.0;
+    for (uint32_t i = r0 + threadIdx.x; i < r1; i += BS) {
+        const float v = (float)a.r64[i] * sc;
+        a.r32[i] = v;
+        bb += (double)v * (double)v;
+    }
+    const double nin = sqrt(block_reduce<BS>(bb, sh));
+    if (threadIdx.x == 0) st.rin_norm[s] = nin;
+    __syncthreads();
+    sys_spmv<float, float>(a.kfe_rp, a.kfe_ci, a.kfe_v, a.r32, a.q32, m0, r1);
+}
+
 }  // namespace
 }  // namespace pp
 
@@ -530,6 +889,17 @@ struct pp_batch {
     uint32_t lo_nnz = 0;
     int *flag = nullptr;
     bool h_v_stale = false;  // h_v predates the values in v64
+    // the reduced form's tiles (batch_build_tiles); tile_width 0: none
+    int tile_width = 0;
+    uint32_t ntiles = 0, nslot = 0;
+    pp::Tile *tiles = nullptr;
+    uint32_t *tile_rows = nullptr, *tile_slots = nullptr;
+    uint16_t *tile_loc = nullptr;
+    unsigned long long *tile_w = nullptr, *tile_sums = nullptr;  // exchanged w, partial sums
+    int32_t *active = nullptr;
+    double *state = nullptr;   // want, rin_norm, rn, normb: nsys each
+    uint32_t *left = nullptr;
+    int *tile_flag = nullptr;  // any, abort
 };
 
 namespace pp {
@@ -918,6 +1288,183 @@ void batch_free_refresh(pp_batch *B) {
     B->refresh = 0;
 }
 
+void batch_free_tiles(pp_batch *B) {
+    dfree(B->tiles); dfree(B->tile_rows); dfree(B->tile_slots); dfree(B->tile_loc); dfree(B->tile_w);
+    dfree(B->tile_sums); dfree(B->active); dfree(B->state); dfree(B->left); dfree(B->tile_flag);
+    B->tiles = nullptr;
+    B->tile_rows = B->tile_slots = B->left = nullptr;
+    B->tile_loc = nullptr;
+    B->tile_w = B->tile_sums = nullptr;
+    B->active = nullptr;
+    B->state = nullptr;
+    B->tile_flag = nullptr;
+    B->tile_width = 0;
+    B->ntiles = B->nslot = 0;
+}
+
+// The tiles of one system: its second-colour rows cut into ntile ranges.
+struct SystemTiles {
+    std::vector<Tile> tiles;               // f, h, ka, kb, out relative to the vectors below
+    std::vector<uint32_t> rows, hrow, out; // F's rows and the halo's; halo rows by entry of `slots`; owned rows' exports
+    std::vector<uint32_t> slots;           // halo: the row, to be replaced by its slot; owned: kNoSlot or the slot
+    std::vector<uint16_t> loc;
+    uint32_t nslot = 0;
+    bool fits = false;
+};
+
+SystemTiles tiles_of_system(const ReducedHost &H, uint32_t r0, int W, uint32_t ntile, uint32_t maxf, uint32_t maxs,
+                            uint32_t maxh) {
+    SystemTiles T;
+    const uint32_t n0 = H.n0, n1 = H.n1;
+    std::vector<uint32_t> fpos(n0, kNoSlot), rpos(n1, kNoSlot), slot(n1, kNoSlot);
+    // rows exported: those some other tile reads (numbered after the tiles are known)
+    std::vector<uint8_t> exported(n1, 0);
+    for (uint32_t k = 0; k < ntile; ++k) {
+        const uint32_t q0 = (uint32_t)((uint64_t)n1 * k / ntile), q1 = (uint32_t)((uint64_t)n1 * (k + 1) / ntile);
+        Tile t{};
+        t.row0 = r0 + n0 + q0;
+        t.ns = q1 - q0;
+        t.f = (uint32_t)T.rows.size();
+        std::vector<uint32_t> F, R;
+        for (uint32_t q = q0; q < q1; ++q)
+            for (uint32_t e = H.kb_rp[q]; e + 1 < H.kb_rp[q + 1]; ++e)
+                if (fpos[H.kb_ci[e]] == kNoSlot) {
+                    fpos[H.kb_ci[e]] = 0;
+                    F.push_back(H.kb_ci[e]);
+                }
+        std::sort(F.begin(), F.end());
+        for (uint32_t f = 0; f < F.size(); ++f) fpos[F[f]] = f;
+        for (uint32_t q = q0; q < q1; ++q) rpos[q] = q - q0;
+        for (uint32_t i : F)
+            for (uint32_t e = H.ka_rp[i]; e < H.ka_rp[i + 1]; ++e) {
+                const uint32_t q = H.ka_ci[e] - n0;
+                if (rpos[q] == kNoSlot) {
+                    rpos[q] = t.ns + (uint32_t)R.size();
+                    R.push_back(q);
+                    exported[q] = 1;
+                }
+            }
+        t.nf = (uint32_t)F.size();
+        t.nh = (uint32_t)R.size();
+        if (t.nf > maxf || t.ns > maxs || t.nh > maxh) return T;
+        t.ka = (uint32_t)T.loc.size();
+        T.loc.resize(T.loc.size() + (size_t)W * t.nf, 0);
+        for (uint32_t f = 0; f < t.nf; ++f)
+            for (uint32_t e = H.ka_rp[F[f]], j = 0; e < H.ka_rp[F[f] + 1]; ++e, ++j)
+                T.loc[t.ka + (size_t)j * t.nf + f] = (uint16_t)rpos[H.ka_ci[e] - n0];
+        t.kb = (uint32_t)T.loc.size();
+        T.loc.resize(T.loc.size() + (size_t)W * t.ns, 0);
+        for (uint32_t q = q0; q < q1; ++q)
+            for (uint32_t e = H.kb_rp[q], j = 0; e + 1 < H.kb_rp[q + 1]; ++e, ++j)
+                T.loc[t.kb + (size_t)j * t.ns + (q - q0)] = (uint16_t)fpos[H.kb_ci[e]];
+        for (uint32_t i : F) T.rows.push_back(r0 + i);
+        for (uint32_t q : R) T.rows.push_back(r0 + n0 + q);
+        t.h = (uint32_t)T.slots.size();
+        for (uint32_t q : R) T.slots.push_back(q);
+        t.out = (uint32_t)T.slots.size();
+        for (uint32_t q = q0; q < q1; ++q) T.slots.push_back(q);
+        for (uint32_t i : F) fpos[i] = kNoSlot;
+        for (uint32_t q : R) rpos[q] = kNoSlot;
+        for (uint32_t q = q0; q < q1; ++q) rpos[q] = kNoSlot;
+        T.tiles.push_back(t);
+    }
+    for (uint32_t q = 0; q < n1; ++q)
+        if (exported[q]) slot[q] = T.nslot++;
+    for (uint32_t &v : T.slots) v = slot[v];
+    T.fits = true;
+    return T;
+}
+
+// The tiles of every system (largest first), when all their rows are short
+// enough: rows of at most 4 or 6 off-diagonal entries (5- and 7-point
+// stencils).  Two tiles of kS * kTileThreads rows fill a unit's registers;
+// batches that would leave units idle take tiles down to 1024 rows (smaller
+// ones wait on one another more than they compute: 24 systems of 60^2 to
+// 200^2 2.9 ms with 512 rows, 2.5 with 1024).  false (nothing kept): a system
+// does not fit.
+bool batch_build_tiles(pp_batch *B, const std::vector<ReducedHost> &reds) {
+    batch_free_tiles(B);
+    const uint32_t ns = B->nsys;
+    uint32_t width = 1;
+    for (const ReducedHost &H : reds) {
+        for (uint32_t i = 0; i < H.n0; ++i) width = std::max(width, H.ka_rp[i + 1] - H.ka_rp[i]);
+        for (uint32_t q = 0; q < H.n1; ++q) width = std::max(width, H.kb_rp[q + 1] - H.kb_rp[q] - 1);
+    }
+    if (width > 6) return false;
+    const int W = width <= 4 ? 4 : 6;
+    const uint32_t maxf = kTileThreads * (W == 4 ? TileShape<4>::kF : TileShape<6>::kF);
+    const uint32_t maxs = kTileThreads * (W == 4 ? TileShape<4>::kS : TileShape<6>::kS);
+    const uint32_t maxh = kTileThreads * (W == 4 ? TileShape<4>::kH : TileShape<6>::kH);
+    const auto count = [&](uint32_t cap) {
+        uint64_t c = 0;
+        for (const ReducedHost &H : reds) c += std::max(1u, (H.n1 + cap - 1) / cap);
+        return c;
+    };
+    // a system's tiles wait for one another, so all of them must run at a time
+    const uint32_t max_tiles = (uint32_t)B->ctx->cu_count;
+    uint32_t cap = maxs;
+    while (cap > 1024 && count(cap / 2) <= (uint64_t)B->ctx->cu_count) cap /= 2;
+    std::vector<SystemTiles> T(ns);
+    std::atomic<bool> fits{true};
+    parallel_for(ns, 1, [&](size_t s0, size_t s1) {
+        for (size_t s = s0; s < s1 && fits; ++s) {
+            uint32_t nt = std::max(1u, (reds[s].n1 + cap - 1) / cap);
+            for (;; nt += std::max(1u, nt / 4)) {  // more tiles until F and the halo fit
+                T[s] = tiles_of_system(reds[s], B->h_roff[s], W, nt, maxf, maxs, maxh);
+                if (T[s].fits) break;
+                if (nt > max_tiles || nt > reds[s].n1) break;
+            }
+            if (!T[s].fits || nt > max_tiles) fits = false;
+        }
+    });
+    if (!fits) return false;
+    std::vector<uint32_t> order(ns);
+    for (uint32_t s = 0; s < ns; ++s) order[s] = s;
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return reds[x].n1 > reds[y].n1; });
+    std::vector<Tile> tiles;
+    std::vector<uint32_t> rows, slots;
+    std::vector<uint16_t> loc;
+    uint32_t nslot = 0;
+    for (uint32_t s : order) {
+        SystemTiles &q = T[s];
+        const uint32_t tile0 = (uint32_t)tiles.size();
+        for (Tile t : q.tiles) {
+            t.sys = s;
+            t.tile0 = tile0;
+            t.ntile = (uint32_t)q.tiles.size();
+            t.f += (uint32_t)rows.size();
+            t.h += (uint32_t)slots.size();
+            t.out += (uint32_t)slots.size();
+            t.ka += (uint32_t)loc.size();
+            t.kb += (uint32_t)loc.size();
+            tiles.push_back(t);
+        }
+        rows.insert(rows.end(), q.rows.begin(), q.rows.end());
+        for (uint32_t v : q.slots) slots.push_back(v == kNoSlot ? kNoSlot : v + nslot);
+        loc.insert(loc.end(), q.loc.begin(), q.loc.end());
+        nslot += q.nslot;
+    }
+    auto up = [](const void *src, size_t bytes) {
+        unsigned char *d = dalloc<unsigned char>(std::max<size_t>(16, bytes));
+        if (bytes) PP_HIP(hipMemcpy(d, src, bytes, hipMemcpyHostToDevice));
+        return d;
+    };
+    B->tiles = (Tile *)up(tiles.data(), tiles.size() * sizeof(Tile));
+    B->tile_rows = upload(rows);
+    B->tile_slots = upload(slots);
+    B->tile_loc = (uint16_t *)up(loc.data(), loc.size() * 2);
+    B->ntiles = (uint32_t)tiles.size();
+    B->nslot = nslot;
+    B->tile_w = dalloc<unsigned long long>(2 * (size_t)std::max(1u, nslot));
+    B->tile_sums = dalloc<unsigned long long>(12 * (size_t)B->ntiles);
+    B->active = dalloc<int>(ns);
+    B->state = dalloc<double>(4 * (size_t)ns);
+    B->left = dalloc<uint32_t>(ns);
+    B->tile_flag = dalloc<int>(2);
+    B->tile_width = W;
+    return true;
+}
+
 // IC(0) of every diagonal block (of the permuted copy under multicolour
 // ordering), as two gather-form sweeps.
 void batch_factor(pp_batch *B) {
@@ -971,7 +1518,11 @@ void batch_factor(pp_batch *B) {
     B->lo_nnz = (uint32_t)lo.ci.size();
     batch_free_refresh(B);  // its maps belong to the sweeps just replaced
     batch_free_reduced(B);
-    if (red_ok) batch_upload_reduced(B, reds);
+    batch_free_tiles(B);
+    if (red_ok) {
+        batch_upload_reduced(B, reds);
+        batch_build_tiles(B, reds);
+    }
 }
 
 void batch_ensure_host_values(pp_batch *B) {
@@ -1121,7 +1672,59 @@ void run_batch(pp_ctx *ctx, pp_batch *B, bool mixed, const BatchArgs &a) {
     PP_HIP(hipStreamSynchronize(ctx->stream));
 }
 
+// The mixed solve over tiles: refinement steps until no system goes on;
+// false: a tile gave up waiting.
+bool run_tiles(pp_ctx *ctx, pp_batch *B, const BatchArgs &a) {
+    const uint32_t ns = B->nsys;
+    StepState st;
+    st.active = B->active;
+    st.want = B->state;
+    st.rin_norm = B->state + ns;
+    st.rn = B->state + 2 * (size_t)ns;
+    st.normb = B->state + 3 * (size_t)ns;
+    st.left = B->left;
+    st.any = B->tile_flag;
+    TileArgs t;
+    t.tiles = B->tiles;
+    t.rows = B->tile_rows;
+    t.slots = B->tile_slots;
+    t.loc = B->tile_loc;
+    t.xw = B->tile_w;
+    t.xp = B->tile_sums;
+    t.nslot = B->nslot;
+    t.ntiles = B->ntiles;
+    t.abort = B->tile_flag + 1;
+    t.deadline = ctx->spin_deadline;
+    t.active = B->active;
+    t.want = st.want;
+    t.rin_norm = st.rin_norm;
+    t.left = B->left;
+    t.kab_rp = B->kab_rp;
+    t.kab_v = B->kab_v;
+    t.red_s1 = B->red_s1;
+    t.red_dt = B->red_dt;
+    t.z = B->q32;
+    t.e = B->e32;
+    t.iters = B->iters;
+    for (int begin = 1;; begin = 0) {
+        launch_fill_zero(ctx, B->tile_flag, (begin ? 2 : 1) * sizeof(int));  // the abort word stays
+        k_batch_step<<<ns, kStepThreads, 0, ctx->stream>>>(a, st, begin);
+        PP_HIP(hipGetLastError());
+        int flag[2];
+        PP_HIP(hipMemcpyAsync(flag, B->tile_flag, sizeof(flag), hipMemcpyDeviceToHost, ctx->stream));
+        PP_HIP(hipStreamSynchronize(ctx->stream));
+        if (flag[1]) return false;
+        if (!flag[0]) return true;
+        launch_fill_zero(ctx, B->tile_w, 2 * (size_t)std::max(1u, B->nslot) * 8);
+        launch_fill_zero(ctx, B->tile_sums, 12 * (size_t)B->ntiles * 8);
+        if (B->tile_width == 4) k_tile_cg<4><<<B->ntiles, kTileThreads, 0, ctx->stream>>>(t);
+        else k_tile_cg<6><<<B->ntiles, kTileThreads, 0, ctx->stream>>>(t);
+        PP_HIP(hipGetLastError());
+    }
+}
+
 void batch_free(pp_batch *B) {
+    batch_free_tiles(B);
     dfree(B->roff); dfree(B->rp); dfree(B->ci); dfree(B->v64); dfree(B->v32);
     B->lo.free_all();
     B->up.free_all();
@@ -1247,7 +1850,7 @@ static int batch_solve_impl(pp_ctx *ctx, pp_batch *B, const pp_solve_opts *opts,
         BatchArgs a = make_args(B, *opts, perm ? B->bp : b, perm ? B->xp : x);
         PP_HIP(hipEventRecord(ctx->ev0, ctx->stream));
         if (perm) launch_permute(ctx, B->ntot, B->gperm, PP_F64, b, B->bp, true);
-        run_batch(ctx, B, mixed, a);
+        if (!(mixed && a.red_n0 && B->tile_width && run_tiles(ctx, B, a))) run_batch(ctx, B, mixed, a);
         if (perm) {
             launch_permute(ctx, B->ntot, B->gperm, PP_F64, B->xp, x, false);
             PP_HIP(hipStreamSynchronize(ctx->stream));
