@@ -277,6 +277,22 @@ class CSRMatrix:
     def getNNZnum(self):
         return int(self.rp[-1])
 
+    @property
+    def v(self):
+        """The values on the host; those set from a tensor are fetched when read."""
+        if self._v is None:
+            L, p = _capi.lib(), C.c_void_p()
+            v = np.empty(self.getNNZnum())
+            self.ctx.check(L.pp_csr_device_ptrs(self.h, None, None, C.byref(p), None))
+            if len(v):
+                self.ctx.check(L.pp_memcpy_d2h(self.ctx.h, v.ctypes.data_as(C.c_void_p), p, v.nbytes))
+            self._v = v
+        return self._v
+
+    @v.setter
+    def v(self, values):
+        self._v = values
+
     def host(self):
         return self.rp, self.ci, self.v
 
@@ -291,7 +307,7 @@ class CSRMatrix:
             _before(self.ctx)
             p, _ = _dev_ptr(values, PP_F64)
             self.ctx.check(L.pp_csr_set_values(self.ctx.h, self.h, p, 1))
-            self.v = values.detach().cpu().numpy().copy()
+            self._v = None
         self.values_version = getattr(self, "values_version", 0) + 1
 
     def MatPVec(self, x, y, alpha=1.0, beta=0.0):

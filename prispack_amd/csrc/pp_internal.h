@@ -9,6 +9,7 @@
 #include <string>
 #include <functional>
 #include <map>
+#include <mutex>
 #include <vector>
 
 #include "../../include/prispack_amd.h"
@@ -386,6 +387,10 @@ struct pp_csr {
     pp_csr *trans = nullptr;         // explicit transpose, built on demand
     std::vector<uint32_t> h_rp, h_ci;
     std::vector<double> h_v;
+    // v64 has newer values than h_v (they came from the device); every reader
+    // of h_v calls csr_host_values first, under this lock
+    bool h_v_stale = false;
+    std::mutex h_v_lock;
     bool f32_dirty = true;
     uint64_t version = 0;            // bumped by every value update
     uint64_t uid = 0;                // unique per object (never reused)
@@ -712,6 +717,7 @@ void csr_tune(pp_ctx *ctx, pp_csr *A);
 // The host copies of A's columns and values, downloaded when A was built on
 // the device without them.
 void csr_ensure_host(pp_csr *A);
+void csr_host_values(pp_csr *A);  // h_v up to date with v64
 // The 16-bit two-base column offsets of nblk row blocks (device arrays:
 // block bounds, row pointers, columns) computed on the device, as
 // two_base_blocks does on the host: the entries in those blocks, off16

@@ -770,6 +770,7 @@ void ml_setup(pp_ctx *ctx, pp_precond *M) {
     A.n = M->A->nrow;
     A.rp = M->A->h_rp;
     A.ci = M->A->h_ci;
+    csr_host_values(M->A);
     A.v = M->A->h_v;
     auto *S = new MlState;
     M->multilevel = S;

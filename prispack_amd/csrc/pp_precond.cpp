@@ -631,6 +631,7 @@ static void ensure_host_setup(pp_precond *M) {
     if (!M->host_pending) return;
     float saved[4];
     std::copy(M->phase_ms, M->phase_ms + 4, saved);
+    csr_host_values(M->A);
     HostCsr A;
     A.n = M->A->nrow;
     A.rp.swap(M->A->h_rp);
@@ -877,9 +878,7 @@ static void devref_run(pp_ctx *ctx, pp_precond *M) {
         pp_csr *P = M->Aperm;
         launch_gather_map(ctx, R.aperm_nnz, R.aperm_map, M->A->v64, PP_F64, P->v64);
         if (P->ell.ok) ell_fill_values(ctx, P->ell, PP_F64, P->rp, P->v64);
-        if (P->h_v.size() == R.aperm_nnz)  // a matrix built on the device keeps no host values
-            PP_HIP(hipMemcpyAsync(P->h_v.data(), P->v64, (size_t)R.aperm_nnz * sizeof(double),
-                                  hipMemcpyDeviceToHost, ctx->stream));
+        if (P->h_v.size() == R.aperm_nnz) P->h_v_stale = true;  // a matrix built on the device keeps no host values
         P->f32_dirty = true;
         ++P->version;
         if (P->trans) {
@@ -995,6 +994,7 @@ pp_csr *precond_permuted_matrix(pp_ctx *ctx, pp_precond *M, pp_csr *A) {
     if (M->Aperm && M->Aperm_src_uid == A->uid && M->Aperm_version == A->version) return M->Aperm;
     csr_free(M->Aperm);
     M->Aperm = nullptr;
+    csr_host_values(A);
     HostCsr H;
     H.n = A->nrow;
     H.rp = A->h_rp;
@@ -1302,6 +1302,7 @@ int pp_precond_setup(pp_ctx *ctx, pp_precond *M) {
             M->host_pending = false;
             M->dev_setup = false;
             // the matrix's host arrays are lent to the factorization, not copied
+            csr_host_values(M->A);
             HostCsr A, Ap;
             A.n = M->A->nrow;
             struct Lend {
