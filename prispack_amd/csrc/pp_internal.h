@@ -636,9 +636,9 @@ template <class T>
 void upload_sweep(const HostSweep &s, DevSweep<T> &d);
 
 // ---- kernels (pp_kernels.hip) ----
-// y = alpha A x + beta y; dot_slot >= 0: also (dot_with, y) into that slot;
-// aux != NULL (with dot_slot): also (aux, dot_with) and (aux, aux) into the
-// next two slots, left as partials for the caller's finish kernel; wgt !=
+// y = alpha A x + beta y; dot_slot >= 0: also (dot_with, y), left in that slot
+// as spmv_grid(A) partials for the kernel that uses the sum; aux != NULL (with
+// dot_slot): also (aux, dot_with) and (aux, aux) in the next two slots; wgt !=
 // NULL weights the last: sum wgt_i aux_i^2
 void launch_spmv(pp_ctx *ctx, const pp_csr *A, int dtype, double alpha, const void *x,
                  double beta, void *y, int dot_slot, const void *dot_with, bool dot_first,
@@ -771,11 +771,14 @@ void launch_level0(pp_ctx *ctx, uint32_t lo, uint32_t hi, int mode, const T *dia
 template <class T>
 void launch_sweep_syncfree(pp_ctx *ctx, const DevSweep<T> &s, int mode, const T *b, T *y);
 
-// PCG device steps (templated on the working precision)
+// PCG device steps (templated on the working precision); np_dv: how many
+// partials of (d, A d) the SpMV left; [lvl0_lo, lvl0_hi): rows of w that the
+// update also produces, the next apply's first forward level
 template <class T>
 void pcg_d_update(pp_ctx *ctx, uint32_t n, bool first, const T *w, T *d, const T *r);
 template <class T>
-void pcg_xr_update(pp_ctx *ctx, uint32_t n, T *x, T *r, const T *d, const T *v, int hist_on, bool publish);
+void pcg_xr_update(pp_ctx *ctx, uint32_t n, unsigned np_dv, T *x, T *r, const T *d, const T *v, int hist_on,
+                   bool publish, T *w, uint32_t lvl0_lo, uint32_t lvl0_hi, int mode0, const T *diag0);
 template <class T>
 void pcg_wv(pp_ctx *ctx, uint32_t n, const T *w, const T *v);
 // single-reduction PCG: finish of the three SpMV reductions (+ check), update

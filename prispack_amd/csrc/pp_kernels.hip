@@ -14,8 +14,8 @@ namespace pp {
 // ---------------------------------------------------------------------------
 // Deterministic reductions.  A workgroup reduces with a fixed butterfly inside
 // each wavefront and a fixed left-to-right pass over the wavefronts; a
-// one-workgroup k_finish launch then sums the per-workgroup partials in index
-// order.  The result depends only on the grid shape, never on scheduling.
+// one-workgroup k_finish launch, or every workgroup of the kernel that uses
+// the sum, then sums the per-workgroup partials in index order.  The result depends only on the grid shape, never on scheduling.
 // ---------------------------------------------------------------------------
 __device__ inline double wave_sum(double v) {
 #pragma unroll
@@ -95,8 +95,8 @@ __device__ inline V ld_stream(const V *p) {
     else return *p;
 }
 
-// Publishes this workgroup's partial sum (plain store).  A separate
-// one-workgroup k_finish launch adds the partials in index order: the kernel
+// Publishes this workgroup's partial sum (plain store).  A later launch (a
+// one-workgroup k_finish, or the user of the sum) adds them: the kernel
 // boundary makes them visible, so no workgroup pays a device-wide fence or a
 // contended atomic (on a multi-XCD part an agent-scope fence writes back and
 // invalidates the L2, which costs more than the whole streaming kernel).
@@ -764,7 +764,6 @@ void launch_spmv(pp_ctx *ctx, const pp_csr *A, int dtype, double alpha, const vo
     const int var = dtype == PP_F64 ? A->spmv_variant : A->spmv_variant32;
     if (var == kVarEll) {  // with sums: as many workgroups (partials) as the CSR-stream launch
         launch_ell(ctx, A->ell, dtype, alpha, x, beta, y, dot_slot, dot_with, aux, wgt, dot ? grid : 0);
-        if (dot && !aux) launch_finish(ctx, dot_slot, grid, ctx->stop_word);  // with aux the caller finishes
         PP_HIP(hipGetLastError());
         return;
     }
@@ -792,7 +791,6 @@ void launch_spmv(pp_ctx *ctx, const pp_csr *A, int dtype, double alpha, const vo
     }
 #undef PP_SPMV_VAR
 #undef PP_SPMV
-    if (dot && !aux) launch_finish(ctx, dot_slot, grid, ctx->stop_word);  // with aux the caller finishes
     PP_HIP(hipGetLastError());
 }
 
@@ -1310,37 +1308,75 @@ template void launch_sweep_syncfree<float>(pp_ctx *, const DevSweep<float> &, in
 //   x += alpha d, r -= alpha v with alpha = (d, r) / (d, v)       [fused (r, r) + check]
 // Every kernel returns at once when the stop word is set, so iterations
 // launched past convergence cost only their launch.
+//
+// The updates are bound by the vectors they stream; what they need of the
+// sums before them every workgroup adds up itself from the partials, while
+// its first elements are on their way.  A separate one-workgroup launch per
+// sum cost 4.4 us each, 13 of the 139 us of an iteration on 128^3 rows (123
+// now, with the forward sweep's first level taken along by k_pcg_xr).
+// Workgroups of kFinishThreads, two per CU, keep that cheap: at most four
+// loads a thread for an SpMV's partials, one for the updates' own (a grid
+// of 2048 workgroups of 256 would read 67 MB of partials per sum).
 // ---------------------------------------------------------------------------
+static unsigned pcg_grid(const pp_ctx *ctx, uint32_t n) {
+    const unsigned need = (n + kFinishThreads - 1) / kFinishThreads;
+    return std::max(1u, std::min(need, 2u * (unsigned)ctx->cu_count));
+}
+
 template <class T>
-__global__ __launch_bounds__(256) void k_pcg_d(uint32_t n, int first, const T *__restrict__ w,
-                                               T *__restrict__ d, const T *__restrict__ r,
-                                               const double *scal, const int *ctl, double *partials) {
+__global__ __launch_bounds__(1024) void k_pcg_d(uint32_t n, int first, const T *__restrict__ w,
+                                                T *__restrict__ d, const T *__restrict__ r,
+                                                const double *scal, const int *ctl,
+                                                const double *__restrict__ wv_partials, unsigned np_wv,
+                                                double *partials) {
 #pragma clang fp contract(off)
-    __shared__ double sh[4];
+    __shared__ double sh[kFinishThreads / 64];
+    __shared__ double wv;
     if (ctl[C_STOP]) return;
-    const T beta = first ? (T)0 : (T)(scal[S_WV] / scal[S_DV]);
+    const uint32_t step = gridDim.x * kFinishThreads;
+    uint32_t i = blockIdx.x * kFinishThreads + threadIdx.x;
+    T wi = 0, di = 0, ri = 0;
+    if (i < n) {
+        wi = w[i];
+        if (!first) di = d[i];
+        ri = r[i];
+    }
+    T beta = 0;
+    if (!first) {
+        const double s = block_sum(sum_partials(wv_partials, np_wv), sh);
+        if (threadIdx.x == 0) wv = s;
+        __syncthreads();
+        beta = (T)(wv / scal[S_DV]);
+    }
     T acc = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    while (i < n) {
         T dn;
-        if (first) dn = w[i];
+        if (first) dn = wi;
         else {
-            T t1 = w[i];
-            T t2 = (-beta) * d[i];
+            T t1 = wi;
+            T t2 = (-beta) * di;
             dn = t1 + t2;
         }
         d[i] = dn;
-        acc += dn * r[i];
+        acc += dn * ri;
+        i += step;
+        if (i < n) {
+            wi = w[i];
+            if (!first) di = d[i];
+            ri = r[i];
+        }
     }
     publish_partial(block_sum((double)acc, sh), partials);
 }
 
 template <class T>
-__global__ __launch_bounds__(256) void k_pcg_wv(uint32_t n, const T *__restrict__ w, const T *__restrict__ v,
-                                                const int *ctl, double *partials) {
-    __shared__ double sh[4];
+__global__ __launch_bounds__(1024) void k_pcg_wv(uint32_t n, const T *__restrict__ w, const T *__restrict__ v,
+                                                 const int *ctl, double *partials) {
+    __shared__ double sh[kFinishThreads / 64];
     if (ctl[C_STOP]) return;
     T acc = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) acc += w[i] * v[i];
+    for (uint32_t i = blockIdx.x * kFinishThreads + threadIdx.x; i < n; i += gridDim.x * kFinishThreads)
+        acc += w[i] * v[i];
     publish_partial(block_sum((double)acc, sh), partials);
 }
 
@@ -1384,14 +1420,38 @@ __device__ void pcg_check(double rr, const double *scal, int *ctl, double *hist,
     ctl[C_CHECK] = c + 1;
 }
 
+// [l0, l1): the rows of the next apply's first forward level, which depend
+// on nothing but r: w there is written here too (an empty range: none).  The
+// kernel of its own that it replaces reads r again: 10.3 us on 128^3 rows.
 template <class T>
-__global__ __launch_bounds__(256) void k_pcg_xr(uint32_t n, T *__restrict__ x, T *__restrict__ r,
-                                                const T *__restrict__ d, const T *__restrict__ v,
-                                                const double *scal, int *ctl, double *partials) {
+__global__ __launch_bounds__(1024) void k_pcg_xr(uint32_t n, T *__restrict__ x, T *__restrict__ r,
+                                                 const T *__restrict__ d, const T *__restrict__ v, double *scal,
+                                                 int *ctl, const double *__restrict__ dv_partials, unsigned np_dv,
+                                                 const double *__restrict__ dr_partials, unsigned np_dr,
+                                                 double *partials, T *__restrict__ w, uint32_t l0, uint32_t l1,
+                                                 int mode0, const T *__restrict__ diag0) {
 #pragma clang fp contract(off)
-    __shared__ double sh[4];
+    __shared__ double sh[kFinishThreads / 64];
+    __shared__ double sums[2];
     if (ctl[C_STOP]) return;
-    const double den = scal[S_DV];
+    const uint32_t step = gridDim.x * kFinishThreads;
+    uint32_t i = blockIdx.x * kFinishThreads + threadIdx.x;
+    T di = 0, vi = 0, xi = 0, ri = 0;
+    if (i < n) {
+        di = d[i];
+        vi = v[i];
+        xi = x[i];
+        ri = r[i];
+    }
+    const double t_dv = sum_partials(dv_partials, np_dv), t_dr = sum_partials(dr_partials, np_dr);
+    const double s_dv = block_sum(t_dv, sh), s_dr = block_sum(t_dr, sh);
+    if (threadIdx.x == 0) {
+        sums[0] = s_dv;
+        sums[1] = s_dr;
+        if (blockIdx.x == 0) scal[S_DV] = s_dv;  // the next beta's denominator
+    }
+    __syncthreads();
+    const double den = sums[0];
     if (den == 0.0 || !(den == den)) {  // (d, A d) = 0: breakdown; NaN: non-finite data
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             ctl[C_STATUS] = den == 0.0 ? PP_ERR_BREAKDOWN : PP_ERR_NOT_FINITE;
@@ -1400,42 +1460,58 @@ __global__ __launch_bounds__(256) void k_pcg_xr(uint32_t n, T *__restrict__ x, T
         }
         return;
     }
-    const T alpha = (T)(scal[S_DR] / den);
+    const T alpha = (T)(sums[1] / den);
     T acc = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        T t1 = alpha * d[i];
-        T xn = x[i] + t1;
+    while (i < n) {
+        T t1 = alpha * di;
+        T xn = xi + t1;
         x[i] = xn;
-        T t2 = (-alpha) * v[i];
-        T rn = r[i] + t2;
+        T t2 = (-alpha) * vi;
+        T rn = ri + t2;
         r[i] = rn;
         acc += rn * rn;
+        if (i >= l0 && i < l1) {
+            T q = rn;
+            if (mode0 == 0 || mode0 == 3) q = q / diag0[i];
+            else if (mode0 == 2) q = q * diag0[i];
+            w[i] = q;
+        }
+        i += step;
+        if (i < n) {
+            di = d[i];
+            vi = v[i];
+            xi = x[i];
+            ri = r[i];
+        }
     }
     publish_partial(block_sum((double)acc, sh), partials);
 }
 
 template <class T>
 void pcg_d_update(pp_ctx *ctx, uint32_t n, bool first, const T *w, T *d, const T *r) {
-    unsigned g = grid_for(ctx, n, 4);
-    k_pcg_d<T><<<g, kBlock, 0, ctx->stream>>>(n, first ? 1 : 0, w, d, r, ctx->scal, ctx->ctl,
-                                              ctx->red.partials + (size_t)S_DR * kMaxPartials);
-    launch_finish(ctx, S_DR, g, ctx->ctl + C_STOP);
+    const unsigned g = pcg_grid(ctx, n);
+    k_pcg_d<T><<<g, kFinishThreads, 0, ctx->stream>>>(n, first ? 1 : 0, w, d, r, ctx->scal, ctx->ctl,
+                                                      ctx->red.partials + (size_t)S_WV * kMaxPartials, g,
+                                                      ctx->red.partials + (size_t)S_DR * kMaxPartials);
     PP_HIP(hipGetLastError());
 }
 
 template <class T>
 void pcg_wv(pp_ctx *ctx, uint32_t n, const T *w, const T *v) {
-    unsigned g = grid_for(ctx, n, 4);
-    k_pcg_wv<T><<<g, kBlock, 0, ctx->stream>>>(n, w, v, ctx->ctl, ctx->red.partials + (size_t)S_WV * kMaxPartials);
-    launch_finish(ctx, S_WV, g, ctx->ctl + C_STOP);
+    k_pcg_wv<T><<<pcg_grid(ctx, n), kFinishThreads, 0, ctx->stream>>>(
+        n, w, v, ctx->ctl, ctx->red.partials + (size_t)S_WV * kMaxPartials);
     PP_HIP(hipGetLastError());
 }
 
 template <class T>
-void pcg_xr_update(pp_ctx *ctx, uint32_t n, T *x, T *r, const T *d, const T *v, int hist_on, bool publish) {
-    unsigned g = grid_for(ctx, n, 4);
-    k_pcg_xr<T><<<g, kBlock, 0, ctx->stream>>>(n, x, r, d, v, ctx->scal, ctx->ctl,
-                                               ctx->red.partials + (size_t)S_RR * kMaxPartials);
+void pcg_xr_update(pp_ctx *ctx, uint32_t n, unsigned np_dv, T *x, T *r, const T *d, const T *v, int hist_on,
+                   bool publish, T *w, uint32_t lvl0_lo, uint32_t lvl0_hi, int mode0, const T *diag0) {
+    const unsigned g = pcg_grid(ctx, n);
+    const double *part = ctx->red.partials;
+    k_pcg_xr<T><<<g, kFinishThreads, 0, ctx->stream>>>(
+        n, x, r, d, v, ctx->scal, ctx->ctl, part + (size_t)S_DV * kMaxPartials, np_dv,
+        part + (size_t)S_DR * kMaxPartials, g, ctx->red.partials + (size_t)S_RR * kMaxPartials, w, lvl0_lo, lvl0_hi,
+        mode0, diag0);
     launch_finish(ctx, S_RR, g, ctx->ctl + C_STOP, FIN_PCG_CHECK, hist_on ? ctx->hist : nullptr,
                   hist_on ? ctx->hist_cap : 0, publish ? ctx->ring_dev : nullptr);
     PP_HIP(hipGetLastError());
@@ -1445,9 +1521,10 @@ template void pcg_d_update<double>(pp_ctx *, uint32_t, bool, const double *, dou
 template void pcg_d_update<float>(pp_ctx *, uint32_t, bool, const float *, float *, const float *);
 template void pcg_wv<double>(pp_ctx *, uint32_t, const double *, const double *);
 template void pcg_wv<float>(pp_ctx *, uint32_t, const float *, const float *);
-template void pcg_xr_update<double>(pp_ctx *, uint32_t, double *, double *, const double *, const double *, int,
-                                    bool);
-template void pcg_xr_update<float>(pp_ctx *, uint32_t, float *, float *, const float *, const float *, int, bool);
+template void pcg_xr_update<double>(pp_ctx *, uint32_t, unsigned, double *, double *, const double *, const double *,
+                                    int, bool, double *, uint32_t, uint32_t, int, const double *);
+template void pcg_xr_update<float>(pp_ctx *, uint32_t, unsigned, float *, float *, const float *, const float *, int,
+                                   bool, float *, uint32_t, uint32_t, int, const float *);
 
 // ---------------------------------------------------------------------------
 // Single-reduction preconditioned CG (Chronopoulos & Gear, J. Comput. Appl.

@@ -221,25 +221,33 @@ PcgResult pcg_device(pp_ctx *ctx, pp_csr *A, pp_precond *M, bool flexible, const
     else PP_HIP(hipMemcpyAsync(w, r, (size_t)n * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
     pcg_d_update<T>(ctx, n, true, w, d, r);
     launch_spmv(ctx, A, DT, 1.0, d, 0.0, v, S_DV, d, false);
-    pcg_xr_update<T>(ctx, n, x, r, d, v, hist_on, false);
+    const unsigned np = spmv_grid(A);
+    // the residual update also produces the next apply's dependency-free
+    // first forward level (one launch less per iteration)
+    const bool l0 = flexible && precond_level0_fusable(M);
+    const uint32_t l0_lo = l0 ? M->lvl0_lo : 0, l0_hi = l0 ? M->lvl0_hi : 0;
+    const T *diag0 = !l0 ? nullptr : sizeof(T) == 8 ? (const T *)M->low64.diag : (const T *)M->low32.diag;
+    const int mode0 = l0 ? M->hlow.mode : 0;
+    pcg_xr_update<T>(ctx, n, np, x, r, d, v, hist_on, false, w, l0_lo, l0_hi, mode0, diag0);
 
     int ctl[C_COUNT];
     const uint32_t every = std::max<uint32_t>(1, check_every);
     auto body = [&] {
         StopScope scope(ctx);  // a body past convergence returns at once, SpMV included
         for (uint32_t k = 0; k < every; ++k) {
-            if (flexible && M) precond_apply(ctx, M, DT, r, w);
+            if (l0) precond_apply_after_level0(ctx, M, DT, r, w);
+            else if (flexible && M) precond_apply(ctx, M, DT, r, w);
             else PP_HIP(hipMemcpyAsync(w, r, (size_t)n * sizeof(T), hipMemcpyDeviceToDevice, ctx->stream));
             pcg_wv<T>(ctx, n, w, v);
             pcg_d_update<T>(ctx, n, false, w, d, r);
             launch_spmv(ctx, A, DT, 1.0, d, 0.0, v, S_DV, d, false);
             // the body's last check publishes the control words to the host
-            pcg_xr_update<T>(ctx, n, x, r, d, v, hist_on, k + 1 == every);
+            pcg_xr_update<T>(ctx, n, np, x, r, d, v, hist_on, k + 1 == every, w, l0_lo, l0_hi, mode0, diag0);
         }
     };
     const std::vector<uint64_t> key = {1,          sizeof(T),  A->uid,     (uint64_t)A->v32,
                                        M ? M->uid : 0, M ? (uint64_t)M->io_permuted : 0, M ? (uint64_t)M->have32 : 0,
-                                       (uint64_t)flexible, every, (uint64_t)hist_on, (uint64_t)ctx->hist,
+                                       (uint64_t)flexible, (uint64_t)l0, every, (uint64_t)hist_on, (uint64_t)ctx->hist,
                                        ctx->hist_cap, (uint64_t)r, (uint64_t)w, (uint64_t)d, (uint64_t)v,
                                        (uint64_t)x, (uint64_t)b, variant_key(A, M)};
     double norm;
