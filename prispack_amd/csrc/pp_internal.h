@@ -601,7 +601,8 @@ double *gmres_coeff_buffer(pp_ctx *ctx);
 template <class TV>
 void launch_gemv_t(pp_ctx *ctx, uint32_t n, uint32_t ncol, const TV *V, size_t ld, const TV *w, double *dest);
 template <class TV>
-void launch_gemv_sub(pp_ctx *ctx, uint32_t n, uint32_t ncol, const TV *V, size_t ld, const double *h, TV *w);
+void launch_gemv_sub(pp_ctx *ctx, uint32_t n, uint32_t ncol, const TV *V, size_t ld, const double *h, TV *w,
+                     double *norm_partials = nullptr);
 // w -= V h1 followed by dest = V^T w, in one pass over V where it can
 template <class TV>
 void launch_gemv_sub_t(pp_ctx *ctx, uint32_t n, uint32_t ncol, const TV *V, size_t ld, const double *h1, TV *w,
@@ -614,19 +615,21 @@ void read_slots(pp_ctx *ctx, int first, int count, double *out);
 // scalars misc[kGmMisc]
 struct GmresDev {
     double *H = nullptr, *c = nullptr, *s = nullptr, *g = nullptr, *h1 = nullptr, *h2 = nullptr, *misc = nullptr;
+    double *gb = nullptr;    // the right-hand side before each step's rotation (g holds the rotated one)
+    double *norm = nullptr;  // partial sums of ||w||^2
     uint32_t mm = 0;
 };
 // GM_HBASE: the residual-history index of the cycle's first step
 enum GmMisc {
-    GM_INVH = 0, GM_RELERR, GM_RNORM, GM_M, GM_STATUS, GM_CONVCYC, GM_BNORM, GM_TOL, GM_NREC, GM_HBASE, kGmMisc = 16
+    GM_RELERR = 0, GM_RNORM, GM_M, GM_STATUS, GM_CONVCYC, GM_BNORM, GM_TOL, GM_NREC, GM_HBASE, kGmMisc = 16
 };
 GmresDev gmres_state(pp_ctx *ctx, uint32_t mm);
 void launch_gmres_cycle_init(pp_ctx *ctx, const GmresDev &st, double beta, double bnorm, double tol,
                              uint32_t hist_base);
-void launch_gmres_step(pp_ctx *ctx, const GmresDev &st, uint32_t j, int quirks, double *hist, uint32_t hist_idx,
-                       uint32_t hist_cap);
+// the rotations, the test and v_{j+1} = w / ||w||, from the partials of ||w||^2 in st.norm
 template <class TV>
-void launch_gmres_next_basis(pp_ctx *ctx, const GmresDev &st, uint32_t n, const TV *w, TV *vnext);
+void launch_gmres_step(pp_ctx *ctx, const GmresDev &st, uint32_t j, int quirks, double *hist, uint32_t hist_idx,
+                       uint32_t hist_cap, uint32_t n, const TV *w, TV *vnext);
 void launch_gmres_backsolve(pp_ctx *ctx, const GmresDev &st, int quirks, double *y);
 void launch_permute(pp_ctx *ctx, uint32_t n, const uint32_t *perm, int dtype, const void *src, void *dst,
                     bool gather);

@@ -699,10 +699,9 @@ PcgResult gmres_device(pp_ctx *ctx, pp_csr *A, pp_precond *M, const pp_solve_opt
                     launch_spmv(ctx, A, PP_F32, 1.0, flexible && M ? zj : vj, 0.0, w32, -1, nullptr, false);
                     launch_gemv_t(ctx, n, j + 1, V32, ld, w32, st.h1);
                     launch_gemv_sub_t(ctx, n, j + 1, V32, ld, st.h1, w32, st.h2);
-                    launch_gemv_sub(ctx, n, j + 1, V32, ld, st.h2, w32);
-                    launch_dot(ctx, PP_F32, n, w32, w32, S_TMP2);
-                    launch_gmres_step(ctx, st, j, quirks, hist_on ? ctx->hist : nullptr, j, hist_cap);
-                    launch_gmres_next_basis(ctx, st, n, w32, V32 + ld * (j + 1));
+                    launch_gemv_sub(ctx, n, j + 1, V32, ld, st.h2, w32, st.norm);
+                    launch_gmres_step(ctx, st, j, quirks, hist_on ? ctx->hist : nullptr, j, hist_cap, n, w32,
+                                      V32 + ld * (j + 1));
                     continue;
                 }
                 double *vj = V + ld * j;
@@ -718,10 +717,9 @@ PcgResult gmres_device(pp_ctx *ctx, pp_csr *A, pp_precond *M, const pp_solve_opt
                 // CGS2: h1 = V^T w, w -= V h1, h2 = V^T w, w -= V h2
                 launch_gemv_t(ctx, n, j + 1, V, ld, w, st.h1);
                 launch_gemv_sub_t(ctx, n, j + 1, V, ld, st.h1, w, st.h2);  // w -= V h1; h2 = V^T w
-                launch_gemv_sub(ctx, n, j + 1, V, ld, st.h2, w);
-                launch_dot(ctx, PP_F64, n, w, w, S_TMP2);
-                launch_gmres_step(ctx, st, j, quirks, hist_on ? ctx->hist : nullptr, j, hist_cap);
-                launch_gmres_next_basis(ctx, st, n, w, V + ld * (j + 1));
+                launch_gemv_sub(ctx, n, j + 1, V, ld, st.h2, w, st.norm);
+                launch_gmres_step(ctx, st, j, quirks, hist_on ? ctx->hist : nullptr, j, hist_cap, n, w,
+                                  V + ld * (j + 1));
             }
         };
         // the cycle's launches are the same every cycle of the same length:
