@@ -268,7 +268,7 @@ def extra_records(torch, pp, args):
         timed(torch, run)
         dt, its = timed(torch, run)
         return {"workload": f"{nsys} 2D variable-coefficient diffusion systems, side U[32,256] (sum n={B.n}), "
-                            "one persistent IC(0)-PCG launch (colour-ordered systems), mixed precision, rtol 1e-8",
+                            "batched IC(0)-PCG (colour-ordered systems), mixed precision, rtol 1e-8",
                 "s": round(dt, 5), "setup_s": round(setup, 3), "block": blk, "iters_max": int(its.max()),
                 "iters_mean": float(its.mean()), "relres": B.report.true_relres,
                 "converged": bool(B.report.converged)}

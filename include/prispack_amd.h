@@ -146,10 +146,11 @@ enum {
     PP_TRSV_AUTO = 0,
     PP_TRSV_LEVELS = 1,    /* one launch per level (graph-captured)               */
     PP_TRSV_SYNCFREE = 2,  /* one launch per sweep, per-row ready flags            */
-    PP_TRSV_BLOCK = 3,     /* both sweeps in one workgroup, the vector in LDS (n * 8
-                              bytes must fit in LDS; larger systems use LEVELS).
-                              AUTO times it against LEVELS at setup when it fits   */
-    PP_TRSV_PIPE = 4,      /* one workgroup as BLOCK, level data staged in an LDS
+    PP_TRSV_BLOCK = 3,     /* both sweeps in one workgroup per dependency-closed
+                              chunk of rows, its vector in LDS (a chunk's n * 8
+                              bytes must fit; else LEVELS).  AUTO takes it when
+                              it fits, unless LEVELS is faster                     */
+    PP_TRSV_PIPE = 4,      /* chunks as BLOCK, level data staged in an LDS
                               ring by the workgroup's other waves (AUTO does not
                               pick it)                                             */
     PP_TRSV_STRIPS = 5     /* contiguous strips of rows, a workgroup each, that pass
@@ -242,8 +243,8 @@ int pp_precond_setup(pp_ctx *ctx, pp_precond *M);
 /* Numeric re-factorization from the matrix's current values (pp_csr_set_values
  * keeps the pattern).  No reference counterpart: the reference's setup() does
  * nothing once ready (IncompleteCholesky.cpp:105) and a new object has to be
- * made.  IC(0) and ILU(0) (any ordering, any schedule but PP_TRSV_BLOCK/PIPE) are
- * factored on the device: one launch per dependency level, one thread per
+ * made.  IC(0) and ILU(0) (any ordering, any schedule but PP_TRSV_BLOCK, PIPE and
+ * STRIPS) are factored on the device: one launch per dependency level, one thread per
  * row, the host factorization's operation order (the factor is the same bit
  * for bit), written into the existing sweeps (graphs captured with them stay
  * valid); the symbolic maps are built by the first call.  Other kinds run the
@@ -406,11 +407,14 @@ int pp_csr_outer_on_pattern(pp_ctx *ctx, const pp_csr *A, double scale, const do
                             const double *x, double *grad_values);
 
 /* ---- batched solves (no reference counterpart): nsys independent CSR systems
- * stored back to back (block-diagonal), solved by one persistent launch of
- * IC(0)-PCG with one workgroup per system.  Offsets are host arrays. ---- */
+ * stored back to back (block-diagonal), solved together by IC(0)-PCG: one
+ * persistent launch with a workgroup per system, or, for mixed solves of
+ * two-colour systems, tiles of a system on a workgroup each.  Offsets are host
+ * arrays. ---- */
 typedef struct pp_batch pp_batch;
 int pp_batch_create(pp_ctx *ctx, uint32_t nsys, const uint32_t *row_off, const uint32_t *rowptr,
                     const uint32_t *colidx, const double *values, pp_batch **out);
+/* New values (same patterns): factored on the device, a workgroup per system. */
 int pp_batch_set_values(pp_ctx *ctx, pp_batch *B, const double *values, int on_device);
 /* PP_ORDER_MULTICOLOR: solve every system as P_s A_s P_s^T with its rows
  * grouped by a greedy colouring (one sweep level per colour instead of one per

@@ -563,9 +563,10 @@ class GMRES(_Solver):
 
 # ----------------------------------------------------------------------------- batched systems
 class BatchedSystems:
-    """Many independent SPD systems (block-diagonal CSR) solved together by ONE
-    persistent, graph-captured IC(0)-PCG launch, one workgroup per system
-    (no reference counterpart).  `systems` is a list of (rp, ci, v) CSR
+    """Many independent SPD systems (block-diagonal CSR) solved together by
+    IC(0)-PCG (no reference counterpart): one persistent launch with a
+    workgroup per system, or, for mixed solves of two-colour systems, tiles of
+    a system on a workgroup each.  `systems` is a list of (rp, ci, v) CSR
     triples; right-hand sides and solutions are concatenated CUDA float64
     tensors.  Solves start from x0 = 0."""
 

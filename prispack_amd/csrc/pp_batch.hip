@@ -1,11 +1,13 @@
 // pp_batch.hip -- batched persistent IC(0)-preconditioned CG over many
-// independent SPD systems of uneven size.  ONE launch solves the whole batch:
-// workgroup s owns system s for the entire solve (SpMV, both triangular
-// sweeps level by level with workgroup barriers, workgroup reductions, the
-// FP64 refinement loop), so no grid-wide synchronisation is ever needed and
-// ~256 systems fill the 256 CUs.  The launch is captured in a hipGraph and
-// replayed.  The workgroup size (the row tile each SpMV / sweep step covers)
-// is chosen per batch by a small timing autotuner.
+// independent SPD systems of uneven size.  k_batch_pcg solves the whole batch
+// in one launch: workgroup s owns system s for the entire solve (SpMV, both
+// triangular sweeps level by level with workgroup barriers, workgroup
+// reductions, the FP64 refinement loop), so no grid-wide synchronisation is
+// ever needed and ~256 systems fill the 256 CUs.  The launch is captured in a
+// hipGraph and replayed.  The workgroup size (the row tile each SpMV / sweep
+// step covers) is chosen per batch by a small timing autotuner.  Mixed solves
+// whose systems all have the reduced form spread each system over tiles
+// instead (k_tile_cg, k_batch_step below).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
