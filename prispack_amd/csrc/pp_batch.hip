@@ -7,7 +7,7 @@
 // hipGraph and replayed.  The workgroup size (the row tile each SpMV / sweep
 // step covers) is chosen per batch by a small timing autotuner.  Mixed solves
 // whose systems all have the reduced form spread each system over tiles
-// instead (k_tile_cg, k_batch_step below).
+// instead (k_tile_cg, k_step_* below).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -493,8 +493,8 @@ __global__ __launch_bounds__(BS) void k_batch_pcg(BatchArgs a) {
 
 // ---------------------------------------------------------------------------
 // The mixed solve of a batch in reduced form with every system's inner CG
-// spread over tiles, a workgroup each (k_tile_cg), and one launch per
-// refinement step around it (k_batch_step).
+// spread over tiles, a workgroup each (k_tile_cg), and the refinement steps
+// around it over slices of rows (k_step_*).
 //
 // One workgroup per system left the largest system alone on one compute unit
 // (65,536 rows: 135 us an iteration, 4.4 MB of operators and vectors streamed
@@ -514,11 +514,11 @@ __global__ __launch_bounds__(BS) void k_batch_pcg(BatchArgs a) {
 // past the deadline raises the abort word, which ends every tile, and the
 // batch is solved by k_batch_pcg instead.
 // A solve of 256 systems of 32^2 to 256^2 rows: 88 ms with one workgroup a
-// system, 8.3 ms now, 6.6 of it here.  Two workgroups of 256 threads a unit
+// system, 7.3 ms now, 6.5 of it here.  Two workgroups of 256 threads a unit
 // hide each other's exchange: one of 512 threads, the same rows and registers
-// a thread, took 8.6 (24 systems of 60^2 to 200^2: 2.72, now 2.51).
+// a thread, took 0.3 ms more (24 systems of 60^2 to 200^2: 2.72 against 2.51).
 // ---------------------------------------------------------------------------
-constexpr int kTileThreads = 256, kStepThreads = 1024;
+constexpr int kTileThreads = 256;
 // rows of F, owned rows, halo rows of a thread, by the entries of a row
 template <int W>
 struct TileShape {
@@ -542,7 +542,7 @@ struct TileArgs {
     uint32_t nslot, ntiles;
     int *abort;
     long long deadline;
-    const int32_t *active;          // per system, set by k_batch_step
+    const int32_t *active;          // per system, set by k_step_test
     const double *want, *rin_norm;
     const uint32_t *left;           // iterations the system may still take
     const uint32_t *kab_rp;
@@ -775,79 +775,169 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_cg(TileArgs a) {
     if (tid == 0 && blockIdx.x == t.tile0) a.iters[t.sys] += (int32_t)m;
 }
 
-// One refinement step of the batch, a workgroup per system: the last inner
-// solve's correction (not in the first step), the FP64 residual and its
-// test, then the next inner solve's right-hand side r = KF rin, rin = (b -
-// A x) / ||b - A x||.
+// One refinement step of the batch: the last inner solve's correction (not in
+// the first step), the FP64 residual and its test, then the next inner
+// solve's right-hand side r = KF rin, rin = (b - A x) / ||b - A x||.  It
+// streams the operators once, so the rows go over all of the chip in slices
+// of kSliceRows, and each of its three sums or row couplings across slices is
+// the end of a launch.  A workgroup per system in one launch took 565 us for
+// 256 systems of 32^2 to 256^2 rows, the largest system's 64 rows a thread
+// behind one another; the five launches take 232 us (residual 127).
+constexpr int kSliceThreads = 256;
+constexpr uint32_t kSliceRows = kSliceThreads, kSliceWidth = 7;  // entries of a row at most (batch_build_tiles)
+struct Slice {
+    uint32_t sys, i0, i1;
+};
 struct StepState {
+    const Slice *slices;
+    const uint32_t *first;  // [nsys + 1] slices of a system
+    double *part;           // two sums of a slice
     int32_t *active;
     double *want, *rin_norm, *rn, *normb;
     uint32_t *left;
     int *any;  // set when a system goes on
 };
-__global__ __launch_bounds__(kStepThreads) void k_batch_step(BatchArgs a, StepState st, int begin) {
-    constexpr int BS = kStepThreads;
-    __shared__ double sh[BS / 64];
-    const uint32_t s = blockIdx.x, r0 = a.roff[s], r1 = a.roff[s + 1], m0 = r0 + a.red_n0[s];
-    if (!begin && !st.active[s]) return;
-    double normb;
-    int outer = 0;
-    uint32_t total = 0;
+
+// Row i0 + thread of K x for the slice's rows [i0, i1): the entries and what
+// they gather come in coalesced and go through LDS, a thread then adds its
+// row's in order (row by row from memory the residual took 329 us, its lanes
+// 40 bytes apart).
+template <class T>
+struct SliceStage {
+    T v[kSliceRows * kSliceWidth], x[kSliceRows * kSliceWidth];
+};
+template <class T>
+__device__ inline T slice_row(const uint32_t *__restrict__ rp, const uint32_t *__restrict__ ci,
+                              const T *__restrict__ val, const T *x, uint32_t i0, uint32_t i1, SliceStage<T> &st) {
+    if (i0 >= i1) return (T)0;
+    const uint32_t e0 = rp[i0], cnt = rp[i1] - e0, i = i0 + threadIdx.x;
+    uint32_t c[kSliceWidth];
+    T v[kSliceWidth], g[kSliceWidth];
+#pragma unroll
+    for (uint32_t u = 0; u < kSliceWidth; ++u) {
+        const uint32_t k = min(threadIdx.x + u * kSliceThreads, cnt - 1);  // every row holds its diagonal
+        c[u] = ci[e0 + k];
+        v[u] = val[e0 + k];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kSliceWidth; ++u) g[u] = x[c[u]];
+#pragma unroll
+    for (uint32_t u = 0; u < kSliceWidth; ++u) {
+        const uint32_t k = threadIdx.x + u * kSliceThreads;
+        if (k < cnt) {
+            st.v[k] = v[u];
+            st.x[k] = g[u];
+        }
+    }
+    __syncthreads();
+    T sum = 0;
+    if (i < i1)
+        for (uint32_t k = rp[i] - e0, e = rp[i + 1] - e0; k < e; ++k) sum += st.v[k] * st.x[k];
+    return sum;
+}
+
+// The sum of a system's slices (q: which of the two), in every thread.
+__device__ inline double slice_sum(const StepState &st, uint32_t s, int q, double *sh) {
+    double v = 0.0;
+    for (uint32_t k = st.first[s] + threadIdx.x; k < st.first[s + 1]; k += kSliceThreads) v += st.part[2 * (size_t)k + q];
+    return block_reduce<kSliceThreads>(v, sh);
+}
+
+// x = 0 and (b, b); or e = [KE [rin_0; e_1]; e_1] (a KE row holds its diagonal
+// and second-colour columns, so it reads rin_0 in its own row only) and x += rn e
+__global__ __launch_bounds__(kSliceThreads) void k_step_correct(BatchArgs a, StepState st, int begin) {
+    __shared__ double sh[kSliceThreads / 64];
+    __shared__ SliceStage<float> stage;
+    const Slice c = st.slices[blockIdx.x];
+    const uint32_t m0 = min(c.i1, a.roff[c.sys] + a.red_n0[c.sys]), i = c.i0 + threadIdx.x;
     if (begin) {
         double bb = 0.0;
-        for (uint32_t i = r0 + threadIdx.x; i < r1; i += BS) {
-            bb += a.b[i] * a.b[i];
+        if (i < c.i1) {
+            bb = a.b[i] * a.b[i];
             a.x[i] = 0.0;
         }
-        normb = sqrt(block_reduce<BS>(bb, sh));
-    } else {
-        normb = st.normb[s];
-        outer = a.outer[s] + 1;
-        total = (uint32_t)a.iters[s];
-        // e = [KE [rin_0; e_1]; e_1]
-        for (uint32_t i = r0 + threadIdx.x; i < m0; i += BS) a.q32[i] = a.r32[i];
-        __syncthreads();
-        sys_spmv<float, float>(a.kfe_rp, a.kfe_ci, a.kfe_v, a.q32, a.e32, r0, m0);
-        __syncthreads();
-        const double rn = st.rn[s];
-        for (uint32_t i = r0 + threadIdx.x; i < r1; i += BS) a.x[i] += rn * (double)a.e32[i];
+        bb = block_reduce<kSliceThreads>(bb, sh);
+        if (threadIdx.x == 0) st.part[2 * (size_t)blockIdx.x] = bb;
+        return;
     }
+    if (!st.active[c.sys]) return;
+    if (i < m0) a.q32[i] = a.r32[i];
     __syncthreads();
-    sys_spmv<double, double>(a.rp, a.ci, a.v64, a.x, a.r64, r0, r1);
-    __syncthreads();
+    const float e0 = slice_row<float>(a.kfe_rp, a.kfe_ci, a.kfe_v, a.q32, c.i0, m0, stage);
+    if (i < c.i1) a.x[i] += st.rn[c.sys] * (double)(i < m0 ? e0 : a.e32[i]);
+}
+
+// b - A x and its squares' sum
+__global__ __launch_bounds__(kSliceThreads) void k_step_residual(BatchArgs a, StepState st, int begin) {
+    __shared__ double sh[kSliceThreads / 64];
+    __shared__ SliceStage<double> stage;
+    const Slice c = st.slices[blockIdx.x];
+    if (!begin && !st.active[c.sys]) return;
+    const uint32_t i = c.i0 + threadIdx.x;
+    const double ax = slice_row<double>(a.rp, a.ci, a.v64, a.x, c.i0, c.i1, stage);
     double rr = 0.0;
-    for (uint32_t i = r0 + threadIdx.x; i < r1; i += BS) {
-        const double t = a.b[i] - a.r64[i];
+    if (i < c.i1) {
+        const double t = a.b[i] - ax;
         a.r64[i] = t;
-        rr += t * t;
+        rr = t * t;
     }
-    const double rn = sqrt(block_reduce<BS>(rr, sh));
+    rr = block_reduce<kSliceThreads>(rr, sh);
+    if (threadIdx.x == 0) st.part[2 * (size_t)blockIdx.x + 1] = rr;
+}
+
+// The test, a workgroup per system.
+__global__ __launch_bounds__(kSliceThreads) void k_step_test(BatchArgs a, StepState st, int begin) {
+    __shared__ double sh[kSliceThreads / 64];
+    const uint32_t s = blockIdx.x;
+    if (!begin && !st.active[s]) return;
+    const double normb = begin ? sqrt(slice_sum(st, s, 0, sh)) : st.normb[s];
+    const double rn = sqrt(slice_sum(st, s, 1, sh));
+    if (threadIdx.x != 0) return;
+    const int outer = begin ? 0 : a.outer[s] + 1;
+    const uint32_t total = begin ? 0 : (uint32_t)a.iters[s];
     const double rel = normb > 0 ? rn / normb : 0.0;
     const bool done = rel < a.tol || !(rel == rel) || (uint32_t)outer >= a.max_outer || total >= a.maxit;
-    if (threadIdx.x == 0) {
-        a.iters[s] = (int32_t)total;
-        a.outer[s] = outer;
-        a.conv[s] = rel < a.tol;
-        a.relres[s] = rel;
-        st.active[s] = !done;
-        st.normb[s] = normb;
-        st.rn[s] = rn;
-        st.want[s] = fmax(a.inner_tol, 0.5 * a.tol * normb / rn);
-        st.left[s] = a.maxit - total;
-        if (!done) *st.any = 1;
-    }
-    if (done) return;
-    const float sc = (float)(1.0 / rn);
+    a.iters[s] = (int32_t)total;
+    a.outer[s] = outer;
+    a.conv[s] = rel < a.tol;
+    a.relres[s] = rel;
+    st.active[s] = !done;
+    st.normb[s] = normb;
+    st.rn[s] = rn;
+    st.want[s] = fmax(a.inner_tol, 0.5 * a.tol * normb / rn);
+    st.left[s] = a.maxit - total;
+    if (!done) *st.any = 1;
+}
+
+// rin and its squares' sum
+__global__ __launch_bounds__(kSliceThreads) void k_step_scale(BatchArgs a, StepState st) {
+    __shared__ double sh[kSliceThreads / 64];
+    const Slice c = st.slices[blockIdx.x];
+    if (!st.active[c.sys]) return;
+    const float sc = (float)(1.0 / st.rn[c.sys]);
+    const uint32_t i = c.i0 + threadIdx.x;
     double bb = 0.0;
-    for (uint32_t i = r0 + threadIdx.x; i < r1; i += BS) {
+    if (i < c.i1) {
         const float v = (float)a.r64[i] * sc;
         a.r32[i] = v;
-        bb += (double)v * (double)v;
+        bb = (double)v * (double)v;
     }
-    const double nin = sqrt(block_reduce<BS>(bb, sh));
-    if (threadIdx.x == 0) st.rin_norm[s] = nin;
-    __syncthreads();
-    sys_spmv<float, float>(a.kfe_rp, a.kfe_ci, a.kfe_v, a.r32, a.q32, m0, r1);
+    bb = block_reduce<kSliceThreads>(bb, sh);
+    if (threadIdx.x == 0) st.part[2 * (size_t)blockIdx.x] = bb;
+}
+
+// r = KF rin; a system's first slice also leaves ||rin||
+__global__ __launch_bounds__(kSliceThreads) void k_step_rhs(BatchArgs a, StepState st) {
+    __shared__ double sh[kSliceThreads / 64];
+    __shared__ SliceStage<float> stage;
+    const Slice c = st.slices[blockIdx.x];
+    if (!st.active[c.sys]) return;
+    const uint32_t m0 = max(c.i0, a.roff[c.sys] + a.red_n0[c.sys]);
+    const float q = slice_row<float>(a.kfe_rp, a.kfe_ci, a.kfe_v, a.r32, m0, c.i1, stage);
+    if (m0 + threadIdx.x < c.i1) a.q32[m0 + threadIdx.x] = q;
+    if (blockIdx.x != st.first[c.sys]) return;
+    const double nin = sqrt(slice_sum(st, c.sys, 0, sh));
+    if (threadIdx.x == 0) st.rin_norm[c.sys] = nin;
 }
 
 }  // namespace
@@ -902,6 +992,9 @@ struct pp_batch {
     double *state = nullptr;   // want, rin_norm, rn, normb: nsys each
     uint32_t *left = nullptr;
     int *tile_flag = nullptr;  // any, abort
+    pp::Slice *slices = nullptr;   // of the refinement steps' rows
+    uint32_t *slice0 = nullptr, nslice = 0;
+    double *slice_sums = nullptr;
 };
 
 namespace pp {
@@ -1293,6 +1386,11 @@ void batch_free_refresh(pp_batch *B) {
 void batch_free_tiles(pp_batch *B) {
     dfree(B->tiles); dfree(B->tile_rows); dfree(B->tile_slots); dfree(B->tile_loc); dfree(B->tile_w);
     dfree(B->tile_sums); dfree(B->active); dfree(B->state); dfree(B->left); dfree(B->tile_flag);
+    dfree(B->slices); dfree(B->slice0); dfree(B->slice_sums);
+    B->slices = nullptr;
+    B->slice0 = nullptr;
+    B->slice_sums = nullptr;
+    B->nslice = 0;
     B->tiles = nullptr;
     B->tile_rows = B->tile_slots = B->left = nullptr;
     B->tile_loc = nullptr;
@@ -1393,6 +1491,14 @@ bool batch_build_tiles(pp_batch *B, const std::vector<ReducedHost> &reds) {
         for (uint32_t q = 0; q < H.n1; ++q) width = std::max(width, H.kb_rp[q + 1] - H.kb_rp[q] - 1);
     }
     if (width > 6) return false;
+    for (uint32_t i = 0; i < B->ntot; ++i)  // a row's diagonal beside them (k_step_*)
+        if (B->h_prp[i + 1] - B->h_prp[i] > kSliceWidth) return false;
+    for (const ReducedHost &H : reds) {
+        for (uint32_t i = 0; i < H.n0; ++i)
+            if (H.ke_rp[i + 1] - H.ke_rp[i] > kSliceWidth) return false;
+        for (uint32_t q = 0; q < H.n1; ++q)
+            if (H.kf_rp[q + 1] - H.kf_rp[q] > kSliceWidth) return false;
+    }
     const int W = width <= 4 ? 4 : 6;
     const uint32_t maxf = kTileThreads * (W == 4 ? TileShape<4>::kF : TileShape<6>::kF);
     const uint32_t maxs = kTileThreads * (W == 4 ? TileShape<4>::kS : TileShape<6>::kS);
@@ -1463,6 +1569,18 @@ bool batch_build_tiles(pp_batch *B, const std::vector<ReducedHost> &reds) {
     B->state = dalloc<double>(4 * (size_t)ns);
     B->left = dalloc<uint32_t>(ns);
     B->tile_flag = dalloc<int>(2);
+    std::vector<Slice> slices;
+    std::vector<uint32_t> slice0;
+    for (uint32_t s = 0; s < ns; ++s) {
+        slice0.push_back((uint32_t)slices.size());
+        for (uint32_t i = B->h_roff[s]; i < B->h_roff[s + 1]; i += kSliceRows)
+            slices.push_back({s, i, std::min(B->h_roff[s + 1], i + kSliceRows)});
+    }
+    slice0.push_back((uint32_t)slices.size());
+    B->slices = (Slice *)up(slices.data(), slices.size() * sizeof(Slice));
+    B->slice0 = upload(slice0);
+    B->nslice = (uint32_t)slices.size();
+    B->slice_sums = dalloc<double>(2 * slices.size());
     B->tile_width = W;
     return true;
 }
@@ -1679,6 +1797,9 @@ void run_batch(pp_ctx *ctx, pp_batch *B, bool mixed, const BatchArgs &a) {
 bool run_tiles(pp_ctx *ctx, pp_batch *B, const BatchArgs &a) {
     const uint32_t ns = B->nsys;
     StepState st;
+    st.slices = B->slices;
+    st.first = B->slice0;
+    st.part = B->slice_sums;
     st.active = B->active;
     st.want = B->state;
     st.rin_norm = B->state + ns;
@@ -1710,7 +1831,11 @@ bool run_tiles(pp_ctx *ctx, pp_batch *B, const BatchArgs &a) {
     t.iters = B->iters;
     for (int begin = 1;; begin = 0) {
         launch_fill_zero(ctx, B->tile_flag, (begin ? 2 : 1) * sizeof(int));  // the abort word stays
-        k_batch_step<<<ns, kStepThreads, 0, ctx->stream>>>(a, st, begin);
+        k_step_correct<<<B->nslice, kSliceThreads, 0, ctx->stream>>>(a, st, begin);
+        k_step_residual<<<B->nslice, kSliceThreads, 0, ctx->stream>>>(a, st, begin);
+        k_step_test<<<ns, kSliceThreads, 0, ctx->stream>>>(a, st, begin);
+        k_step_scale<<<B->nslice, kSliceThreads, 0, ctx->stream>>>(a, st);
+        k_step_rhs<<<B->nslice, kSliceThreads, 0, ctx->stream>>>(a, st);
         PP_HIP(hipGetLastError());
         int flag[2];
         PP_HIP(hipMemcpyAsync(flag, B->tile_flag, sizeof(flag), hipMemcpyDeviceToHost, ctx->stream));

@@ -33,6 +33,7 @@ def vardiff(side, seed):
 BATCHES = {
     "small": lambda: [ppo.laplacian(2, 1, 1), ppo.laplacian(3, 2, 1), vardiff(5, 1), vardiff(16, 2)],
     "around_a_tile": lambda: [vardiff(s, s) for s in (45, 46, 63, 64, 65, 90, 91)],
+    "around_a_slice": lambda: [ppo.laplacian(*g, 1) for g in ((17, 15), (16, 16), (257, 1), (73, 7), (32, 16), (2, 1))],
     "uneven": lambda: [vardiff(s, s) for s in (200, 33, 129, 8, 70)],
     "seven_point": lambda: [ppo.laplacian(16, 15, 14), ppo.laplacian(24, 23, 22), vardiff(40, 3)],
     "many_tiles": lambda: [ppo.laplacian(90, 2100, 1), vardiff(20, 5)],
