@@ -242,8 +242,10 @@ void lowrank_lanczos(pp_ctx *ctx, MlState &S, int l, uint32_t rank, uint32_t ste
         // start vector: seeded uniform(-1, 1)
         std::vector<double> u0(n);
         PP_CHECK(pp_fill_random(0, 12345 + l, n, u0.data()) == PP_OK, PP_ERR_INVALID, "rng");
-        PP_HIP(hipMemcpy(u, u0.data(), n * 8, hipMemcpyHostToDevice));
-        PP_HIP(hipMemcpy(w, u, n * 8, hipMemcpyDeviceToDevice));
+        // both on the solves' stream: a copy between device arrays on the default
+        // stream returns before it is done, and this stream does not wait for that one
+        PP_HIP(hipMemcpyAsync(u, u0.data(), (size_t)n * 8, hipMemcpyHostToDevice, ctx->stream));
+        PP_HIP(hipMemcpyAsync(w, u, (size_t)n * 8, hipMemcpyDeviceToDevice, ctx->stream));
         rec_solve(ctx, S, l, w);
         double b0 = dot_dev(ctx, n, w, u);
         PP_CHECK(b0 > 0 && std::isfinite(b0), PP_ERR_BREAKDOWN, "Lanczos start vector has non-positive C-norm");
@@ -461,8 +463,10 @@ void lowrank_lanczos_restarted(pp_ctx *ctx, MlState &S, int l, uint32_t rank, in
         // start: a seeded random z1, v1 = C^{-1} z1 scaled to v1^T C v1 = 1
         std::vector<double> u0(n);
         PP_CHECK(pp_fill_random(0, 12345 + l, n, u0.data()) == PP_OK, PP_ERR_INVALID, "rng");
-        PP_HIP(hipMemcpy(u, u0.data(), (size_t)n * 8, hipMemcpyHostToDevice));
-        PP_HIP(hipMemcpy(w, u, (size_t)n * 8, hipMemcpyDeviceToDevice));
+        // both on the solves' stream: a copy between device arrays on the default
+        // stream returns before it is done, and this stream does not wait for that one
+        PP_HIP(hipMemcpyAsync(u, u0.data(), (size_t)n * 8, hipMemcpyHostToDevice, ctx->stream));
+        PP_HIP(hipMemcpyAsync(w, u, (size_t)n * 8, hipMemcpyDeviceToDevice, ctx->stream));
         rec_solve(ctx, S, l, w);
         double b0 = dot_dev(ctx, n, w, u);
         PP_CHECK(b0 > 0 && std::isfinite(b0), PP_ERR_BREAKDOWN, "Lanczos start vector has non-positive C-norm");
