@@ -693,9 +693,12 @@ void build_row_blocks(const std::vector<uint32_t> &rp, std::vector<uint32_t> &bl
 }
 
 // result = sum of partials[0..np) in index order (one workgroup); op
-// FIN_PCG_CHECK also runs the PCG convergence test on it.
+// FIN_PCG_CHECK also runs the PCG convergence test on it, or stops at the
+// breakdown that k_pcg_xr's workgroups found.
 enum FinishOp : int { FIN_SUM = 0, FIN_PCG_CHECK = 1 };
 __device__ void pcg_check(double rr, const double *scal, int *ctl, double *hist, uint32_t hist_cap);
+// den = (d, A d): zero is a breakdown, NaN means non-finite data
+__device__ inline bool pcg_breakdown(double den) { return den == 0.0 || !(den == den); }
 // ring != NULL (the last check of an iteration body): afterwards the control
 // words are copied into the next mapped pinned slot for the host (plain
 // vector stores over the fabric), also when the body was skipped.  The
@@ -736,10 +739,17 @@ __global__ __launch_bounds__(1024) void k_finish(const double *__restrict__ part
         if (ring && threadIdx.x == 0) publish_ctl(ctl, ring);
         return;
     }
+    const double den = op == FIN_PCG_CHECK ? scal[S_DV] : 1.0;
     double s = block_sum(sum_partials(partials, np), sh);
     if (threadIdx.x == 0) {
-        *result = s;
-        if (op == FIN_PCG_CHECK) pcg_check(s, scal, ctl, hist, hist_cap);
+        if (pcg_breakdown(den)) {
+            ctl[C_STATUS] = den == 0.0 ? PP_ERR_BREAKDOWN : PP_ERR_NOT_FINITE;
+            ctl[C_STOP] = 1;
+            ctl[C_M] = ctl[C_CHECK];
+        } else {
+            *result = s;
+            if (op == FIN_PCG_CHECK) pcg_check(s, scal, ctl, hist, hist_cap);
+        }
         if (ring) publish_ctl(ctl, ring);
     }
 }
@@ -1426,7 +1436,7 @@ __device__ void pcg_check(double rr, const double *scal, int *ctl, double *hist,
 template <class T>
 __global__ __launch_bounds__(1024) void k_pcg_xr(uint32_t n, T *__restrict__ x, T *__restrict__ r,
                                                  const T *__restrict__ d, const T *__restrict__ v, double *scal,
-                                                 int *ctl, const double *__restrict__ dv_partials, unsigned np_dv,
+                                                 const int *ctl, const double *__restrict__ dv_partials, unsigned np_dv,
                                                  const double *__restrict__ dr_partials, unsigned np_dr,
                                                  double *partials, T *__restrict__ w, uint32_t l0, uint32_t l1,
                                                  int mode0, const T *__restrict__ diag0) {
@@ -1452,14 +1462,9 @@ __global__ __launch_bounds__(1024) void k_pcg_xr(uint32_t n, T *__restrict__ x, 
     }
     __syncthreads();
     const double den = sums[0];
-    if (den == 0.0 || !(den == den)) {  // (d, A d) = 0: breakdown; NaN: non-finite data
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            ctl[C_STATUS] = den == 0.0 ? PP_ERR_BREAKDOWN : PP_ERR_NOT_FINITE;
-            ctl[C_STOP] = 1;
-            ctl[C_M] = ctl[C_CHECK];
-        }
-        return;
-    }
+    // x and r stay as they are; k_finish, the next launch, sets the stop word
+    // (a workgroup that starts late would read it in one wavefront and not in another)
+    if (pcg_breakdown(den)) return;
     const T alpha = (T)(sums[1] / den);
     T acc = 0;
     while (i < n) {

@@ -70,3 +70,30 @@ def test_history_against_oracle(torch, grid, precond):
     k = min(len(h), len(ho))
     assert k >= min(want["iters"], 1)
     np.testing.assert_allclose(h[:k], ho[:k], rtol=0, atol=eps)
+
+
+def _blocks2(count, block):
+    """count copies of a 2 x 2 block on the diagonal."""
+    n = 2 * count
+    cols = np.repeat(np.arange(n) // 2 * 2, 2) + np.tile([0, 1], n)
+    return np.arange(0, 2 * n + 1, 2, dtype=np.uint32), cols.astype(np.uint32), np.tile(np.ravel(block), count)
+
+
+# [[1, 1], [1, 1]] with b = (1, 0): step 1 goes to x = (1, 0), step 2 has (d, A d) = 0;
+# [[0, 1], [1, 0]] with b = (1, 0): (d, A d) = 0 at once; all of it in small whole numbers
+@pytest.mark.parametrize("launch", [0, 1])
+@pytest.mark.parametrize("count", [1, 513, 350_001])
+@pytest.mark.parametrize("block,x", [([[1, 1], [1, 1]], (1.0, 0.0)), ([[0, 1], [1, 0]], (0.0, 0.0)),
+                                     ([[1, np.nan], [np.nan, 1]], (0.0, 0.0))])
+def test_breakdown_leaves_x_at_the_step_before(torch, block, x, count, launch):
+    import prispack_amd as pp
+    M = pp.CSRMatrix(*_blocks2(count, np.array(block, float)))
+    b = np.tile([1.0, 0.0], count)
+    for host in (False, True):
+        S = pp.CG(M.n, None, tol=1e-10, maxIter=50).setCGVariant("reference")
+        S.opts.launch = launch
+        got = np.zeros(M.n) if host else torch.zeros(M.n, dtype=torch.float64, device="cuda")
+        with pytest.raises(pp.PrisPackError) as e:
+            S.solve(M, b if host else torch.tensor(b, device="cuda"), got)
+        assert e.value.status == (8 if np.isnan(block).any() else 7) and not S.getConvergence()
+        assert np.array_equal(got if host else got.cpu().numpy(), np.tile(x, count))
