@@ -383,9 +383,11 @@ __global__ void k_gmres_cycle_init(GmresDev st, double beta, double bnorm, doubl
 // test, and v_{j+1} = (1/h_{j+1,j}) w, evaluated like HostVector::add with
 // b = 0.  Whether v_{j+1} is written hangs on the test, so every workgroup
 // runs the rotations itself (thread 0, operands in LDS: about 1 us for 30
-// columns) and workgroup 0 alone writes the state.  Nothing that another
-// workgroup reads is written here: the right-hand side before the rotations
-// is kept in gb, next to g.  One launch instead of four (sum, finish, a
+// columns) and workgroup 0 alone writes the state.  Of what the others read it
+// writes the stop word alone (the right-hand side before the rotations is kept
+// in gb, next to g), which one thread of a workgroup reads for all of it: where
+// that thread finds this very step's stop, the workgroup ends as the test would
+// have had it end.  One launch instead of four (sum, finish, a
 // single-thread step with its operands in device memory, scaling): 21.5 us
 // on 100^3 rows, now 6.7 us.
 template <class TV>
@@ -396,9 +398,9 @@ __global__ __launch_bounds__(kTailThreads) void k_gmres_step(GmresDev st, uint32
                                                              const TV *__restrict__ w, TV *__restrict__ v) {
 #pragma clang fp contract(off)
     __shared__ double sh[kTailThreads / 64], col[kMaxCols + 1], cs[kMaxCols], sn[kMaxCols], inv;
-    __shared__ int go;
-    if (ctl[C_STOP]) return;
+    __shared__ int go, stopped;
     const uint32_t step = gridDim.x * kTailThreads, t = threadIdx.x;
+    if (t == 0) stopped = ctl[C_STOP];
     uint32_t i = blockIdx.x * kTailThreads + t;
     TV wi = 0;
     if (i < n) wi = w[i];
@@ -412,6 +414,7 @@ __global__ __launch_bounds__(kTailThreads) void k_gmres_step(GmresDev st, uint32
         sn[t] = st.s[t];
     }
     __syncthreads();
+    if (stopped) return;
     if (t == 0) {
         const uint32_t ld = st.mm + 1;
         double *H = st.H + (size_t)j * ld;

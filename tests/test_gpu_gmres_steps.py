@@ -66,3 +66,28 @@ def test_preconditioned_residual(torch, grid, precision):
     # the estimate is below 1e-9; the residual itself adds the basis's
     # rounding, 2^-24 of the cycle's first residual in FP32
     assert np.linalg.norm(r) <= 1.1e-9 * np.linalg.norm(b) * (1 if precision == "fp64" else 10)
+
+
+@pytest.mark.parametrize("launch", [0, 1])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [3, 1025, 700_001])
+def test_stop_inside_a_cycle(torch, n, precision, launch):
+    # three distinct eigenvalues: the third step of every cycle stops it, on
+    # one workgroup and on all of the grid, the same bits each time
+    import prispack_amd as pp
+    d = np.array([1.0, 2.0, 5.0])[np.arange(n) % 3]
+    M = pp.CSRMatrix(np.arange(n + 1, dtype=np.uint32), np.arange(n, dtype=np.uint32), d)
+    b = torch.tensor(ppo.normal(n, 6), device="cuda")
+    out = []
+    for _ in range(3):
+        S = pp.GMRES(n, None, tolerance=1e-9, precision=precision)
+        S.setRestart(True, 30)
+        S.opts.launch = launch
+        x = torch.zeros_like(b)
+        S.solve(M, b, x)
+        assert S.getConvergence()
+        r = b - torch.tensor(d, device="cuda") * x
+        assert float(r.norm()) <= 1.1e-9 * float(b.norm()) * (1 if precision == "fp64" else 10)
+        out.append((S.getNumIter(), x))
+    for it, x in out[1:]:
+        assert it == out[0][0] and torch.equal(x, out[0][1])
