@@ -1761,11 +1761,10 @@ __global__ __launch_bounds__(1024) void k_red_step(const double *__restrict__ pa
     __shared__ double sh[3 * (kFinishThreads / 64)];
     __shared__ double bc[2];
     __shared__ int go;
-    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    if (ctl[C_STOP]) {  // an earlier check stopped (or this launch's first workgroup already did)
-        if (ring && lead) publish_ctl(ctl, ring);
-        return;
-    }
+    // one thread reads the stop word for its workgroup: the first workgroup may
+    // set it while a late one starts, whose wavefronts must not part ways
+    int prior_stop = 0;
+    if (threadIdx.x == 0) prior_stop = __hip_atomic_load(ctl + C_STOP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // the first kU elements of this thread are loaded before the reduction
     // (they do not depend on alpha / beta), so their latency overlaps it
     constexpr int kU = 4;
@@ -1786,7 +1785,7 @@ __global__ __launch_bounds__(1024) void k_red_step(const double *__restrict__ pa
     double t[3], a64, b64;
 #pragma unroll
     for (int q = 0; q < 3; ++q) t[q] = sum_partials(partials + (size_t)q * kMaxPartials, np);
-    if (!red_check(t, 0, scal, ctl, ring, parity, sh, bc, &go, a64, b64)) return;
+    if (!red_check(t, prior_stop, scal, ctl, ring, parity, sh, bc, &go, a64, b64)) return;
     const T alpha = (T)a64, beta = (T)b64;
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
