@@ -616,6 +616,9 @@ void pp_ctx_destroy(pp_ctx *ctx) {
     dfree(ctx->ctl);
     dfree(ctx->hist);
     dfree(ctx->flush_buf);
+    for (auto &s : ctx->strip_slots)
+        for (auto &side : s) dfree(side.p);
+    for (void *p : ctx->old_strip_slots) dfree(p);
     for (int i = 0; i < 48; ++i) dfree(ctx->ws[i]);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->pinned_ctl) (void)hipHostFree(ctx->pinned_ctl);

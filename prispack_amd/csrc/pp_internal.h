@@ -160,6 +160,14 @@ struct pp_ctx {
     unsigned char *arena = nullptr;
     size_t arena_cap = 0, arena_used = 0;
     size_t arena_off[48] = {}, arena_len[48] = {};
+    // exchange buffers of the strip sweeps that run on this context (FP64,
+    // FP32; forward, backward), grown by strip_slots; the smaller ones they
+    // replaced stay until the context goes, a captured graph may hold them
+    struct StripSlots {
+        void *p = nullptr;
+        uint32_t n = 0;
+    } strip_slots[2][2];
+    std::vector<void *> old_strip_slots;
     long long spin_deadline = 0;   // wall_clock64 ticks a sync-free wait may last
     // while set (StopScope), SpMV / dot / GEMV / convert kernels return at
     // once when the word is non-zero, like the sweeps and the PCG kernels
@@ -283,8 +291,7 @@ template <class T>
 struct StripSide {
     unsigned char *head = nullptr, *data = nullptr;  // per strip, steps
     uint32_t *imp = nullptr;        // imported slots
-    T *slots = nullptr;             // exchange buffer
-    uint32_t nslots = 0, max_words = 0;
+    uint32_t nslots = 0, max_words = 0;  // of the exchange buffer, of LDS
     int mode = 0;
     void free_all();
 };
@@ -754,8 +761,15 @@ void launch_lane_sweep(pp_ctx *ctx, const ChunkSet &C, const LaneSweep<T> &S, co
 // PP_TRSV_STRIPS: false (nothing kept) when the strips do not fit LDS.
 template <class T>
 bool build_strip_sweeps(pp_ctx *ctx, const HostSweep &lo, const HostSweep &up, StripSweep<T> &L);
+// launch_strip_sweeps: false (nothing launched) where the context's exchange
+// buffers are too small and cannot grow, inside a capture or a zero-allocation
+// solve.  strip_reserve grows them ahead of that.
 template <class T>
-void launch_strip_sweeps(pp_ctx *ctx, const StripSweep<T> &L, const T *x, T *y);
+bool launch_strip_sweeps(pp_ctx *ctx, const StripSweep<T> &L, const T *x, T *y);
+template <class T>
+bool strip_reserve(pp_ctx *ctx, const StripSweep<T> &L);
+void precond_reserve(pp_ctx *ctx, const pp_precond *M);
+void ml_reserve(pp_ctx *ctx, const pp_precond *M);
 // The same sweeps from the level-ordered storage (DevChunkSweep), one
 // wavefront computing the levels while the rest of the workgroup stages
 // their data in LDS (PP_TRSV_PIPE, pp_sweep_pipe.hip); sweep_pipe_rings:

@@ -876,6 +876,12 @@ void ml_need_f32(pp_ctx *ctx, pp_precond *M) {
     S->have32 = true;
 }
 
+void ml_reserve(pp_ctx *ctx, const pp_precond *M) {
+    const auto *S = static_cast<const MlState *>(M->multilevel);
+    precond_reserve(ctx, S->last);
+    for (const MlLevel &L : S->lev) precond_reserve(ctx, L.Bpc);
+}
+
 void ml_apply(pp_ctx *ctx, pp_precond *M, int dtype, const void *x, void *y) {
     auto *S = static_cast<MlState *>(M->multilevel);
     PP_CHECK(S, PP_ERR_NOT_READY, "multilevel preconditioner not set up");

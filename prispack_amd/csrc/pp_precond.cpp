@@ -1006,6 +1006,16 @@ pp_csr *precond_permuted_matrix(pp_ctx *ctx, pp_precond *M, pp_csr *A) {
     return M->Aperm;
 }
 
+// The strip sweeps' exchange buffers on ctx, for a solve that may capture its
+// first apply (M's own context has them since M's set-up).
+void precond_reserve(pp_ctx *ctx, const pp_precond *M) {
+    if (!M) return;
+    if (M->multilevel) ml_reserve(ctx, M);
+    if (M->trsv != PP_TRSV_STRIPS) return;
+    strip_reserve(ctx, M->strips64);
+    if (M->have32) strip_reserve(ctx, M->strips32);
+}
+
 // True when a solve may produce the forward sweep's first level itself
 // (launch_level0 on the right-hand side) and call precond_apply_after_level0.
 bool precond_level0_fusable(const pp_precond *M) {
@@ -1082,14 +1092,13 @@ void precond_apply(pp_ctx *ctx, pp_precond *M, int dtype, const void *x, void *y
         }
         return;
     }
-    if (M->trsv == PP_TRSV_STRIPS) {
+    if (M->trsv == PP_TRSV_STRIPS) {  // else the level sweeps below: the same bits
         if (dtype == PP_F64) {
-            launch_strip_sweeps<double>(ctx, M->strips64, (const double *)x, (double *)y);
+            if (launch_strip_sweeps<double>(ctx, M->strips64, (const double *)x, (double *)y)) return;
         } else {
             precond_need_f32(M);
-            launch_strip_sweeps<float>(ctx, M->strips32, (const float *)x, (float *)y);
+            if (launch_strip_sweeps<float>(ctx, M->strips32, (const float *)x, (float *)y)) return;
         }
-        return;
     }
     if (M->trsv == PP_TRSV_PIPE) {
         if (dtype == PP_F64) {

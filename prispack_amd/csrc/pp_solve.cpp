@@ -820,6 +820,7 @@ static int solve_impl(pp_ctx *ctx, pp_csr *A, pp_precond *M, const pp_solve_opts
         PP_CHECK(A && opts && b && x, PP_ERR_INVALID, "NULL argument");
         PP_CHECK(A->nrow == A->ncol, PP_ERR_INVALID, "square matrix required");
         if (M) PP_CHECK(M->ready, PP_ERR_NOT_READY, "preconditioner used before setup()");
+        precond_reserve(ctx, M);
         pp_solve_report R;
         std::memset(&R, 0, sizeof(R));
         const pp_solve_opts &o = *opts;

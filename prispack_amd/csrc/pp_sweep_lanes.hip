@@ -304,8 +304,11 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
 // other wavefronts poll the slots in the order the steps need them and put the
 // values into LDS.  A slot holds a signalling NaN, which no sum is, until its
 // value arrives, so a value is its own ready flag (a value passes between
-// two compute units in about 0.6 us, 0.45 on one XCD).  The slots of one
-// sweep are emptied while the other runs.
+// two compute units in about 0.6 us, 0.45 on one XCD).  The buffers belong to
+// the context, whose stream keeps its applies apart (two contexts may apply
+// one preconditioner at the same time): the forward sweep's is empty between
+// applies, because the backward sweep empties the slots it used, and the
+// backward sweep's is emptied by the forward sweep before it.
 // A strip waits only for strips before it in its sweep's direction, whose
 // workgroups are dispatched before its own, so the first unfinished strip
 // always proceeds; a wait past the deadline sets C_SPIN, and every wavefront
@@ -806,14 +809,14 @@ void upload_strips(const StripHost<T> &H, int mode, StripSide<T> &D) {
     D.head = up(H.head.data(), H.head.size() * sizeof(StripHead));
     D.imp = (uint32_t *)up(H.imp.data(), H.imp.size() * 4);
     D.nslots = H.nslots;
-    D.slots = dalloc<T>(std::max(1u, H.nslots));
     D.max_words = H.max_words;
     D.mode = mode;
 }
 
+// slots: this sweep's exchange buffer; other, on: the other sweep's, to be emptied
 template <class T>
-void launch_strip_side(pp_ctx *ctx, const StripSweep<T> &L, const StripSide<T> &D, const StripSide<T> &O, const T *x,
-                       T *y) {
+void launch_strip_side(pp_ctx *ctx, const StripSweep<T> &L, const StripSide<T> &D, T *slots, uint32_t on, T *other,
+                       const T *x, T *y) {
     const uint32_t ctl_off = (uint32_t)((L.max_words * sizeof(T) + 15) / 16 * 16);
     const size_t lds = ctl_off + kStripCtl;
     PP_CHECK(lds <= ctx->max_lds && D.data, PP_ERR_INVALID, "strip sweep: storage missing or strip exceeds LDS");
@@ -823,8 +826,8 @@ void launch_strip_side(pp_ctx *ctx, const StripSweep<T> &L, const StripSide<T> &
             PP_HIP(hipFuncSetAttribute((const void *)k_sweep_strips<T, G, S, HostSweep::MODE>,                    \
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                    \
         k_sweep_strips<T, G, S, HostSweep::MODE><<<L.nstrip, kLaneThreads, lds, ctx->stream>>>(                   \
-            (const StripHead *)D.head, (const char *)D.data, D.imp, D.slots, O.nslots, O.slots, \
-            ctl_off, x, y, ctx->spin_deadline, ctx->ctl, ctx->stop_word);                                \
+            (const StripHead *)D.head, (const char *)D.data, D.imp, slots, on, other, ctl_off, x, y,             \
+            ctx->spin_deadline, ctx->ctl, ctx->stop_word);                                                        \
     }
 #define PP_STRIPS(G, S)          \
     PP_STRIP(G, S, DIVIDE)       \
@@ -979,10 +982,8 @@ void StripSide<T>::free_all() {
     dfree(head);
     dfree(data);
     dfree(imp);
-    dfree(slots);
     head = data = nullptr;
     imp = nullptr;
-    slots = nullptr;
     nslots = max_words = 0;
 }
 template <class T>
@@ -1032,21 +1033,46 @@ bool build_strip_sweeps(pp_ctx *ctx, const HostSweep &lo, const HostSweep &up, S
     upload_strips<T>(H[1], up.mode, L.up);
     L.nstrip = K;
     L.max_words = std::max(L.lo.max_words, L.up.max_words);
-    for (StripSide<T> *D : {&L.lo, &L.up}) {
-        k_slots_empty<T><<<256, 256, 0, ctx->stream>>>(D->nslots, D->slots);
-        PP_HIP(hipGetLastError());
-    }
+    strip_reserve(ctx, L);
     return true;
 }
 template bool build_strip_sweeps<double>(pp_ctx *, const HostSweep &, const HostSweep &, StripSweep<double> &);
 template bool build_strip_sweeps<float>(pp_ctx *, const HostSweep &, const HostSweep &, StripSweep<float> &);
 
 template <class T>
-void launch_strip_sweeps(pp_ctx *ctx, const StripSweep<T> &L, const T *x, T *y) {
-    launch_strip_side(ctx, L, L.lo, L.up, x, y);
-    launch_strip_side(ctx, L, L.up, L.lo, (const T *)y, y);
+bool strip_reserve(pp_ctx *ctx, const StripSweep<T> &L) {
+    pp_ctx::StripSlots *S = ctx->strip_slots[sizeof(T) == 4];
+    const uint32_t want[2] = {L.lo.nslots, L.up.nslots};
+    if (S[0].p && S[1].p && S[0].n >= want[0] && S[1].n >= want[1]) return true;
+    if (ctx->arena) return false;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    PP_HIP(hipStreamIsCapturing(ctx->stream, &capturing));
+    if (capturing != hipStreamCaptureStatusNone) return false;
+    for (int k = 0; k < 2; ++k) {
+        if (S[k].p && S[k].n >= want[k]) continue;
+        const uint32_t n = std::max({1024u, want[k], 2 * S[k].n});
+        void *p = nullptr;  // not from the set-ups' block pool: it lives as long as the context
+        if (hipMalloc(&p, (size_t)n * sizeof(T)) != hipSuccess) throw Error(PP_ERR_NOMEM, "strip exchange buffer");
+        if (S[k].p) ctx->old_strip_slots.push_back(S[k].p);
+        S[k] = {p, n};
+        k_slots_empty<T><<<256, 256, 0, ctx->stream>>>(n, (T *)p);
+        PP_HIP(hipGetLastError());
+    }
+    return true;
 }
-template void launch_strip_sweeps<double>(pp_ctx *, const StripSweep<double> &, const double *, double *);
-template void launch_strip_sweeps<float>(pp_ctx *, const StripSweep<float> &, const float *, float *);
+template bool strip_reserve<double>(pp_ctx *, const StripSweep<double> &);
+template bool strip_reserve<float>(pp_ctx *, const StripSweep<float> &);
+
+template <class T>
+bool launch_strip_sweeps(pp_ctx *ctx, const StripSweep<T> &L, const T *x, T *y) {
+    if (!strip_reserve(ctx, L)) return false;
+    const pp_ctx::StripSlots *S = ctx->strip_slots[sizeof(T) == 4];
+    T *lo = (T *)S[0].p, *up = (T *)S[1].p;
+    launch_strip_side<T>(ctx, L, L.lo, lo, L.up.nslots, up, x, y);
+    launch_strip_side<T>(ctx, L, L.up, up, L.lo.nslots, lo, y, y);
+    return true;
+}
+template bool launch_strip_sweeps<double>(pp_ctx *, const StripSweep<double> &, const double *, double *);
+template bool launch_strip_sweeps<float>(pp_ctx *, const StripSweep<float> &, const float *, float *);
 
 }  // namespace pp

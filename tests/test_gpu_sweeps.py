@@ -160,3 +160,82 @@ def test_strip_solves_match_levels(pp, torch, kind, launch):
             out.append((s.getNumIter(), x))
     for it, x in out[1:]:
         assert it == out[0][0] and torch.equal(x, out[0][1])
+
+
+def _apply_on(ctx, P, x, y):
+    import ctypes
+    from prispack_amd import _capi
+    p = [ctypes.c_void_p(t.data_ptr()) for t in (x, y)]
+    ctx.check(_capi.lib().pp_precond_apply(ctx.h, P.h, int(x.dtype.itemsize == 4), *p))
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_strips_on_two_contexts_at_once(pp, torch, f32):
+    # a preconditioner's applies on two contexts overlap: each context has its
+    # own exchange buffers; a second, larger factor makes them grow in between
+    import threading
+    Ps = []
+    for grid in ((40, 33, 29), (48, 40, 33)):
+        M = pp.CSRMatrix(*ppo.laplacian(*grid))
+        Ps.append([pp.IncompleteCholesky(M, 1e-2, trsv=t, make_f32=f32) for t in (1, 5)])
+        for P in Ps[-1]:
+            P.setup()
+        assert Ps[-1][1].info().trsv == 5
+    dt = torch.float32 if f32 else torch.float64
+    jobs = []  # (preconditioner, operand, expected, result) by thread
+    for k in range(2):
+        jobs.append([])
+        for i in range(40):
+            levels, strips = Ps[int(20 <= i < 30)]
+            n = strips.A.n
+            x = torch.tensor(ppo.normal(n, 100 * k + i), dtype=dt, device="cuda")
+            jobs[k].append((strips, x, levels.MInvSolve(x.clone()), torch.zeros_like(x)))
+    torch.cuda.synchronize()
+    ctxs = [pp.Context(0), pp.Context(0)]
+    gate, failed = threading.Barrier(2), []
+
+    def work(k):
+        try:
+            gate.wait()
+            for P, x, _, y in jobs[k]:
+                _apply_on(ctxs[k], P, x, y)
+            ctxs[k].sync()
+        except Exception as e:
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    for k in range(2):
+        for i, (_, _, want, got) in enumerate(jobs[k]):
+            assert torch.equal(want, got), (k, i)
+
+
+def test_strips_captured(pp, torch):
+    # an apply captured on a context that has exchange buffers, and on one
+    # that cannot get them inside the capture (level sweeps, the same bits)
+    M = pp.CSRMatrix(*ppo.laplacian(40, 33, 29))
+    P = pp.IncompleteCholesky(M, 1e-2, trsv=5)
+    P.setup()
+    x, y = (torch.zeros(M.n, dtype=torch.float64, device="cuda") for _ in range(2))
+    stream = torch.cuda.Stream()
+    for ready in (True, False):
+        ctx = pp.Context(0)
+        ctx.check(pp._capi.lib().pp_ctx_set_stream(ctx.h, stream.cuda_stream))
+        if ready:
+            _apply_on(ctx, P, x, y)
+            ctx.sync()
+        g = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g, stream=stream, capture_error_mode="thread_local"):
+            _apply_on(ctx, P, x, y)
+        for k in range(4):
+            x.copy_(torch.tensor(ppo.normal(M.n, 7 + k), device="cuda"))
+            want = P.MInvSolve(x.clone())  # on another context, between the replays
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want), (ready, k)
+        del g
