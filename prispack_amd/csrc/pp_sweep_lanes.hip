@@ -357,6 +357,8 @@ struct Exchange {
             if (cw[CW_ABORT]) done = 0xffffffffu;
             have = (uint32_t)__builtin_amdgcn_readfirstlane(done);
         }
+        // the step's gathers are ordinary loads: they stay behind the polls
+        asm volatile("" ::: "memory");
     }
     __device__ void put(uint32_t number, T s) {
         using U = typename SlotBits<T>::U;
