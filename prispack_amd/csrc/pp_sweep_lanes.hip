@@ -822,8 +822,10 @@ void launch_strip_side(pp_ctx *ctx, const StripSweep<T> &L, const StripSide<T> &
     const uint32_t ctl_off = (uint32_t)((L.max_words * sizeof(T) + 15) / 16 * 16);
     const size_t lds = ctl_off + kStripCtl;
     PP_CHECK(lds <= ctx->max_lds && D.data, PP_ERR_INVALID, "strip sweep: storage missing or strip exceeds LDS");
+    bool launched = false;
 #define PP_STRIP(G, S, MODE)                                                                                      \
     if (L.group == G && L.slots == S && D.mode == HostSweep::MODE) {                                              \
+        launched = true;                                                                                          \
         if (lds > 65536)                                                                                          \
             PP_HIP(hipFuncSetAttribute((const void *)k_sweep_strips<T, G, S, HostSweep::MODE>,                    \
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                    \
@@ -841,6 +843,7 @@ void launch_strip_side(pp_ctx *ctx, const StripSweep<T> &L, const StripSide<T> &
     PP_STRIPS(4, 8)
 #undef PP_STRIPS
 #undef PP_STRIP
+    PP_CHECK(launched, PP_ERR_UNSUPPORTED, "strip sweep: no kernel of this step shape and diagonal mode");
     PP_HIP(hipGetLastError());
 }
 
@@ -950,8 +953,10 @@ void launch_lane_sweep(pp_ctx *ctx, const ChunkSet &C, const LaneSweep<T> &L, co
     const size_t lds = (size_t)(C.max_rows + kExtra) * sizeof(T);
     PP_CHECK(C.nchunk && L.data && lds <= ctx->max_lds, PP_ERR_INVALID,
              "chunked sweep: storage missing or chunk exceeds LDS");
+    bool launched = false;
 #define PP_LANES_M(W, G, S, MLO, MUP)                                                                          \
     if (L.mode_lo == HostSweep::MLO && L.mode_up == HostSweep::MUP) {                                          \
+        launched = true;                                                                                       \
         if (lds > 65536)                                                                                       \
             PP_HIP(hipFuncSetAttribute(                                                                        \
                 (const void *)k_sweep_lanes<T, W, G, S, HostSweep::MLO, HostSweep::MUP>,                       \
@@ -973,6 +978,7 @@ void launch_lane_sweep(pp_ctx *ctx, const ChunkSet &C, const LaneSweep<T> &L, co
     PP_LANES(4, 4, 4)
 #undef PP_LANES
 #undef PP_LANES_M
+    PP_CHECK(launched, PP_ERR_UNSUPPORTED, "chunked sweep: no kernel of this step shape and diagonal modes");
     PP_HIP(hipGetLastError());
 }
 template void launch_lane_sweep<double>(pp_ctx *, const ChunkSet &, const LaneSweep<double> &, const double *,
