@@ -364,7 +364,10 @@ typedef struct {
                                (PP_MIXED reduced CG: the steps after an FP32
                                step fell short of its own residual test on the
                                true residual) */
-    uint32_t reserved[6];
+    uint32_t batch_tiles;     /* batched solves: workgroups the inner solves were
+                                 spread over, several a system (0: one workgroup
+                                 per system)                                       */
+    uint32_t reserved[5];
 } pp_solve_report;
 
 void pp_solve_opts_default(pp_solve_opts *o, int solver);
@@ -414,6 +417,14 @@ int pp_csr_outer_on_pattern(pp_ctx *ctx, const pp_csr *A, double scale, const do
 typedef struct pp_batch pp_batch;
 int pp_batch_create(pp_ctx *ctx, uint32_t nsys, const uint32_t *row_off, const uint32_t *rowptr,
                     const uint32_t *colidx, const double *values, pp_batch **out);
+typedef struct pp_batch_info {
+    uint32_t nsys, rows, nnz;
+    uint32_t tiles;            /* workgroups a mixed solve's inner iterations are
+                                  spread over (0: one per system)               */
+    uint32_t device_refactors; /* pp_batch_set_values calls factored on the device */
+    uint32_t reserved[11];
+} pp_batch_info;
+int pp_batch_info_get(const pp_batch *B, pp_batch_info *info);
 /* New values (same patterns): factored on the device, a workgroup per system. */
 int pp_batch_set_values(pp_ctx *ctx, pp_batch *B, const double *values, int on_device);
 /* PP_ORDER_MULTICOLOR: solve every system as P_s A_s P_s^T with its rows

@@ -602,6 +602,12 @@ class BatchedSystems:
         self.ctx.check(_capi.lib().pp_batch_set_ordering(self.ctx.h, self.h, int(ordering)))
         self.ordering = int(ordering)
 
+    def info(self):
+        """Sizes, the tiles of a mixed solve, the value updates factored on the device."""
+        i = _capi.BatchInfo()
+        check(_capi.lib().pp_batch_info_get(self.h, C.byref(i)))
+        return i
+
     def tune(self):
         """Pick the workgroup size (row tile of the SpMV and sweep steps) by timing."""
         bs = C.c_int()

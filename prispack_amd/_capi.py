@@ -62,8 +62,13 @@ class SolveReport(C.Structure):
     _fields_ = [("iters", C.c_int32), ("converged", C.c_int32), ("final_error", C.c_double),
                 ("true_relres", C.c_double), ("outer_iters", C.c_int32), ("inner_iters", C.c_int32),
                 ("solve_ms", C.c_double), ("status", C.c_int32), ("nhist", C.c_int32),
-                ("cg_variant", C.c_int32), ("inner_fp64_steps", C.c_int32),
-                ("reserved", C.c_uint32 * 6)]
+                ("cg_variant", C.c_int32), ("inner_fp64_steps", C.c_int32), ("batch_tiles", C.c_uint32),
+                ("reserved", C.c_uint32 * 5)]
+
+
+class BatchInfo(C.Structure):
+    _fields_ = [("nsys", C.c_uint32), ("rows", C.c_uint32), ("nnz", C.c_uint32), ("tiles", C.c_uint32),
+                ("device_refactors", C.c_uint32), ("reserved", C.c_uint32 * 11)]
 
 
 vp = C.c_void_p
@@ -133,6 +138,7 @@ SIGS = {
                                    C.POINTER(SolveReport)]),
     "pp_csr_outer_on_pattern": (C.c_int, [vp, vp, C.c_double, vp, vp, vp]),
     "pp_batch_create": (C.c_int, [vp, u32, u32p, u32p, u32p, f64p, C.POINTER(vp)]),
+    "pp_batch_info_get": (C.c_int, [vp, C.POINTER(BatchInfo)]),
     "pp_batch_set_values": (C.c_int, [vp, vp, vp, C.c_int]),
     "pp_csr_spmv_bytes": (C.c_int, [vp, C.c_int, C.POINTER(C.c_uint64)]),
     "pp_csr_spmv_variant": (C.c_int, [vp, C.c_int, C.POINTER(C.c_int)]),

@@ -980,6 +980,7 @@ struct pp_batch {
     uint32_t *dvmap = nullptr, *pos = nullptr, *lo_src = nullptr, *dsrc = nullptr, *up_map = nullptr;
     uint32_t lo_nnz = 0;
     int *flag = nullptr;
+    uint32_t device_refactors = 0;
     bool h_v_stale = false;  // h_v predates the values in v64
     // the reduced form's tiles (batch_build_tiles); tile_width 0: none
     int tile_width = 0;
@@ -1405,7 +1406,7 @@ void batch_free_tiles(pp_batch *B) {
 // The tiles of one system: its second-colour rows cut into ntile ranges.
 struct SystemTiles {
     std::vector<Tile> tiles;               // f, h, ka, kb, out relative to the vectors below
-    std::vector<uint32_t> rows, hrow, out; // F's rows and the halo's; halo rows by entry of `slots`; owned rows' exports
+    std::vector<uint32_t> rows;            // F's rows and the halo's
     std::vector<uint32_t> slots;           // halo: the row, to be replaced by its slot; owned: kNoSlot or the slot
     std::vector<uint16_t> loc;
     uint32_t nslot = 0;
@@ -1927,6 +1928,17 @@ int pp_batch_create(pp_ctx *ctx, uint32_t nsys, const uint32_t *row_off, const u
     });
 }
 
+int pp_batch_info_get(const pp_batch *B, pp_batch_info *info) {
+    if (!B || !info) return PP_ERR_INVALID;
+    std::memset(info, 0, sizeof(*info));
+    info->nsys = B->nsys;
+    info->rows = B->ntot;
+    info->nnz = B->nnz;
+    info->tiles = B->tile_width ? B->ntiles : 0;
+    info->device_refactors = B->device_refactors;
+    return PP_OK;
+}
+
 int pp_batch_set_values(pp_ctx *ctx, pp_batch *B, const double *values, int on_device) {
     if (!ctx) return PP_ERR_INVALID;
     return guarded_batch(ctx, [&] {
@@ -1936,7 +1948,10 @@ int pp_batch_set_values(pp_ctx *ctx, pp_batch *B, const double *values, int on_d
         PP_HIP(hipStreamSynchronize(nullptr));  // a device copy may return before it is done
         B->h_v_stale = true;
         if (B->refresh == 0) batch_refresh_build(B);
-        if (B->refresh == 1 && batch_refresh(B)) return;
+        if (B->refresh == 1 && batch_refresh(B)) {
+            ++B->device_refactors;
+            return;
+        }
         // on the host (it also names the first failing system)
         batch_ensure_host_values(B);
         std::vector<float> v32 = to_f32(B->h_v);
@@ -1977,7 +1992,8 @@ static int batch_solve_impl(pp_ctx *ctx, pp_batch *B, const pp_solve_opts *opts,
         BatchArgs a = make_args(B, *opts, perm ? B->bp : b, perm ? B->xp : x);
         PP_HIP(hipEventRecord(ctx->ev0, ctx->stream));
         if (perm) launch_permute(ctx, B->ntot, B->gperm, PP_F64, b, B->bp, true);
-        if (!(mixed && a.red_n0 && B->tile_width && run_tiles(ctx, B, a))) run_batch(ctx, B, mixed, a);
+        const bool tiled = mixed && a.red_n0 && B->tile_width && run_tiles(ctx, B, a);
+        if (!tiled) run_batch(ctx, B, mixed, a);
         if (perm) {
             launch_permute(ctx, B->ntot, B->gperm, PP_F64, B->xp, x, false);
             PP_HIP(hipStreamSynchronize(ctx->stream));
@@ -2005,6 +2021,7 @@ static int batch_solve_impl(pp_ctx *ctx, pp_batch *B, const pp_solve_opts *opts,
             rep->solve_ms = ms;
             rep->status = PP_OK;
             rep->cg_variant = mixed && a.red_n0 ? PP_CG_REDUCED : PP_CG_REFERENCE;
+            rep->batch_tiles = tiled ? B->ntiles : 0;
         }
     });
 }

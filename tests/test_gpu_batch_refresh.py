@@ -60,6 +60,7 @@ def test_refresh_matches_fresh_batch(pp, torch, ordering, on_device):
         new = scaled(systems, 100 * (step + 1))
         v = np.concatenate([A[2] for A in new])
         B.set_values(torch.tensor(v, device="cuda") if on_device else v)
+        assert B.info().device_refactors == step + 1  # not the host's factorization
         F = pp.BatchedSystems(new, ordering=ordering)
         for (i0, x0), (i1, x1) in zip(solves(torch, B, b), solves(torch, F, b)):
             assert np.array_equal(i0, i1) and torch.equal(x0, x1)
@@ -69,6 +70,22 @@ def test_refresh_matches_fresh_batch(pp, torch, ordering, on_device):
     if ordering == 1:
         for (i0, x0), (i1, x1) in zip(solves(torch, B, b), solves(torch, F, b)):
             assert np.array_equal(i0, i1) and torch.equal(x0, x1)
+
+
+def test_unsorted_rows_are_factored_on_the_host(pp, torch):
+    def reversed_rows(A):
+        rp, ci, v = A
+        back = np.concatenate([np.arange(rp[i], rp[i + 1])[::-1] for i in range(len(rp) - 1)])
+        return rp, ci[back], v[back]
+
+    systems = [reversed_rows(ppo.laplacian(9, 8, 1)), ppo.laplacian(7, 6, 1)]
+    B = pp.BatchedSystems(systems)
+    new = scaled(systems, 300)
+    b = torch.ones(B.n, dtype=torch.float64, device="cuda")
+    B.set_values(torch.tensor(np.concatenate([A[2] for A in new]), device="cuda"))
+    assert B.info().device_refactors == 0
+    for (i0, x0), (i1, x1) in zip(solves(torch, B, b), solves(torch, pp.BatchedSystems(new), b)):
+        assert np.array_equal(i0, i1) and torch.equal(x0, x1)
 
 
 def test_refresh_reports_a_failing_pivot(pp, torch):
@@ -84,7 +101,8 @@ def test_refresh_reports_a_failing_pivot(pp, torch):
         bad[k:int(B.rp[r0 + 18])] *= np.where(B.ci[k:int(B.rp[r0 + 18])] == r0 + 17, -1.0, 1.0)
         with pytest.raises(PrisPackError) as e:
             B.set_values(torch.tensor(bad, device="cuda"))
-        assert "system 1" in str(e.value)
+        assert "system 1" in str(e.value) and B.info().device_refactors == 0
         B.set_values(torch.tensor(B.v, device="cuda"))  # and good values work again
+        assert B.info().device_refactors == 1
         for (i0, x0), (i1, x1) in zip(first, solves(torch, B, b)):
             assert np.array_equal(i0, i1) and torch.equal(x0, x1)

@@ -53,6 +53,11 @@ def test_tiled_mixed_solve(pp, torch, name):
     it64 = B.solve(b, x64, precision="fp64", tol=1e-8)
     it = B.solve(b, x, precision="mixed", tol=1e-8)
     assert B.report.converged and B.report.true_relres < 1e-8 and B.report.cg_variant == 3
+    # the path under test ran: every system a tile at least
+    if name == "halo_too_wide":
+        assert B.info().tiles == B.report.batch_tiles == 0
+    else:
+        assert B.info().tiles == B.report.batch_tiles >= len(systems)
     assert np.array_equal(it, B.solve(b, y, precision="mixed", tol=1e-8)) and torch.equal(x, y)
     for s in range(len(systems)):
         lo, hi = int(B.row_off[s]), int(B.row_off[s + 1])
@@ -72,7 +77,7 @@ def test_tiled_solve_stops_at_its_iteration_limit(pp, torch):
     b = torch.ones(B.n, dtype=torch.float64, device="cuda")
     x = torch.zeros_like(b)
     it = B.solve(b, x, precision="mixed", tol=1e-8, maxit=25)
-    assert not B.report.converged and it.max() <= 25
+    assert not B.report.converged and it.max() <= 25 and B.report.batch_tiles > 0
     # a zero right-hand side needs no iteration
     b[:B.row_off[1]] = 0.0
     it = B.solve(b, x, precision="mixed", tol=1e-8)
