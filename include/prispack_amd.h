@@ -52,6 +52,12 @@ int pp_ctx_create(int device, pp_ctx **out);
  * NULL restores the context's own stream. */
 int pp_ctx_set_stream(pp_ctx *ctx, void *hip_stream);
 void *pp_ctx_stream(pp_ctx *ctx);
+/* The longest a workgroup waits for another one's value (the sync-free and the
+ * strip sweeps, the tiles of a batched solve, the device colouring) before it
+ * gives up: the call then fails with PP_ERR_HIP, or falls back where it can.
+ * Default 2 s; 0: give up at the first look that finds nothing.  For kernels
+ * launched (or captured) from now on. */
+int pp_ctx_set_wait_limit(pp_ctx *ctx, double seconds);
 int pp_ctx_sync(pp_ctx *ctx);
 void pp_ctx_destroy(pp_ctx *ctx);
 const char *pp_last_error(const pp_ctx *ctx);

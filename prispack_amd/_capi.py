@@ -82,6 +82,7 @@ SIGS = {
     "pp_ctx_create": (C.c_int, [C.c_int, C.POINTER(vp)]),
     "pp_ctx_set_stream": (C.c_int, [vp, vp]),
     "pp_ctx_stream": (vp, [vp]),
+    "pp_ctx_set_wait_limit": (C.c_int, [vp, C.c_double]),
     "pp_ctx_sync": (C.c_int, [vp]),
     "pp_ctx_destroy": (None, [vp]),
     "pp_last_error": (C.c_char_p, [vp]),

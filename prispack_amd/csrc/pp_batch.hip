@@ -630,7 +630,6 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_cg(TileArgs a) {
     const double tol = a.want[t.sys], normb = a.rin_norm[t.sys];
     const uint32_t maxit = a.left[t.sys];
     const bool shared = t.ntile > 1;
-    const long long t0 = shared ? wall_clock64() : 0;
     uint32_t m = maxit;
     double gold = 0.0, aold = 1.0;
     bool first = true;
@@ -692,6 +691,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_cg(TileArgs a) {
                 const uint32_t cnt = min(nw - w0, kWords);
                 bool wait_p = tid < cnt;
                 const unsigned long long *src = xp + 6 * (size_t)t.tile0 + w0 + tid;
+                WaitClock clock;
                 for (uint32_t iter = 1;; ++iter) {
                     bool more = false;
                     const unsigned long long v = wait_p ? get_word(src) : 0;
@@ -712,8 +712,8 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_cg(TileArgs a) {
                         more = more || wait_h[k];
                     }
                     if (!__any(more)) break;
-                    if ((iter & 63) == 0 &&
-                        (wall_clock64() - t0 > a.deadline ||
+                    if (WaitClock::due(iter, a.deadline) &&
+                        (clock.expired(a.deadline) ||
                          __hip_atomic_load(a.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
                         atomicOr(a.abort, 1);
                         stop = 1;

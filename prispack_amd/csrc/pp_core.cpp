@@ -572,6 +572,7 @@ int pp_ctx_create(int device, pp_ctx **out) {
         if (hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, device) != hipSuccess ||
             clock_khz <= 0)
             clock_khz = 100000;
+        c->clock_hz = clock_khz * 1e3;
         c->spin_deadline = (long long)clock_khz * 1000LL * 2;  // a dependency wait may last 2 s
         c->red.partials = dalloc<double>((size_t)S_COUNT * kMaxPartials);
         c->scal = dalloc<double>(S_COUNT);
@@ -601,6 +602,13 @@ int pp_ctx_set_stream(pp_ctx *ctx, void *s) {
 }
 
 void *pp_ctx_stream(pp_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }
+
+int pp_ctx_set_wait_limit(pp_ctx *ctx, double seconds) {
+    return guarded(ctx, [&] {
+        PP_CHECK(seconds >= 0 && seconds <= 86400, PP_ERR_INVALID, "wait limit must be 0 to 86400 seconds");
+        ctx->spin_deadline = (long long)(seconds * ctx->clock_hz);
+    });
+}
 
 int pp_ctx_sync(pp_ctx *ctx) {
     return guarded(ctx, [&] { PP_HIP(hipStreamSynchronize(ctx->stream)); });

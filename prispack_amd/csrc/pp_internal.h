@@ -168,7 +168,8 @@ struct pp_ctx {
         uint32_t n = 0;
     } strip_slots[2][2];
     std::vector<void *> old_strip_slots;
-    long long spin_deadline = 0;   // wall_clock64 ticks a sync-free wait may last
+    double clock_hz = 1e8;         // of wall_clock64
+    long long spin_deadline = 0;   // wall_clock64 ticks a wait may last (pp_ctx_set_wait_limit)
     // while set (StopScope), SpMV / dot / GEMV / convert kernels return at
     // once when the word is non-zero, like the sweeps and the PCG kernels
     const int *stop_word = nullptr;
@@ -769,6 +770,20 @@ bool launch_strip_sweeps(pp_ctx *ctx, const StripSweep<T> &L, const T *x, T *y);
 template <class T>
 bool strip_reserve(pp_ctx *ctx, const StripSweep<T> &L);
 void precond_reserve(pp_ctx *ctx, const pp_precond *M);
+
+// The bound of one wait.  due(): polls of it (from 1) have come up empty, is
+// it time to look at the clock (every 64 polls; at each one with a deadline of
+// 0, which gives up at the first empty poll).  expired(): the deadline has
+// passed since this wait's first look; the kernel's run time does not count.
+struct WaitClock {
+    long long t0 = 0;
+    __device__ static bool due(uint32_t polls, long long deadline) { return (polls & (deadline ? 63u : 0u)) == 0; }
+    __device__ bool expired(long long deadline) {
+        const long long now = wall_clock64();
+        if (!t0) t0 = now;
+        return now - t0 >= deadline;
+    }
+};
 void ml_reserve(pp_ctx *ctx, const pp_precond *M);
 // The same sweeps from the level-ordered storage (DevChunkSweep), one
 // wavefront computing the levels while the rest of the workgroup stages

@@ -311,8 +311,9 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
 // backward sweep's is emptied by the forward sweep before it.
 // A strip waits only for strips before it in its sweep's direction, whose
 // workgroups are dispatched before its own, so the first unfinished strip
-// always proceeds; a wait past the deadline sets C_SPIN, and every wavefront
-// runs to its end (the rows become NaN).
+// always proceeds; a wait past the deadline (nothing new among the 256 imports
+// a wavefront polls) sets C_SPIN, and every wavefront runs to its end (the rows
+// become NaN).
 // ---------------------------------------------------------------------------
 constexpr int kImport = kLaneThreads / 64 - 1, kBatch = 4;
 constexpr uint32_t kStripCtl = 32;  // bytes of LDS: per import wavefront the imports it has seen; the abort word
@@ -419,7 +420,6 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
         // turns; cw[f]: the imports below it are in LDS, as far as wavefront
         // f is concerned
         const uint32_t f = wave - 1;
-        const long long t0 = wall_clock64();
         bool abort = false;
         const auto slot_of = [&](uint32_t i) { return imp[h.imp + min(i, h.nimp - 1)]; };
         uint32_t to[kBatch] = {};
@@ -436,6 +436,8 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
                 slot[b] = reinterpret_cast<U *>(slots) + to[b];
                 to[b] = slot_of(i0 + (kImport * kBatch + b) * 64 + lane);  // the next batch's
             }
+            WaitClock clock;
+            bool got = false;
             for (uint32_t iter = 1;; ++iter) {
                 U v[kBatch];
 #pragma unroll
@@ -447,6 +449,7 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
                     if (v[b] != kEmpty) {
                         xs[nr + 1 + i0 + b * 64 + lane] = __builtin_bit_cast(T, v[b]);
                         wait[b] = false;
+                        got = true;
                     }
                     const unsigned long long m = __ballot(wait[b]);
                     if (m) seen = b * 64 + __builtin_ctzll(m);
@@ -455,8 +458,12 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
                 // all of them: the next one to see is the next batch's first
                 cw[f] = i0 + (seen < kBatch * 64 ? seen : kImport * kBatch * 64);
                 if (seen == kBatch * 64) break;
-                if ((iter & 63) == 0 && (wall_clock64() - t0 > deadline ||
-                                         __hip_atomic_load(&ctl[C_SPIN], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                if (!WaitClock::due(iter, deadline)) continue;
+                if (__any(got)) {  // another wait from here on
+                    got = false;
+                    clock = WaitClock();
+                } else if (clock.expired(deadline) ||
+                           __hip_atomic_load(&ctl[C_SPIN], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                     atomicOr(&ctl[C_SPIN], 1);
                     cw[CW_ABORT] = 1;
                     abort = true;
