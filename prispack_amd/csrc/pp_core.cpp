@@ -150,6 +150,20 @@ void read_ctl(pp_ctx *ctx, int *out) {
     std::memcpy(out, ctx->pinned_ctl, C_COUNT * sizeof(int));
 }
 
+void throw_given_up(pp_ctx *ctx) {
+    volatile int *late = ctx->late_host;
+    if (!*late) return;
+    *late = 0;
+    throw Error(PP_ERR_HIP, "a triangular sweep timed out waiting for a dependency; its result holds NaN");
+}
+
+void check_spin(pp_ctx *ctx, const int *ctl) {
+    if (!ctl[C_SPIN]) return;
+    (void)hipStreamSynchronize(ctx->stream);  // what is queued behind the sweep neither reports later nor publishes
+    throw_given_up(ctx);
+    throw Error(PP_ERR_HIP, "a triangular sweep timed out waiting for a dependency");
+}
+
 void Graph::reset() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (g) (void)hipGraphDestroy(g);
@@ -581,9 +595,12 @@ int pp_ctx_create(int device, pp_ctx **out) {
         PP_HIP(hipMemset(c->ctl, 0, C_COUNT * sizeof(int)));
         PP_HIP(hipHostMalloc((void **)&c->pinned, 640 * sizeof(double), hipHostMallocDefault));
         PP_HIP(hipHostMalloc((void **)&c->pinned_ctl, 64 * sizeof(int), hipHostMallocDefault));
-        PP_HIP(hipHostMalloc((void **)&c->ring_host, pp_ctx::kRing * C_COUNT * sizeof(int),
+        PP_HIP(hipHostMalloc((void **)&c->ring_host, (pp_ctx::kRing + 1) * C_COUNT * sizeof(int),
                              hipHostMallocMapped | hipHostMallocCoherent));
         PP_HIP(hipHostGetDevicePointer((void **)&c->ring_dev, c->ring_host, 0));
+        c->late_host = c->ring_host + pp_ctx::kRing * C_COUNT;
+        c->late_dev = c->ring_dev + pp_ctx::kRing * C_COUNT;
+        *c->late_host = 0;
         PP_HIP(hipEventCreate(&c->ev0));
         PP_HIP(hipEventCreate(&c->ev1));
         ensure_hist(c.get(), 4096);
@@ -611,7 +628,10 @@ int pp_ctx_set_wait_limit(pp_ctx *ctx, double seconds) {
 }
 
 int pp_ctx_sync(pp_ctx *ctx) {
-    return guarded(ctx, [&] { PP_HIP(hipStreamSynchronize(ctx->stream)); });
+    return guarded(ctx, [&] {
+        PP_HIP(hipStreamSynchronize(ctx->stream));
+        throw_given_up(ctx);
+    });
 }
 
 void pp_ctx_destroy(pp_ctx *ctx) {
@@ -659,6 +679,7 @@ int pp_memcpy_d2h(pp_ctx *ctx, void *dst, const void *src, size_t bytes) {
     return guarded(ctx, [&] {
         PP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
         PP_HIP(hipStreamSynchronize(ctx->stream));
+        throw_given_up(ctx);
     });
 }
 

@@ -146,6 +146,9 @@ struct pp_ctx {
     int *pinned_ctl = nullptr;    // pinned host mirror of ctl
     int *ring_host = nullptr;     // mapped pinned slots the PCG bodies publish ctl into
     int *ring_dev = nullptr;      // the same memory as the device sees it
+    // behind the ring, mapped like it: set by a sweep that gave up waiting, for
+    // calls that return before the sweep has run (throw_given_up)
+    int *late_host = nullptr, *late_dev = nullptr;
     std::vector<double> last_hist;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     static constexpr int kRing = 4;      // publication slots of ring_host
@@ -770,6 +773,18 @@ bool launch_strip_sweeps(pp_ctx *ctx, const StripSweep<T> &L, const T *x, T *y);
 template <class T>
 bool strip_reserve(pp_ctx *ctx, const StripSweep<T> &L);
 void precond_reserve(pp_ctx *ctx, const pp_precond *M);
+
+// A sweep gave up waiting: C_SPIN for the launches behind it and the solves'
+// checks, the host's word for calls that return before it has run.
+__device__ inline void give_up(int *ctl, int *late) {
+    atomicOr(&ctl[C_SPIN], 1);
+    __hip_atomic_store(late, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// The host's side, on a stream that has been waited for: an error if a sweep
+// has given up since the last look.  check_spin: the same for a solve that read
+// the control words ctl (it waits for the stream first).
+void throw_given_up(pp_ctx *ctx);
+void check_spin(pp_ctx *ctx, const int *ctl);
 
 // The bound of one wait.  due(): polls of it (from 1) have come up empty, is
 // it time to look at the clock (every 64 polls; at each one with a deadline of

@@ -1253,7 +1253,7 @@ __global__ __launch_bounds__(256) void k_sweep_syncfree(const uint32_t *__restri
                                                         const uint32_t *__restrict__ ci,
                                                         const T *__restrict__ val, const T *__restrict__ diag,
                                                         int mode, const T *__restrict__ b, T *y, uint32_t n,
-                                                        long long deadline, int *ctl) {
+                                                        long long deadline, int *ctl, int *late) {
 #pragma clang fp contract(off)
     using U = typename SentinelBits<T>::U;
     constexpr U kSent = SentinelBits<T>::value;
@@ -1289,7 +1289,7 @@ __global__ __launch_bounds__(256) void k_sweep_syncfree(const uint32_t *__restri
         }
         if (__all(done)) break;
         if (wall_clock64() - t0 > deadline) {
-            if (!done) atomicOr(&ctl[C_SPIN], 1);
+            if (!done) give_up(ctl, late);
             break;
         }
         // another wave already gave up: its dependents would wait in vain
@@ -1305,7 +1305,7 @@ void launch_sweep_syncfree(pp_ctx *ctx, const DevSweep<T> &s, int mode, const T 
     const unsigned g = (s.n + kBlock - 1) / kBlock;
     k_fill_sentinel<T><<<grid_for(ctx, s.n), kBlock, 0, ctx->stream>>>(s.n, y, ctx->ctl);
     k_sweep_syncfree<T><<<g, kBlock, 0, ctx->stream>>>(s.perm, s.rp, s.ci, s.val, s.diag, mode, b, y, s.n,
-                                                        ctx->spin_deadline, ctx->ctl);
+                                                        ctx->spin_deadline, ctx->ctl, ctx->late_dev);
     PP_HIP(hipGetLastError());
 }
 template void launch_sweep_syncfree<double>(pp_ctx *, const DevSweep<double> &, int, const double *, double *);

@@ -779,6 +779,11 @@ void ml_setup(pp_ctx *ctx, pp_precond *M) {
     auto *S = new MlState;
     M->multilevel = S;
     try {
+        // a sweep below that gives up is this set-up's error; an earlier one's word
+        // would end the sweeps below at once
+        PP_HIP(hipStreamSynchronize(ctx->stream));
+        throw_given_up(ctx);
+        launch_fill_zero(ctx, ctx->ctl, C_COUNT * sizeof(int));
         S->symmetric = spd;
         S->n = A.n;
         const uint32_t nlev = M->opts.levels ? M->opts.levels : 3;
@@ -845,8 +850,12 @@ void ml_setup(pp_ctx *ctx, pp_precond *M) {
         }
         M->low64.nlev = nlev;
         M->up64.nlev = nlev;
+        PP_HIP(hipStreamSynchronize(ctx->stream));
+        throw_given_up(ctx);
     } catch (...) {
+        (void)hipStreamSynchronize(ctx->stream);
         ml_free(M);
+        throw_given_up(ctx);  // the cause of whatever the NaN led to
         throw;
     }
 }

@@ -149,7 +149,7 @@ void drive_bodies(pp_ctx *ctx, Body &body, bool use_graph, uint64_t max_replays,
     bool run = true, published = false;
     if (check_first) {
         read_ctl(ctx, ctl);
-        PP_CHECK(!ctl[C_SPIN], PP_ERR_HIP, "sync-free triangular sweep timed out waiting for a dependency");
+        check_spin(ctx, ctl);
         run = !ctl[C_STOP];
     }
     if (run) {
@@ -158,7 +158,7 @@ void drive_bodies(pp_ctx *ctx, Body &body, bool use_graph, uint64_t max_replays,
             if (!wait_published(checked)) break;  // read the words synchronously below
             for (int i = 0; i < C_COUNT; ++i) ctl[i] = slots[(checked % R) * C_COUNT + i];
             ++checked;
-            PP_CHECK(!ctl[C_SPIN], PP_ERR_HIP, "sync-free triangular sweep timed out waiting for a dependency");
+            check_spin(ctx, ctl);
             if (ctl[C_STOP]) published = true;  // bodies after the stop leave the words as they are
             if (ctl[C_STOP] || checked >= max_replays) break;
         }
@@ -744,7 +744,7 @@ PcgResult gmres_device(pp_ctx *ctx, pp_csr *A, pp_precond *M, const pp_solve_opt
         {
             int ctl[C_COUNT];
             read_ctl(ctx, ctl);
-            PP_CHECK(!ctl[C_SPIN], PP_ERR_HIP, "sync-free triangular sweep timed out waiting for a dependency");
+            check_spin(ctx, ctl);
         }
         nrec += (uint32_t)misc[GM_NREC];
         m = (uint32_t)misc[GM_M];
@@ -784,7 +784,7 @@ PcgResult gmres_device(pp_ctx *ctx, pp_csr *A, pp_precond *M, const pp_solve_opt
     {
         int ctl[C_COUNT];
         read_ctl(ctx, ctl);
-        PP_CHECK(!ctl[C_SPIN], PP_ERR_HIP, "sync-free triangular sweep timed out waiting for a dependency");
+        check_spin(ctx, ctl);
     }
     res.conv = conv;
     res.iters = k * (int32_t)mm + (int32_t)m;  // GMRES.cpp:218

@@ -381,7 +381,8 @@ __global__ void k_slots_empty(uint32_t n, T *slots) {
 template <class T, int G, int S, int MODE>
 __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_sweep_strips(
     const StripHead *__restrict__ heads, const char *data, const uint32_t *__restrict__ imp, T *slots,
-    uint32_t other_n, T *other, uint32_t ctl_off, const T *x, T *y, long long deadline, int *ctl, const int *stop) {
+    uint32_t other_n, T *other, uint32_t ctl_off, const T *x, T *y, long long deadline, int *ctl, int *late,
+    const int *stop) {
     using U = typename SlotBits<T>::U;
     constexpr U kEmpty = SlotBits<T>::empty;
     extern __shared__ unsigned char lds_raw[];
@@ -464,7 +465,7 @@ __global__ __launch_bounds__(kLaneThreads) __attribute__((amdgpu_waves_per_eu(1,
                     clock = WaitClock();
                 } else if (clock.expired(deadline) ||
                            __hip_atomic_load(&ctl[C_SPIN], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                    atomicOr(&ctl[C_SPIN], 1);
+                    give_up(ctl, late);
                     cw[CW_ABORT] = 1;
                     abort = true;
                     break;
@@ -838,7 +839,7 @@ void launch_strip_side(pp_ctx *ctx, const StripSweep<T> &L, const StripSide<T> &
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                    \
         k_sweep_strips<T, G, S, HostSweep::MODE><<<L.nstrip, kLaneThreads, lds, ctx->stream>>>(                   \
             (const StripHead *)D.head, (const char *)D.data, D.imp, slots, on, other, ctl_off, x, y,             \
-            ctx->spin_deadline, ctx->ctl, ctx->stop_word);                                                        \
+            ctx->spin_deadline, ctx->ctl, ctx->late_dev, ctx->stop_word);                                                      \
     }
 #define PP_STRIPS(G, S)          \
     PP_STRIP(G, S, DIVIDE)       \

@@ -99,3 +99,78 @@ def test_batch_falls_back(torch, ctx):
         u, bs = (t[int(B.row_off[s]):int(B.row_off[s + 1])].cpu().numpy() for t in (x[1], b))
         # the solve's test and the rounding of a second FP64 residual
         assert np.linalg.norm(bs - ppo.spmv(A, u)) <= 1.01e-8 * np.linalg.norm(bs), s
+
+
+def test_strip_apply_returns_before_the_sweep(torch, ctx):
+    # the call is asynchronous, as with the level sweeps; a sweep that gives up
+    # afterwards is reported by the next call that waits, once
+    import ctypes
+    import prispack_amd as pp
+    from prispack_amd import _capi
+    L = _capi.lib()
+    M = pp.CSRMatrix(*ppo.laplacian(40, 33, 29), ctx=ctx)
+    P = pp.IncompleteCholesky(M, 1e-2, trsv=5)
+    P.setup()
+    x = torch.tensor(ppo.normal(M.n, 3), device="cuda")
+    want, y = P.MInvSolve(x.clone()), torch.zeros_like(x)
+    px, py = (ctypes.c_void_p(t.data_ptr()) for t in (x, y))
+    stream = torch.cuda.Stream()
+    w = torch.ones(8192, 8192, device="cuda")
+    torch.cuda.synchronize()
+    ctx.check(L.pp_ctx_set_stream(ctx.h, stream.cuda_stream))
+    try:
+        for seconds in (0.0, 2.0):
+            limit(ctx, seconds)
+            with torch.cuda.stream(stream):
+                for _ in range(20):
+                    v = w @ w
+            ctx.check(L.pp_precond_apply(ctx.h, P.h, 0, px, py))
+            assert not stream.query()
+            if seconds == 0.0:
+                with pytest.raises(pp.PrisPackError) as e:
+                    ctx.sync()
+                assert e.value.status == 2 and bool(torch.isnan(y).any())
+            ctx.sync()
+        assert torch.equal(y, want)
+    finally:
+        limit(ctx, 2.0)
+        torch.cuda.synchronize()
+        ctx.check(L.pp_ctx_set_stream(ctx.h, None))
+
+
+@pytest.mark.parametrize("kind", ["AMSED", "GMSLR"])
+def test_multilevel_over_strips(torch, ctx, kind):
+    # the subdomain factors wait, not the preconditioner applied: the apply and
+    # the set-up fail all the same
+    import ctypes
+    import prispack_amd as pp
+    A = ppo.laplacian(24, 22, 20) if kind == "AMSED" else ppo.upwind(24, 22, 20, 20.0, 10.0, 5.0)
+    M = pp.CSRMatrix(*A, ctx=ctx)
+    make = lambda trsv: getattr(pp, kind)(M, levels=2, ndom=4, rank=4, trsv=trsv)
+    P1, P = make(1), make(5)
+    P1.setup()
+    P.setup()
+    assert P.info().trsv == 5
+    x = torch.tensor(ppo.normal(M.n, 3), device="cuda")
+    want = P1.MInvSolve(x.clone())
+    for _ in range(2):
+        limit(ctx, 0.0)
+        with pytest.raises(pp.PrisPackError) as e:
+            P.MInvSolve(x.clone())
+        assert e.value.status == 2
+        with pytest.raises(pp.PrisPackError) as e:
+            make(5).setup()
+        assert e.value.status == 2
+        limit(ctx, 2.0)
+        for _ in range(2):
+            assert torch.equal(P.MInvSolve(x.clone()), want)  # the same set-up, bit for bit
+    Q = make(5)  # a set-up behind a failed apply that nobody waited for
+    limit(ctx, 0.0)
+    y = torch.zeros_like(x)
+    torch.cuda.synchronize()
+    ctx.check(pp._capi.lib().pp_precond_apply(ctx.h, P.h, 0, *(ctypes.c_void_p(t.data_ptr()) for t in (x, y))))
+    limit(ctx, 2.0)
+    with pytest.raises(pp.PrisPackError):
+        ctx.sync()
+    Q.setup()
+    assert torch.equal(Q.MInvSolve(x.clone()), want)
