@@ -1976,8 +1976,9 @@ int pp_batch_set_ordering(pp_ctx *ctx, pp_batch *B, int ordering) {
             B->pci = upload(B->h_pci);
             B->bp = dalloc<double>(B->ntot);
             B->xp = dalloc<double>(B->ntot);
-            batch_upload_permuted_values(B);
         }
+        // also where the order had been used before: the values may have come since
+        if (ordering == PP_ORDER_MULTICOLOR) batch_upload_permuted_values(B);
         batch_factor(B);
     });
 }

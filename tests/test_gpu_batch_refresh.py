@@ -72,6 +72,22 @@ def test_refresh_matches_fresh_batch(pp, torch, ordering, on_device):
             assert np.array_equal(i0, i1) and torch.equal(x0, x1)
 
 
+def test_values_set_under_the_other_order(pp, torch):
+    # the permuted copy of an order used before follows values set under another
+    systems = [ppo.vardiff2d(s, np.exp(ppo.normal(s * s, 40 + s))) for s in (7, 32)]
+    new = scaled(systems, 500)
+    b = torch.tensor(np.concatenate([ppo.uniform(len(A[0]) - 1, 5 + s) for s, A in enumerate(systems)]), device="cuda")
+    for on_device in (False, True):
+        B = pp.BatchedSystems(systems, ordering=1)
+        B.set_ordering(0)
+        v = np.concatenate([A[2] for A in new])
+        B.set_values(torch.tensor(v, device="cuda") if on_device else v)
+        B.set_ordering(1)
+        F = pp.BatchedSystems(new, ordering=1)
+        for (i0, x0), (i1, x1) in zip(solves(torch, B, b), solves(torch, F, b)):
+            assert np.array_equal(i0, i1) and torch.equal(x0, x1)
+
+
 def test_unsorted_rows_are_factored_on_the_host(pp, torch):
     def reversed_rows(A):
         rp, ci, v = A
