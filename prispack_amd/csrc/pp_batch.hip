@@ -981,6 +981,10 @@ struct pp_batch {
     uint32_t lo_nnz = 0;
     int *flag = nullptr;
     uint32_t device_refactors = 0;
+    // the values before the last ones set, an array swapped with v64; after
+    // values whose factorization failed: those of the factor still in use
+    double *v64_before = nullptr;
+    bool factor_before = false;
     bool h_v_stale = false;  // h_v predates the values in v64
     // the reduced form's tiles (batch_build_tiles); tile_width 0: none
     int tile_width = 0;
@@ -1634,6 +1638,7 @@ void batch_factor(pp_batch *B) {
         append_parts(up, ups[s]);
         B->max_levels = std::max(B->max_levels, nlev[s]);
     }
+    B->factor_before = false;
     upload_batch_sweep(lo, B->lo);
     upload_batch_sweep(up, B->up);
     B->lo_nnz = (uint32_t)lo.ci.size();
@@ -1689,18 +1694,26 @@ void batch_refresh_build(pp_batch *B) {
     B->refresh = 1;
 }
 
-// Factors v64's values on the device; false: a pivot is not positive.
-bool batch_refresh(pp_batch *B) {
+// the copies the solves multiply with, from the values v
+void batch_refresh_values(pp_batch *B, const double *v) {
+    pp_ctx *ctx = B->ctx;
+    const unsigned g = std::max(1u, std::min<uint32_t>((B->nnz + 1023) / 1024, 16384u));
+    k_batch_values<<<g, 256, 0, ctx->stream>>>(B->nnz, nullptr, v, nullptr, B->v32);
+    if (B->ordering == PP_ORDER_MULTICOLOR)
+        k_batch_values<<<g, 256, 0, ctx->stream>>>(B->nnz, B->dvmap, v, B->pv64, B->pv32);
+    PP_HIP(hipGetLastError());
+}
+
+// Factors the values v on the device; false: a pivot is not positive.
+bool batch_refresh(pp_batch *B, const double *v) {
     pp_ctx *ctx = B->ctx;
     const bool perm = B->ordering == PP_ORDER_MULTICOLOR;
-    const unsigned g = std::max(1u, std::min<uint32_t>((B->nnz + 1023) / 1024, 16384u));
-    k_batch_values<<<g, 256, 0, ctx->stream>>>(B->nnz, nullptr, B->v64, nullptr, B->v32);
-    if (perm) k_batch_values<<<g, 256, 0, ctx->stream>>>(B->nnz, B->dvmap, B->v64, B->pv64, B->pv32);
+    batch_refresh_values(B, v);
     RefreshArgs a;
     a.roff = B->roff;
     a.rp = perm ? B->prp : B->rp;
     a.ci = perm ? B->pci : B->ci;
-    a.av = perm ? B->pv64 : B->v64;
+    a.av = perm ? B->pv64 : v;
     a.lo = B->lo;
     a.up = B->up;
     a.pos = B->pos;
@@ -1853,7 +1866,7 @@ bool run_tiles(pp_ctx *ctx, pp_batch *B, const BatchArgs &a) {
 
 void batch_free(pp_batch *B) {
     batch_free_tiles(B);
-    dfree(B->roff); dfree(B->rp); dfree(B->ci); dfree(B->v64); dfree(B->v32);
+    dfree(B->roff); dfree(B->rp); dfree(B->ci); dfree(B->v64); dfree(B->v32); dfree(B->v64_before);
     B->lo.free_all();
     B->up.free_all();
     dfree(B->r64); dfree(B->rr64); dfree(B->w64); dfree(B->d64); dfree(B->p64);
@@ -1943,14 +1956,27 @@ int pp_batch_set_values(pp_ctx *ctx, pp_batch *B, const double *values, int on_d
     if (!ctx) return PP_ERR_INVALID;
     return guarded_batch(ctx, [&] {
         PP_CHECK(B && values, PP_ERR_INVALID, "NULL argument");
+        if (B->refresh == 0) batch_refresh_build(B);
+        // the factorization on the device overwrites the factor: the values it
+        // came from are kept until it has succeeded
+        if (B->refresh == 1 && !B->factor_before) {
+            if (!B->v64_before) B->v64_before = dalloc<double>(B->nnz);
+            std::swap(B->v64, B->v64_before);
+        }
         PP_HIP(hipMemcpy(B->v64, values, B->nnz * sizeof(double),
                          on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice));
         PP_HIP(hipStreamSynchronize(nullptr));  // a device copy may return before it is done
         B->h_v_stale = true;
-        if (B->refresh == 0) batch_refresh_build(B);
-        if (B->refresh == 1 && batch_refresh(B)) {
-            ++B->device_refactors;
-            return;
+        if (B->refresh == 1) {
+            B->factor_before = !batch_refresh(B, B->v64);
+            if (!B->factor_before) {
+                ++B->device_refactors;
+                return;
+            }
+            // the factor in use comes back, as the host path leaves it where it fails
+            batch_refresh(B, B->v64_before);
+            batch_refresh_values(B, B->v64);
+            PP_HIP(hipStreamSynchronize(B->ctx->stream));
         }
         // on the host (it also names the first failing system)
         batch_ensure_host_values(B);

@@ -72,6 +72,38 @@ def test_refresh_matches_fresh_batch(pp, torch, ordering, on_device):
             assert np.array_equal(i0, i1) and torch.equal(x0, x1)
 
 
+@pytest.mark.parametrize("ordering", [0, 1])
+def test_failing_pivot_keeps_the_factor_in_use(pp, torch, ordering):
+    # as after a failed factorization on the host: the new values, the factor of
+    # the ones before.  Three FP64 iterations against the oracle's with just that.
+    from mc_order import greedy_order, permute
+    from prispack_amd import PrisPackError
+    systems = [ppo.vardiff2d(s, np.exp(ppo.normal(s * s, 40 + s))) for s in (9, 33, 12)]
+    B = pp.BatchedSystems(systems, ordering=ordering)
+    b = torch.tensor(np.concatenate([ppo.uniform(len(A[0]) - 1, 5 + s) for s, A in enumerate(systems)]), device="cuda")
+    for step in range(2):
+        good = scaled(systems, 700) if step else systems
+        if step:
+            B.set_values(np.concatenate([A[2] for A in good]))
+        for fail in range(2):  # twice: the factor stays that of the good values
+            bad = scaled(systems, 800 + fail)
+            rp, ci, v = bad[1]
+            v[np.flatnonzero((ci == 77) & (np.repeat(np.arange(len(rp) - 1), np.diff(rp.astype(int))) == 77))] *= -1.0
+            with pytest.raises(PrisPackError) as e:
+                B.set_values(torch.tensor(np.concatenate([A[2] for A in bad]), device="cuda"))
+            assert e.value.status == 3 and "system 1" in str(e.value)
+            x = torch.zeros_like(b)
+            B.solve(b, x, precision="fp64", tol=1e-300, maxit=3)
+            for s in range(len(systems)):
+                lo, hi = int(B.row_off[s]), int(B.row_off[s + 1])
+                order = greedy_order(systems[s])[0] if ordering else np.arange(hi - lo)
+                F = ppo.Prec(permute(good[s], order), "ic0")
+                w = ppo.cg(permute(bad[s], order), b[lo:hi].cpu().numpy()[order], F, tol=1e-300, maxit=3)["x"]
+                got = x[lo:hi].cpu().numpy()[order]
+                # three steps' rounding: a few eps, magnified by how far alpha and beta lie from one
+                assert np.linalg.norm(got - w) <= 1e-11 * np.linalg.norm(w), (step, fail, s)
+
+
 def test_values_set_under_the_other_order(pp, torch):
     # the permuted copy of an order used before follows values set under another
     systems = [ppo.vardiff2d(s, np.exp(ppo.normal(s * s, 40 + s))) for s in (7, 32)]
