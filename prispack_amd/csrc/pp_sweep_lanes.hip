@@ -668,16 +668,14 @@ uint64_t place_steps(const std::vector<std::vector<StepRef>> &steps, int G, size
     return total;
 }
 
+// pl, pu: every chunk's plans for W wavefronts, G lanes a row, S entries a lane
 template <class T, int S>
-void build_steps(const HostSweep &lo, const HostSweep &up, const ChunkSet &C, int W, int G, LaneSweep<T> &L) {
-    std::vector<LanePlan> pl(C.nchunk), pu(C.nchunk);
+void build_steps(const HostSweep &lo, const HostSweep &up, const ChunkSet &C, int W, int G,
+                 const std::vector<LanePlan> &pl, const std::vector<LanePlan> &pu, LaneSweep<T> &L) {
     std::vector<LaneHead> head(C.nchunk);
     std::vector<std::vector<StepRef>> steps(C.nchunk);
     parallel_for(C.nchunk, 1, [&](size_t c0, size_t c1) {
         for (size_t c = c0; c < c1; ++c) {
-            uint32_t span;
-            pl[c] = std::move(plan_steps(lo, {C.start[c], C.start[c + 1]}, 64 * W / G, G * S, span)[0]);
-            pu[c] = std::move(plan_steps(up, {C.start[c], C.start[c + 1]}, 64 * W / G, G * S, span)[0]);
             append_steps(lo, pl[c], steps[c]);
             head[c].rounds_lo = (uint32_t)steps[c].size() / kAhead;
             append_steps(up, pu[c], steps[c]);
@@ -883,12 +881,18 @@ uint32_t lane_sweep_max_rows(size_t lds) {
 //     {1,1,4} 500, {1,1,8} 514, {1,4,4} 415, {1,2,8} 459, {4,4,4} 602
 //   128^2 ICT(1e-2), 509 levels of 32 rows, 4 entries: 138, 192, 387, 272, 304
 //   27^3 ICT(3e-3), 312 levels of 63 rows, 12 entries: 257, 251, 450, 289, 211
+// Levels of hundreds of rows take the whole workgroup, a lane a row, {4,1,4}
+// (with one workgroup's 1024 threads a level and two barriers, in brackets):
+//   IC(0) in colour order, 4 levels: 140^2 96 -> 48 us (49), 27^3 128 -> 63 (58)
+//   ILUT(5, 0.1) in colour order, 27^3, 43 levels: 131 -> 59 (85)
+//   27^3 ICT(0.1), 158 levels, 3 entries: 94 -> 55 (184); ICT(1e-2): 135 -> 111
 struct LaneShape {
     int waves, group, slots;
     float us;
 };
 constexpr LaneShape kShapes[] = {{1, 1, 4, 0.125f}, {1, 1, 8, 0.18f}, {1, 4, 4, 0.18f},
-                                 {1, 2, 8, 0.22f},  {1, 4, 8, 0.30f}, {4, 4, 4, 0.27f}};
+                                 {1, 2, 8, 0.22f},  {1, 4, 8, 0.30f}, {4, 4, 4, 0.27f},
+                                 {4, 1, 4, 0.21f}};
 
 // The fewest steps a sweep's rows [r0, r1) can take: the longest chain of
 // parts, the parts over the width.
@@ -916,42 +920,52 @@ template <class T>
 void build_lane_sweep(const HostSweep &lo, const HostSweep &up, const ChunkSet &C, LaneSweep<T> &L) {
     L.free_all();
     constexpr size_t K = sizeof(kShapes) / sizeof(kShapes[0]);
-    // chunks share the 256 compute units
-    const auto price = [&](const LaneShape &h, bool planned) {
-        std::vector<uint32_t> steps(C.nchunk, 0);
-        parallel_for(C.nchunk, 1, [&](size_t c0, size_t c1) {
-            for (size_t c = c0; c < c1; ++c)
-                for (const HostSweep *s : {&lo, &up}) {
-                    const uint32_t width = 64 * h.waves / h.group, entries = h.group * h.slots;
-                    uint32_t span = 0;
-                    if (planned) plan_steps(*s, {C.start[c], C.start[c + 1]}, width, entries, span);
-                    else span = fewest_steps(*s, C.start[c], C.start[c + 1], width, entries);
-                    steps[c] += span;
-                }
+    // plans: the chunks' plans of the shape (lower, upper), else (NULL) only
+    // the fewest steps they can take; chunks share the 256 compute units
+    // (a small factor's plans take less time than starting threads for them)
+    using Plans = std::vector<LanePlan>[2];
+    const size_t grain = lo.rp[lo.n] + up.rp[up.n] < 1u << 16 ? 2 * C.nchunk : 1;
+    const auto price = [&](const LaneShape &h, Plans *plans) {
+        const HostSweep *sweep[2] = {&lo, &up};
+        std::vector<uint32_t> steps(2 * C.nchunk, 0);
+        if (plans)
+            for (auto &p : *plans) p.resize(C.nchunk);
+        parallel_for(2 * C.nchunk, grain, [&](size_t q0, size_t q1) {
+            for (size_t q = q0; q < q1; ++q) {
+                const uint32_t c = q / 2, width = 64 * h.waves / h.group, entries = h.group * h.slots;
+                if (plans)
+                    (*plans)[q % 2][c] =
+                        std::move(plan_steps(*sweep[q % 2], {C.start[c], C.start[c + 1]}, width, entries, steps[q])[0]);
+                else
+                    steps[q] = fewest_steps(*sweep[q % 2], C.start[c], C.start[c + 1], width, entries);
+            }
         });
         double longest = 0, total = 0;
-        for (uint32_t v : steps) {
-            longest = std::max(longest, (double)v);
-            total += v;
+        for (size_t q = 0; q < steps.size(); q += 2) {
+            longest = std::max(longest, (double)steps[q] + steps[q + 1]);
+            total += (double)steps[q] + steps[q + 1];
         }
         return std::max(longest, total / 256) * h.us;
     };
     // shapes by their least price; planned until none left can be cheaper
     std::vector<std::pair<double, size_t>> least(K);
-    for (size_t k = 0; k < K; ++k) least[k] = {price(kShapes[k], false), k};
+    for (size_t k = 0; k < K; ++k) least[k] = {price(kShapes[k], nullptr), k};
     std::sort(least.begin(), least.end());
-    size_t best = least[0].second;
-    double best_us = price(kShapes[best], true);
-    for (size_t q = 1; q < K && least[q].first < best_us; ++q) {
-        const double us = price(kShapes[least[q].second], true);
-        if (us < best_us) {
+    size_t best = K;
+    double best_us = 0;
+    Plans plans;
+    for (size_t q = 0; q < K && (best == K || least[q].first < best_us); ++q) {
+        Plans p;
+        const double us = price(kShapes[least[q].second], &p);
+        if (best == K || us < best_us) {
             best = least[q].second;
             best_us = us;
+            for (int k = 0; k < 2; ++k) plans[k].swap(p[k]);
         }
     }
     const LaneShape &h = kShapes[best];
-    if (h.slots == 4) build_steps<T, 4>(lo, up, C, h.waves, h.group, L);
-    else build_steps<T, 8>(lo, up, C, h.waves, h.group, L);
+    if (h.slots == 4) build_steps<T, 4>(lo, up, C, h.waves, h.group, plans[0], plans[1], L);
+    else build_steps<T, 8>(lo, up, C, h.waves, h.group, plans[0], plans[1], L);
 }
 template void build_lane_sweep<double>(const HostSweep &, const HostSweep &, const ChunkSet &, LaneSweep<double> &);
 template void build_lane_sweep<float>(const HostSweep &, const HostSweep &, const ChunkSet &, LaneSweep<float> &);
@@ -984,6 +998,7 @@ void launch_lane_sweep(pp_ctx *ctx, const ChunkSet &C, const LaneSweep<T> &L, co
     PP_LANES(1, 2, 8)
     PP_LANES(1, 4, 8)
     PP_LANES(4, 4, 4)
+    PP_LANES(4, 1, 4)
 #undef PP_LANES
 #undef PP_LANES_M
     PP_CHECK(launched, PP_ERR_UNSUPPORTED, "chunked sweep: no kernel of this step shape and diagonal modes");

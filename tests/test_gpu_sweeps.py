@@ -47,7 +47,16 @@ def diagonal(d):
     return np.arange(n + 1, dtype=np.uint32), np.arange(n, dtype=np.uint32), d
 
 
+def dense(n):
+    a = np.random.default_rng(n).standard_normal((n, n))
+    a = a @ a.T + n * np.eye(n)
+    return (np.arange(n + 1, dtype=np.uint32) * n, np.tile(np.arange(n, dtype=np.uint32), n), a.ravel())
+
+
 CASES = {
+    # the shapes that the chunked sweep takes: one wavefront with a row on 1 lane of 4 entries (one_row, chain,
+    # 2d_short) or 8 (two_levels_long), on 2 of 8 (ilut), on 4 of 4 (narrow, 2d_fill, long_rows, ildlt) or 8
+    # (dense); four wavefronts with 4 lanes (3d_wide, blocks) or 1 (two_levels, ilu0) of 4
     # name: matrix, kind, arguments
     "one_row": lambda: (diagonal(np.array([3.0])), "ict", dict(threshold=1e-3)),
     "chain": lambda: (ppo.laplacian(700, 1, 1), "ict", dict(threshold=0.0)),
@@ -61,6 +70,9 @@ CASES = {
     "ilut": lambda: (ppo.upwind(19, 18, 17, 20.0, 10.0, 5.0), "ilut", dict(lfill=20, tolerance=1e-2)),
     "ilu0": lambda: (ppo.upwind(19, 18, 17, 20.0, 10.0, 5.0), "ilu0", dict()),
     "blocks": lambda: (blocks(ppo.laplacian(22, 21, 20), 9), "ildlt", dict(tolerance=1e-3)),
+    "dense": lambda: (dense(230), "ict", dict(threshold=0.0)),
+    "two_levels_long": lambda: (ppo.upwind(27, 27, 27, 20.0, 10.0, 5.0), "ilut",
+                                dict(lfill=20, tolerance=1e-2, ordering=1)),
 }
 
 
