@@ -1486,7 +1486,7 @@ SystemTiles tiles_of_system(const ReducedHost &H, uint32_t r0, int W, uint32_t n
 // batches that would leave units idle take tiles down to 1024 rows (smaller
 // ones wait on one another more than they compute: 24 systems of 60^2 to
 // 200^2 2.9 ms with 512 rows, 2.5 with 1024).  false (nothing kept): a system
-// does not fit.
+// does not fit, or all are small.
 bool batch_build_tiles(pp_batch *B, const std::vector<ReducedHost> &reds) {
     batch_free_tiles(B);
     const uint32_t ns = B->nsys;
@@ -1505,6 +1505,16 @@ bool batch_build_tiles(pp_batch *B, const std::vector<ReducedHost> &reds) {
             if (H.kf_rp[q + 1] - H.kf_rp[q] > kSliceWidth) return false;
     }
     const int W = width <= 4 ? 4 : 6;
+    // Small systems stay with k_batch_pcg, one launch for the whole solve: the
+    // refinement steps' launches and waits take 170 us more than it does, and an
+    // iteration saves only as the largest system grows.  16 (1000) equal systems,
+    // us a solve in k_batch_pcg and over tiles: 5-point 22^2 380, 422 (601, 692);
+    // 24^2 451, 440 (788, 754) and 389, 417 (688, 704) with constant
+    // coefficients; 26^2 479, 459 (938, 793).  7-point 9^3 290, 341 (627, 539),
+    // 10^3 324, 351 (782, 599), 11^3 409, 391 (1156, 693).
+    uint32_t largest = 0;
+    for (const ReducedHost &H : reds) largest = std::max(largest, H.n0 + H.n1);
+    if (largest < (W == 4 ? 600u : 1100u)) return false;
     const uint32_t maxf = kTileThreads * (W == 4 ? TileShape<4>::kF : TileShape<6>::kF);
     const uint32_t maxs = kTileThreads * (W == 4 ? TileShape<4>::kS : TileShape<6>::kS);
     const uint32_t maxh = kTileThreads * (W == 4 ? TileShape<4>::kH : TileShape<6>::kH);

@@ -1,7 +1,8 @@
 """The batched mixed solve spread over tiles (reduced CG, several workgroups a
 system) against the FP64 batch solve: systems of one row pair to many tiles,
 5- and 7-point rows, sizes around a tile's, and a system whose tiles' sums
-need more than one round of words.  Every system's solution meets the true
+need more than one round of words; batches of small systems only, which keep
+one workgroup a system.  Every system's solution meets the true
 residual test, checked on the host with the oracle's product; repeated solves
 are equal bit for bit (every sum has a fixed order)."""
 import numpy as np
@@ -31,9 +32,16 @@ def vardiff(side, seed):
 
 
 BATCHES = {
-    "small": lambda: [ppo.laplacian(2, 1, 1), ppo.laplacian(3, 2, 1), vardiff(5, 1), vardiff(16, 2)],
+    "small": lambda: [ppo.laplacian(2, 1, 1), ppo.laplacian(3, 2, 1), vardiff(5, 1), vardiff(16, 2)],  # one workgroup
+    "small_beside_a_larger": lambda: [ppo.laplacian(2, 1, 1), ppo.laplacian(3, 2, 1), vardiff(5, 1), vardiff(16, 2),
+                                      vardiff(25, 3)],
+    "below_the_line": lambda: [ppo.laplacian(599, 1, 1), ppo.laplacian(23, 26, 1)],
+    "at_the_line": lambda: [ppo.laplacian(600, 1, 1), ppo.laplacian(23, 26, 1)],
+    "below_the_line_3d": lambda: [ppo.laplacian(7, 157, 1), ppo.laplacian(10, 11, 9)],  # 1099 rows and less
+    "at_the_line_3d": lambda: [ppo.laplacian(10, 11, 10), ppo.laplacian(5, 4, 3)],
     "around_a_tile": lambda: [vardiff(s, s) for s in (45, 46, 63, 64, 65, 90, 91)],
-    "around_a_slice": lambda: [ppo.laplacian(*g, 1) for g in ((17, 15), (16, 16), (257, 1), (73, 7), (32, 16), (2, 1))],
+    "around_a_slice": lambda: [ppo.laplacian(*g, 1) for g in ((17, 15), (16, 16), (257, 1), (73, 7), (32, 16), (2, 1),
+                                                              (31, 20))],
     "uneven": lambda: [vardiff(s, s) for s in (200, 33, 129, 8, 70)],
     "seven_point": lambda: [ppo.laplacian(16, 15, 14), ppo.laplacian(24, 23, 22), vardiff(40, 3)],
     "many_tiles": lambda: [ppo.laplacian(90, 2100, 1), vardiff(20, 5)],
@@ -54,7 +62,7 @@ def test_tiled_mixed_solve(pp, torch, name):
     it = B.solve(b, x, precision="mixed", tol=1e-8)
     assert B.report.converged and B.report.true_relres < 1e-8 and B.report.cg_variant == 3
     # the path under test ran: every system a tile at least
-    if name == "halo_too_wide":
+    if name in ("halo_too_wide", "small", "below_the_line", "below_the_line_3d"):
         assert B.info().tiles == B.report.batch_tiles == 0
     else:
         assert B.info().tiles == B.report.batch_tiles >= len(systems)
