@@ -403,7 +403,7 @@ protected:
 
 // Sweep schedule and row ordering shared by the triangular factors.
 struct TriangularOptions {
-    int trsv = PP_TRSV_AUTO;         // PP_TRSV_LEVELS / PP_TRSV_SYNCFREE
+    int trsv = PP_TRSV_AUTO;          // or one of PP_TRSV_*
     int ordering = PP_ORDER_NATURAL;  // PP_ORDER_MULTICOLOR for IC(0)/ILU(0)
     bool keepFP32 = false;            // also keep an FP32 factor (mixed solves)
 };
