@@ -197,6 +197,7 @@ class Context:
 
     def __init__(self, device=0):
         self.device = device
+        self._users, self._dropped = 0, False
         h = C.c_void_p()
         check(_capi.lib().pp_ctx_create(device, C.byref(h)))
         self.h = h
@@ -213,13 +214,29 @@ class Context:
     def sync(self):
         self.check(_capi.lib().pp_ctx_sync(self.h))
 
-    def __del__(self):
+    # Matrices, preconditioners and batches use their context when they are
+    # destroyed, and objects of a reference cycle (a traceback makes one) are
+    # finalized in any order: the last of them to go takes the context along.
+    def _enter(self):
+        self._users += 1
+
+    def _leave(self):
+        self._users -= 1
+        if self._dropped and not self._users:
+            self._destroy()
+
+    def _destroy(self):
         try:
             if getattr(self, "h", None):
                 _capi.lib().pp_ctx_destroy(self.h)
                 self.h = None
         except Exception:
             pass
+
+    def __del__(self):
+        self._dropped = True
+        if not getattr(self, "_users", 0):
+            self._destroy()
 
 
 def _torch():
@@ -261,6 +278,7 @@ class CSRMatrix:
         self.ctx.check(_capi.lib().pp_csr_create(self.ctx.h, n, self.ncol, _p(self.rp, C.c_uint32),
                                                  _p(ci_, C.c_uint32), _p(v_, C.c_double), C.byref(h)))
         self.h = h
+        self.ctx._enter()
 
     @classmethod
     def from_scipy(cls, M, ctx=None):
@@ -333,6 +351,7 @@ class CSRMatrix:
             if getattr(self, "h", None):
                 _capi.lib().pp_csr_destroy(self.h)
                 self.h = None
+                self.ctx._leave()
         except Exception:
             pass
 
@@ -354,6 +373,7 @@ class BasePrecondition:
         h = C.c_void_p()
         self.ctx.check(_capi.lib().pp_precond_create(self.ctx.h, self.A.h, C.byref(self._opts), C.byref(h)))
         self.h = h
+        self.ctx._enter()
 
     def setup(self):
         self.ctx.check(_capi.lib().pp_precond_setup(self.ctx.h, self.h))
@@ -428,6 +448,7 @@ class BasePrecondition:
             if getattr(self, "h", None):
                 _capi.lib().pp_precond_destroy(self.h)
                 self.h = None
+                self.ctx._leave()
         except Exception:
             pass
 
@@ -590,6 +611,7 @@ class BatchedSystems:
                                                    _p(self.rp, C.c_uint32), _p(self.ci, C.c_uint32),
                                                    _p(self.v, C.c_double), C.byref(h)))
         self.h = h
+        self.ctx._enter()
         self.block = 256
         self.report = _capi.SolveReport()
         self.ordering = 0
@@ -664,6 +686,7 @@ class BatchedSystems:
             if getattr(self, "h", None):
                 _capi.lib().pp_batch_destroy(self.h)
                 self.h = None
+                self.ctx._leave()
         except Exception:
             pass
 

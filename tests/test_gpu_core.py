@@ -711,3 +711,20 @@ def test_pipe_sweep_shapes(pp, torch, case):
             P1.MInvSolve(a)
             P4.MInvSolve(b)
             assert np.array_equal(host(a), host(b)), (seed, dt)
+
+
+def test_objects_of_a_cycle_outlive_their_context(torch):
+    # a traceback keeps a context and its objects in one reference cycle, whose
+    # members the collector finalizes in any order, the context first here
+    import gc
+    import prispack_amd as pp
+    for _ in range(3):
+        own = pp.Context(0)
+        M = pp.CSRMatrix(*ppo.laplacian(7, 6, 1), ctx=own)
+        P = pp.IC0(M)
+        P.setup()
+        B = pp.BatchedSystems([ppo.laplacian(5, 4, 1)], ctx=own)
+        own.kept = M.kept = P.kept = B.kept = [own, M, P, B]
+        del own, M, P, B
+        gc.collect()
+        assert float(torch.ones(8, device="cuda").sum()) == 8.0  # no error left behind
