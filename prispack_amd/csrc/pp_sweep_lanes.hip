@@ -714,14 +714,16 @@ void build_steps(const HostSweep &lo, const HostSweep &up, const ChunkSet &C, in
 uint32_t strip_words(const HostSweep &s, const std::vector<uint32_t> &start) {
     std::vector<uint32_t> words(start.size() - 1);
     parallel_for(words.size(), 1, [&](size_t k0, size_t k1) {
-        std::vector<uint32_t> remote;
+        std::vector<uint32_t> seen(s.n, 0);  // the last strip of this thread that reads the row, + 1
         for (size_t k = k0; k < k1; ++k) {
-            remote.clear();
-            for (uint32_t e = s.rp[start[k]]; e < s.rp[start[k + 1]]; ++e)
-                if (s.ci[e] < start[k] || s.ci[e] >= start[k + 1]) remote.push_back(s.ci[e]);
-            std::sort(remote.begin(), remote.end());
-            const size_t n = std::unique(remote.begin(), remote.end()) - remote.begin();
-            words[k] = start[k + 1] - start[k] + 1 + (uint32_t)n;
+            words[k] = start[k + 1] - start[k] + 1;
+            for (uint32_t e = s.rp[start[k]]; e < s.rp[start[k + 1]]; ++e) {
+                const uint32_t j = s.ci[e];
+                if ((j < start[k] || j >= start[k + 1]) && seen[j] != k + 1) {
+                    seen[j] = (uint32_t)k + 1;
+                    ++words[k];
+                }
+            }
         }
     });
     return *std::max_element(words.begin(), words.end());
