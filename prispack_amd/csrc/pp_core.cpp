@@ -614,7 +614,25 @@ int pp_ctx_set_stream(pp_ctx *ctx, void *s) {
     // pooled blocks may still be in use by work queued on the old stream
     if (ctx->pool_dirty && hipStreamSynchronize(ctx->stream) != hipSuccess) return PP_ERR_HIP;
     ctx->pool_dirty = false;
-    ctx->stream = s ? (hipStream_t)s : ctx->own_stream;
+    const hipStream_t next = s ? (hipStream_t)s : ctx->own_stream;
+    if (next != ctx->stream && ctx->strips_queued) {
+        // strip sweeps still running on the old stream use the buffers that the
+        // new one's will use: the new stream waits for it, the host where the
+        // new one is capturing (what the old one captures has not run)
+        hipStreamCaptureStatus was = hipStreamCaptureStatusNone, will = hipStreamCaptureStatusNone;
+        bool ordered = hipStreamIsCapturing(ctx->stream, &was) == hipSuccess &&
+                       hipStreamIsCapturing(next, &will) == hipSuccess;
+        if (ordered && was == hipStreamCaptureStatusNone)
+            ordered = will != hipStreamCaptureStatusNone
+                          ? hipStreamSynchronize(ctx->stream) == hipSuccess
+                          : hipEventRecord(ctx->strip_event, ctx->stream) == hipSuccess &&
+                                hipStreamWaitEvent(next, ctx->strip_event, 0) == hipSuccess;
+        if (!ordered) {  // a stream that its owner has destroyed
+            (void)hipGetLastError();
+            if (hipDeviceSynchronize() != hipSuccess) return PP_ERR_HIP;
+        }
+    }
+    ctx->stream = next;
     return PP_OK;
 }
 
@@ -630,6 +648,7 @@ int pp_ctx_set_wait_limit(pp_ctx *ctx, double seconds) {
 int pp_ctx_sync(pp_ctx *ctx) {
     return guarded(ctx, [&] {
         PP_HIP(hipStreamSynchronize(ctx->stream));
+        ctx->strips_queued = false;
         throw_given_up(ctx);
     });
 }
@@ -651,6 +670,7 @@ void pp_ctx_destroy(pp_ctx *ctx) {
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->pinned_ctl) (void)hipHostFree(ctx->pinned_ctl);
     if (ctx->ring_host) (void)hipHostFree(ctx->ring_host);
+    if (ctx->strip_event) (void)hipEventDestroy(ctx->strip_event);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);

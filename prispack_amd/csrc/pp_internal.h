@@ -171,6 +171,10 @@ struct pp_ctx {
         uint32_t n = 0;
     } strip_slots[2][2];
     std::vector<void *> old_strip_slots;
+    // strip sweeps launched since the last pp_ctx_sync: a stream set meanwhile
+    // waits for the one before it (pp_ctx_set_stream), they use the same buffers
+    bool strips_queued = false;
+    hipEvent_t strip_event = nullptr;
     double clock_hz = 1e8;         // of wall_clock64
     long long spin_deadline = 0;   // wall_clock64 ticks a wait may last (pp_ctx_set_wait_limit)
     // while set (StopScope), SpMV / dot / GEMV / convert kernels return at

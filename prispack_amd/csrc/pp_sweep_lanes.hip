@@ -1081,6 +1081,7 @@ bool strip_reserve(pp_ctx *ctx, const StripSweep<T> &L) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     PP_HIP(hipStreamIsCapturing(ctx->stream, &capturing));
     if (capturing != hipStreamCaptureStatusNone) return false;
+    if (!ctx->strip_event) PP_HIP(hipEventCreateWithFlags(&ctx->strip_event, hipEventDisableTiming));
     for (int k = 0; k < 2; ++k) {
         if (S[k].p && S[k].n >= want[k]) continue;
         const uint32_t n = std::max({1024u, want[k], 2 * S[k].n});
@@ -1101,6 +1102,7 @@ bool launch_strip_sweeps(pp_ctx *ctx, const StripSweep<T> &L, const T *x, T *y) 
     if (!strip_reserve(ctx, L)) return false;
     const pp_ctx::StripSlots *S = ctx->strip_slots[sizeof(T) == 4];
     T *lo = (T *)S[0].p, *up = (T *)S[1].p;
+    ctx->strips_queued = true;
     launch_strip_side<T>(ctx, L, L.lo, lo, L.up.nslots, up, x, y);
     launch_strip_side<T>(ctx, L, L.up, up, L.lo.nslots, lo, y, y);
     return true;

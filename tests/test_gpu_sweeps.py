@@ -226,6 +226,29 @@ def test_strips_on_two_contexts_at_once(pp, torch, f32):
             assert torch.equal(want, got), (k, i)
 
 
+def test_strips_on_a_context_that_changes_streams(pp, torch):
+    # applies queued on one stream after another: they share the context's buffers
+    M = pp.CSRMatrix(*ppo.laplacian(40, 33, 29))
+    P1, P = (pp.IncompleteCholesky(M, 1e-2, trsv=t) for t in (1, 5))
+    P1.setup()
+    P.setup()
+    ctx = pp.Context(0)
+    streams = [torch.cuda.Stream() for _ in range(3)] + [None]
+    xs = [torch.tensor(ppo.normal(M.n, 300 + i), device="cuda") for i in range(24)]
+    want, ys = [P1.MInvSolve(x.clone()) for x in xs], [torch.zeros_like(x) for x in xs]
+    torch.cuda.synchronize()
+    for i, (x, y) in enumerate(zip(xs, ys)):
+        for k in ([i + 1, i + 2] if i % 5 == 4 else []) + [i]:  # also streams that get no apply in between
+            s = streams[k % 4]
+            ctx.check(pp._capi.lib().pp_ctx_set_stream(ctx.h, s.cuda_stream if s else None))
+        _apply_on(ctx, P, x, y)
+    ctx.sync()
+    torch.cuda.synchronize()
+    ctx.check(pp._capi.lib().pp_ctx_set_stream(ctx.h, None))
+    for i, (w, y) in enumerate(zip(want, ys)):
+        assert torch.equal(w, y), i
+
+
 def test_strips_captured(pp, torch):
     # an apply captured on a context that has exchange buffers, and on one
     # that cannot get them inside the capture (level sweeps, the same bits)
