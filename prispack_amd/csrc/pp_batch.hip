@@ -1972,13 +1972,12 @@ int pp_batch_set_values(pp_ctx *ctx, pp_batch *B, const double *values, int on_d
         if (B->refresh == 0) batch_refresh_build(B);
         // the factorization on the device overwrites the factor: the values it
         // came from are kept until it has succeeded
-        if (B->refresh == 1 && !B->factor_before) {
-            if (!B->v64_before) B->v64_before = dalloc<double>(B->nnz);
-            std::swap(B->v64, B->v64_before);
-        }
-        PP_HIP(hipMemcpy(B->v64, values, B->nnz * sizeof(double),
+        const bool keep = B->refresh == 1 && !B->factor_before;
+        if (keep && !B->v64_before) B->v64_before = dalloc<double>(B->nnz);
+        PP_HIP(hipMemcpy(keep ? B->v64_before : B->v64, values, B->nnz * sizeof(double),
                          on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice));
         PP_HIP(hipStreamSynchronize(nullptr));  // a device copy may return before it is done
+        if (keep) std::swap(B->v64, B->v64_before);
         B->h_v_stale = true;
         if (B->refresh == 1) {
             B->factor_before = !batch_refresh(B, B->v64);
